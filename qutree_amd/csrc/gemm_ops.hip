@@ -15,69 +15,17 @@
 // loads, so every wavefront runs the same number of k-steps and MFMA issue
 // stays uniform.  Two accumulator pairs alternate between k-steps so that
 // consecutive MFMAs do not depend on each other.
-#include <hip/hip_ext.h>
-
 #include <algorithm>
 #include <type_traits>
 
+#include "gemm_dev.hpp"
 #include "gemm_ops.hpp"
 
 namespace qtg {
 
 namespace {
 
-// Launches k; with kt set, through hipExtLaunchKernelGGL so that kt's events
-// carry the kernel's own start and stop times (no marker packets around it).
-template <typename K, typename... A>
-void launch_timed(K k, dim3 grid, dim3 block, unsigned lds, hipStream_t s, const KernelTiming* kt, A... a) {
-  if (kt) hipExtLaunchKernelGGL(k, grid, block, lds, s, kt->start, kt->stop, 0, a...);
-  else hipLaunchKernelGGL(k, grid, block, lds, s, a...);
-}
-
-
-template <typename T>
-struct MF;
-template <>
-struct MF<double> {
-  typedef double v4 __attribute__((ext_vector_type(4)));
-  static __device__ inline v4 mma(double a, double b, v4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ inline int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <>
-struct MF<float> {
-  typedef float v4 __attribute__((ext_vector_type(4)));
-  static __device__ inline v4 mma(float a, float b, v4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ inline int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
-// (cr, ci) += a * b on one complex k-step (a is already conjugated if needed)
-template <typename T>
-__device__ inline void cmma(typename MF<T>::v4& cr, typename MF<T>::v4& ci, const cplx<T>& a, const cplx<T>& b) {
-  cr = MF<T>::mma(a.re, b.re, cr);
-  cr = MF<T>::mma(-a.im, b.im, cr);
-  ci = MF<T>::mma(a.re, b.im, ci);
-  ci = MF<T>::mma(a.im, b.re, ci);
-}
-
 constexpr int kWaves = kGemmWaves;  // wavefronts (tasks) per workgroup
-
-// Wavefront index in the workgroup, as a wave-uniform (scalar) value, so that
-// descriptor loads and address arithmetic stay on the scalar unit.
-__device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
-
-// base[off] when ok, else zero.  The load itself is unconditional, from
-// base[0] when !ok (base is the start of an operand, always in bounds): a
-// guarded load would let the compiler select between the operand and a stack
-// zero and fall back to generic (flat) loads.
-template <typename T>
-__device__ inline cplx<T> ldz(const cplx<T>* __restrict__ base, int64_t off, bool ok) {
-  const cplx<T> v = base[ok ? off : 0];
-  return ok ? v : czero<T>();
-}
 
 // Descriptor of a task: one load from the per-task table built on the host.
 __device__ inline int task_desc(const int32_t* __restrict__ wgdesc, int64_t task) { return wgdesc[task]; }
@@ -292,16 +240,6 @@ __device__ inline void gm_store(const GmDesc& d, const GmTile& g, const cplx<TO>
 // it instead of predicated (their products land in tile rows and columns
 // that are never stored), and only the K tail zeroed.  The tile is
 // accumulated transposed when bef >= 4 (gm_rows_on_lanes).
-
-// base[idx] for idx < 2^27: a 32-bit byte offset from the base
-template <typename V>
-__device__ inline V ld32(const V* base, uint32_t idx) {
-  return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + (idx * (uint32_t)sizeof(V)));
-}
-template <typename V>
-__device__ inline V* at32(V* base, uint32_t idx) {
-  return reinterpret_cast<V*>(reinterpret_cast<char*>(base) + (idx * (uint32_t)sizeof(V)));
-}
 
 // Lean tile coordinates: no division when the output has one column tile
 __device__ inline GmTile gm_tile_lean(const GmDesc& d, uint32_t t) {

@@ -160,6 +160,21 @@ int launch_gm_single(const GmDesc& d, const void* x, const void* m, void* o, hip
 template <typename T>
 int launch_gc_single(const GcDesc& d, const void* x, const void* y, void* o, hipStream_t s);
 
+// One hole contraction alone on the card (gemm_block.hip), for descriptors
+// with gc_lean_ok.  nt 1: a workgroup of 16 wavefronts per 16 x 16 tile, each
+// on a sixteenth of K.  nt 2: 32 x 32 macro tiles, four wavefronts, K split
+// over S workgroups as well when S > 1; the S partial tiles (part_elems()
+// complex elements, caller's buffer) are then summed by a second launch.
+struct GcOnePlan {
+  int nt, S;
+  int64_t macro, tiles;  // macro tiles, 16 x 16 tiles
+  int64_t part_elems() const { return S > 1 ? tiles * S * 256 : 0; }
+};
+GcOnePlan plan_gc_one(const GcDesc& d, int64_t max_part_elems);
+template <typename T>
+int launch_gc_one(const GcDesc& d, const GcOnePlan& p, const void* x, const void* y, void* o, void* part,
+                  hipStream_t s);
+
 // Real FP64 mode product (op GM_N or GM_T; one descriptor, no K split).
 int launch_gm_real(const GmDesc& d, const double* x, const double* m, double* o, hipStream_t s);
 

@@ -95,18 +95,6 @@ int mode_product_one(const qtg_mode_product_desc& d, cplx<R>* C, const cplx<R>* 
   return launch_gm_single<R>(g, B, M, C, s);
 }
 
-template <typename R>
-int hole_one(const qtg_hole_contraction_desc& d, cplx<R>* Sm, const cplx<R>* A, const cplx<R>* B, hipStream_t s) {
-  if (!Sm || !A || !B) {
-    set_error("hole contraction: null pointer");
-    return QTG_EARG;
-  }
-  GcDesc g;
-  int rc = to_gc(d, g);
-  if (rc) return rc;
-  return launch_gc_single<R>(g, A, B, Sm, s);
-}
-
 struct Plan {
   int kind = 0;  // 0 mode product, 1 hole contraction
   bool c64 = false;
@@ -142,9 +130,14 @@ static_assert(kNoAllocTableOff % 256 == 0, "table alignment");
 }  // namespace
 }  // namespace qtg
 
-// In host code this name is only a handle for hipGetSymbolAddress: kernels
-// receive the per-device address it returns (scratch_address).
+// In host code these names are only handles for hipGetSymbolAddress: kernels
+// receive the per-device address it returns (symbol_address).
 static __device__ __align__(256) unsigned char scratch[qtg::kNoAllocBytes];
+// Partial tiles of single hole contractions split over workgroups, in slots
+// (see PartPool): 8 MiB hold the 128 shares of a 64 x 64 complex128 output.
+constexpr int kPartSlots = 2;
+constexpr size_t kPartBytes = (size_t)8 << 20;
+static __device__ __align__(256) unsigned char part_scratch[kPartSlots * kPartBytes];
 
 namespace qtg {
 namespace {
@@ -153,27 +146,100 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
 
-// The current device's copy of `scratch`, looked up once per device with
-// that device current.
+// The current device's copy of a device array, looked up once per device
+// with that device current (cache under mu, which the caller holds).
+int symbol_address(const void* symbol, int dev, void* (&cache)[kMaxDevices], const char* what, void** out) {
+  if (dev < 0 || dev >= kMaxDevices) {
+    set_error(std::string(what) + ": device index out of range");
+    return QTG_EDEVICE;
+  }
+  if (!cache[dev]) {
+    void* p = nullptr;
+    const hipError_t e = hipGetSymbolAddress(&p, symbol);
+    if (e != hipSuccess || !p) {
+      set_error(std::string(what) + ": hipGetSymbolAddress: " + hipGetErrorString(e));
+      return QTG_EDEVICE;
+    }
+    cache[dev] = p;
+  }
+  *out = cache[dev];
+  return QTG_OK;
+}
+
 int scratch_address(void** out) {
   int dev = 0;
   QTG_HIP_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kMaxDevices) {
-    set_error("no-allocation contraction: device index out of range");
-    return QTG_EDEVICE;
-  }
   std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (!g_scratch_ptr[dev]) {
-    void* p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p) {
-      set_error(std::string("no-allocation contraction: hipGetSymbolAddress: ") + hipGetErrorString(e));
-      return QTG_EDEVICE;
-    }
-    g_scratch_ptr[dev] = p;
+  return symbol_address(HIP_SYMBOL(scratch), dev, g_scratch_ptr, "no-allocation contraction", out);
+}
+
+// The slots of part_scratch, per device.  A call holds the lock while it
+// enqueues its two launches and records the slot's event behind them; the
+// next user of a slot, on whatever stream and thread, makes its stream wait
+// for that event unless it has passed.  Nothing is allocated but the events.
+struct PartPool {
+  std::mutex mu;
+  void* base[kMaxDevices] = {};
+  hipEvent_t ev[kMaxDevices][kPartSlots] = {};
+  bool used[kMaxDevices][kPartSlots] = {};
+  unsigned next[kMaxDevices] = {};
+};
+PartPool g_parts;
+
+template <typename R>
+int hole_split(const GcDesc& g, const GcOnePlan& p, const cplx<R>* A, const cplx<R>* B, cplx<R>* Sm, hipStream_t s) {
+  int dev = 0;
+  QTG_HIP_TRY(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(g_parts.mu);
+  void* base = nullptr;
+  int rc = symbol_address(HIP_SYMBOL(part_scratch), dev, g_parts.base, "hole contraction", &base);
+  if (rc) return rc;
+  // a slot whose last use has ended, else the one used longest ago
+  int slot = -1;
+  for (int i = 0; i < kPartSlots && slot < 0; ++i)
+    if (!g_parts.used[dev][i] || hipEventQuery(g_parts.ev[dev][i]) == hipSuccess) slot = i;
+  (void)hipGetLastError();  // hipErrorNotReady of a query
+  if (slot < 0) {
+    slot = (int)(g_parts.next[dev] % kPartSlots);
+    QTG_HIP_TRY(hipStreamWaitEvent(s, g_parts.ev[dev][slot], 0));
   }
-  *out = g_scratch_ptr[dev];
-  return QTG_OK;
+  g_parts.next[dev] = (unsigned)slot + 1;
+  if (!g_parts.ev[dev][slot])
+    QTG_HIP_TRY(hipEventCreateWithFlags(&g_parts.ev[dev][slot], hipEventDisableTiming));
+  g_parts.used[dev][slot] = true;
+  rc = launch_gc_one<R>(g, p, A, B, Sm, static_cast<unsigned char*>(base) + (size_t)slot * kPartBytes, s);
+  // also after a failed launch: the first of the two may run
+  const hipError_t e = hipEventRecord(g_parts.ev[dev][slot], s);
+  if (!rc && e != hipSuccess) {
+    set_error(std::string("hole contraction: hipEventRecord: ") + hipGetErrorString(e));
+    rc = QTG_EDEVICE;
+  }
+  return rc;
+}
+
+// Reductions long enough for it split over workgroups (plan_gc_one), except
+// under stream capture: a replayed graph would use its slot unordered with
+// other calls.
+template <typename R>
+int hole_one(const qtg_hole_contraction_desc& d, cplx<R>* Sm, const cplx<R>* A, const cplx<R>* B, hipStream_t s) {
+  if (!Sm || !A || !B) {
+    set_error("hole contraction: null pointer");
+    return QTG_EARG;
+  }
+  GcDesc g;
+  int rc = to_gc(d, g);
+  if (rc) return rc;
+  if (!gc_lean_ok(g)) return launch_gc_single<R>(g, A, B, Sm, s);
+  GcOnePlan p = plan_gc_one(g, (int64_t)(kPartBytes / sizeof(cplx<R>)));
+  if (p.S > 1) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      p = plan_gc_one(g, 0);
+    }
+  }
+  if (p.S > 1) return hole_split<R>(g, p, A, B, Sm, s);
+  return launch_gc_one<R>(g, p, A, B, Sm, nullptr, s);
 }
 
 }  // namespace

@@ -1,0 +1,80 @@
+"""The register-blocked contraction kernels (gemm_block.hip) at the edges of
+their tiles and of the rules that choose them, against numpy in FP64.
+
+Bounds: a sum of K products has a relative error of at most about K u in the
+worst case and about sqrt(K) u for random terms (u = 2^-53 or 2^-24); the
+checks allow 4 sqrt(K + 16) u of the result's 2-norm."""
+import numpy as np
+import pytest
+
+import qutree_amd as Q
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(rng, shape, c64):
+    z = rng.normal(size=shape) + 1j * rng.normal(size=shape)
+    return z.astype(np.complex64 if c64 else np.complex128)
+
+
+def close(got, ref, K, c64):
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    lim = 4 * np.sqrt(K + 16) * (2.0 ** -24 if c64 else 2.0 ** -53)
+    print(f"  err {err:.2e} limit {lim:.2e}", flush=True)
+    assert err < lim
+
+
+# reductions around one workgroup's 768, the shortest shares, one element;
+# outputs around the 16 and 32 wide tiles
+ONE_HOLE = [(1, 1, 1, 1), (3, 16, 17, 5), (1, 33, 2, 768), (769, 15, 31, 1), (32, 32, 32, 24), (5, 65, 48, 333),
+            (64, 64, 64, 64), (2, 17, 130, 4001), (7, 5, 3, 30011), (300, 31, 33, 257)]
+
+
+@pytest.mark.parametrize("c64", [False, True])
+@pytest.mark.parametrize("before,nA,nB,after", ONE_HOLE)
+def test_single_hole_contraction(before, nA, nB, after, c64):
+    print(f"case single hole {before} {nA} {nB} {after} c64={c64}", flush=True)
+    rng = np.random.default_rng(before + nA)
+    A, B, S0 = rand(rng, (after, nA, before), c64), rand(rng, (after, nB, before), c64), rand(rng, (nB, nA), c64)
+    ref = np.einsum("ajb,alb->lj", A.conj().astype(np.complex128), B.astype(np.complex128), optimize=True)
+    dA, dB = Q.DeviceBuffer.from_array(A), Q.DeviceBuffer.from_array(B)
+    fn = Q.lib().qtg_hole_contraction_c if c64 else Q.lib().qtg_hole_contraction_z
+    for acc in (0, 1):
+        dS = Q.DeviceBuffer.from_array(S0)
+        Q.check(fn(dS.ptr, dA.ptr, dB.ptr, before, nA, nB, after, acc, None))
+        got = dS.download(S0.dtype).reshape(nB, nA)
+        close(got, ref + S0 if acc else ref, before * after, c64)
+
+
+def test_single_hole_contraction_streams():
+    """Long reductions back to back on several streams share two slots of
+    partial tiles: every result stays that of its own operands."""
+    print("case single hole on streams", flush=True)
+    import ctypes as C
+    rng = np.random.default_rng(3)
+    before, n, after = 40, 24, 400
+    L = Q.lib()
+    streams = []
+    for _ in range(3):
+        s = C.c_void_p()
+        Q.check(L.qtg_stream_create(C.byref(s)))
+        streams.append(s)
+    A = [rand(rng, (after, n, before), False) for _ in range(6)]
+    d = [Q.DeviceBuffer.from_array(a) for a in A]
+    out = [Q.DeviceBuffer(16 * n * n) for _ in range(36)]
+    for i in range(36):
+        Q.check(L.qtg_hole_contraction_z(out[i].ptr, d[i // 6].ptr, d[i % 6].ptr, before, n, n, after, 0,
+                                         streams[i % 3]))
+    Q.synchronize()
+    first = {}
+    for i in range(36):
+        ref = np.einsum("ajb,alb->lj", A[i // 6].conj(), A[i % 6], optimize=True)
+        got = out[i].download(np.complex128).reshape(n, n)
+        close(got, ref, before * after, False)
+        first[i] = got
+    for i in range(36):  # again, alone: the same bits
+        Q.check(L.qtg_hole_contraction_z(out[i].ptr, d[i // 6].ptr, d[i % 6].ptr, before, n, n, after, 0, None))
+        Q.synchronize()
+        assert np.array_equal(out[i].download(np.complex128).reshape(n, n), first[i])
+    for s in streams:
+        Q.check(L.qtg_stream_destroy(s))
