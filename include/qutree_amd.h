@@ -162,9 +162,10 @@ int qtg_qr_batch_z(const double* A, double* Q, int64_t m, int64_t n, int64_t cou
  * (tight serving loops, harnesses that forbid hipMalloc).  The same grouped
  * hole contractions as qtg_hole_contraction_plan_create + qtg_plan_execute
  * (complex128; X from A_base, Y from B_base, offsets in complex elements),
- * but the descriptor tables are staged in a fixed device array of the library
- * (about 1.3 MB per GPU, held until the process ends) instead of a plan's
- * allocation: at most 4096 descriptors and 2^18 16 x 16 output tiles
+ * but the descriptor tables and partial tiles are staged in fixed device
+ * arrays of the library (about 4.6 MB and 16 MB per GPU, held until the
+ * process ends) instead of a plan's allocation: at most 4096 descriptors and
+ * 2^18 16 x 16 output tiles, a reduction beyond 1024 counting four-fold
  * (QTG_ESHAPE beyond).  Allocates no device memory; returns when the result
  * is written.  Every call on one GPU shares that array, so calls that overlap
  * on one GPU (other host threads) race. */

@@ -2,18 +2,25 @@
 // of the grouped mode product and hole contraction whose launch fills the
 // card, where operand traffic and not latency decides.
 //
-// gc_block (hole contraction): a workgroup owns a macro tile of up to
-// NT x NT output tiles of 16 x 16; every wavefront holds all of it in
-// registers and walks its own share of the reduction, so each element of the
-// bra and the ket is loaded once per macro tile, and the shares are summed in
-// LDS in wavefront order.  One wavefront per 16 x 16 tile (gc_grouped) reads
-// each operand once per tile of the other index, from workgroups that the
-// dispatcher spreads over XCDs with L2s of their own.  S > 1 splits a
-// reduction over S workgroups as well; their partial tiles are summed in
-// order by gc_block_sum.
+// gc_block (hole contraction): a workgroup owns a macro tile of NT x NT
+// output tiles of 16 x 16; every wavefront holds all of it in registers and
+// walks its own share of the reduction, so each element of the bra and the
+// ket is loaded once per macro tile, and the shares are summed in LDS in
+// wavefront order.  One wavefront per 16 x 16 tile (gc_grouped) reads each
+// operand once per tile of the other index, from workgroups that the
+// dispatcher spreads over XCDs with L2s of their own.  A reduction may be
+// shared by several workgroups; their partial tiles are summed in order by
+// gc_block_sum.  4096 order-3 complex128 tensors with legs 8-64 (4.3 GB of
+// operands): 1552 -> 1086 us, 3.9 TB/s, where a large copy reaches 4.9; 1000
+// complex64 tensors of legs 3-61: 418 -> 318 us.
 //
-// Descriptors pass gc_lean_ok (32-bit offsets, see gemm_ops.hip).
+// gm_block (mode product): a wavefront owns 2 x 2 output tiles, so X is read
+// once per 32 columns and M once per 32 rows.  The 4096 tensors' products:
+// 1284 -> 1222 us (3.5 TB/s read and written).
+//
+// Descriptors pass gm_lean_ok / gc_lean_ok (32-bit offsets, see gemm_ops.hip).
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm_dev.hpp"
 #include "gemm_ops.hpp"
@@ -23,105 +30,119 @@ namespace qtg {
 namespace {
 
 // --------------------------------------------------------- hole contraction
-// This wavefront's share [kbeg, kend) of the macro tile (nrb x ncb tiles at
-// columns j0 of the bra, l0 of the ket), KS k-steps of four per stage, the
-// next stage's operands in flight behind the current MFMAs (4 per tile and
-// k-step, 64 cycles each in FP64).  Columns past the tensor are clamped into
-// it (never stored); k past the share reads in range and counts zero.
-template <typename T, int NT, int KS>
-__device__ inline void gc_block_product(const GcDesc& d, int j0, int l0, int nrb, int ncb, int kbeg, int kend,
+// This wavefront's share [kbeg, kend) of NR x NC tiles at columns j0 of the
+// bra and l0 of the ket, KS k-steps of four per stage, the next stage's
+// operands in flight behind the current MFMAs (4 per tile and k-step, 64
+// cycles each in FP64): the loads of a stage stand in straight-line code and
+// nothing touches their values before the stage that uses them.  Columns past
+// the tensor are clamped into it (never stored); only the last, partial stage
+// masks k past the share.
+template <typename T, int NT, int NR, int NC, int KS>
+__device__ inline void gc_block_product(const GcDesc& d, int j0, int l0, int kbeg, int kend,
                                         const cplx<T>* __restrict__ X, const cplx<T>* __restrict__ Y,
                                         typename MF<T>::v4 (&cr)[NT][NT], typename MF<T>::v4 (&ci)[NT][NT]) {
   const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
   const uint32_t bef = (uint32_t)d.bef, aft = (uint32_t)d.aft;
   const uint32_t xs = bef * (uint32_t)d.nx, ys = bef * (uint32_t)d.ny;  // stride of a
   const uint32_t xmax = (bef - 1u) + (aft - 1u) * xs, ymax = (bef - 1u) + (aft - 1u) * ys;
-  uint32_t xrow[NT], yrow[NT];
+  uint32_t xrow[NR], yrow[NC];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    xrow[t] = (uint32_t)min(j0 + t * 16 + li, d.nx - 1) * bef;
-    yrow[t] = (uint32_t)min(l0 + t * 16 + li, d.ny - 1) * bef;
-  }
+  for (int t = 0; t < NR; ++t) xrow[t] = (uint32_t)min(j0 + t * 16 + li, d.nx - 1) * bef;
+#pragma unroll
+  for (int t = 0; t < NC; ++t) yrow[t] = (uint32_t)min(l0 + t * 16 + li, d.ny - 1) * bef;
   const cplx<T>* xp = X + d.x;
   const cplx<T>* yp = Y + d.y;
-  int kc = kbeg + kk;
-  uint32_t b = (uint32_t)kc % bef;
-  const uint32_t a0 = (uint32_t)kc / bef;
+  const int k0 = kbeg + kk;
+  uint32_t b = (uint32_t)k0 % bef;
+  const uint32_t a0 = (uint32_t)k0 / bef;
   uint32_t px = b + a0 * xs, py = b + a0 * ys;
   const uint32_t q4 = 4u / bef, r4 = 4u % bef;
   const uint32_t dx = r4 + q4 * xs, dy = r4 + q4 * ys;
-  auto load = [&](cplx<T>(&xv)[KS][NT], cplx<T>(&yv)[KS][NT]) {
+  auto load = [&](cplx<T>(&xv)[KS][NR], cplx<T>(&yv)[KS][NC]) {
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
-      const bool kv = kc < kend;
       const uint32_t ox = min(px, xmax), oy = min(py, ymax);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        if (t < nrb) {
-          const cplx<T> x = ld32(xp, xrow[t] + ox);
-          xv[u][t] = mk<T>(kv ? x.re : (T)0, kv ? x.im : (T)0);
-        }
-        if (t < ncb) {
-          const cplx<T> y = ld32(yp, yrow[t] + oy);
-          yv[u][t] = mk<T>(kv ? y.re : (T)0, kv ? y.im : (T)0);
-        }
-      }
-      kc += 4;
+      for (int t = 0; t < NR; ++t) xv[u][t] = ld32(xp, xrow[t] + ox);
+#pragma unroll
+      for (int t = 0; t < NC; ++t) yv[u][t] = ld32(yp, yrow[t] + oy);
       b += r4;
-      px += dx;
-      py += dy;
-      if (b >= bef) {
-        b -= bef;
-        px += xs - bef;
-        py += ys - bef;
+      const bool carry = b >= bef;
+      b -= carry ? bef : 0u;
+      px += dx + (carry ? xs - bef : 0u);
+      py += dy + (carry ? ys - bef : 0u);
+    }
+  };
+  auto kstep = [&](const cplx<T>(&xv)[NR], const cplx<T>(&yv)[NC]) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const T nxi = -xv[i].im;
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        cr[i][j] = MF<T>::mma(xv[i].re, yv[j].re, cr[i][j]);
+        ci[i][j] = MF<T>::mma(xv[i].re, yv[j].im, ci[i][j]);
+        cr[i][j] = MF<T>::mma(xv[i].im, yv[j].im, cr[i][j]);
+        ci[i][j] = MF<T>::mma(nxi, yv[j].re, ci[i][j]);
       }
     }
   };
-  // the k-steps of a stage that starts at k0
-  auto steps = [&](int k0, const cplx<T>(&xv)[KS][NT], const cplx<T>(&yv)[KS][NT]) {
+  // one stage that starts at k; the share's last stage masks its tail
+  auto stage = [&](int k, cplx<T>(&xv)[KS][NR], cplx<T>(&yv)[KS][NC]) {
+    if (k + 4 * KS <= kend) {
+#pragma unroll
+      for (int u = 0; u < KS; ++u) kstep(xv[u], yv[u]);
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
-      if (u > 0 && k0 + 4 * u >= kend) break;
+      if (k + 4 * u >= kend) break;
+      const bool kv = k + 4 * u + kk < kend;
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        if (i >= nrb) break;
-        const T nxi = -xv[u][i].im;
+      for (int t = 0; t < NR; ++t) xv[u][t] = mk<T>(kv ? xv[u][t].re : (T)0, kv ? xv[u][t].im : (T)0);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          if (j >= ncb) break;
-          cr[i][j] = MF<T>::mma(xv[u][i].re, yv[u][j].re, cr[i][j]);
-          ci[i][j] = MF<T>::mma(xv[u][i].re, yv[u][j].im, ci[i][j]);
-          cr[i][j] = MF<T>::mma(xv[u][i].im, yv[u][j].im, cr[i][j]);
-          ci[i][j] = MF<T>::mma(nxi, yv[u][j].re, ci[i][j]);
-        }
-      }
+      for (int t = 0; t < NC; ++t) yv[u][t] = mk<T>(kv ? yv[u][t].re : (T)0, kv ? yv[u][t].im : (T)0);
+      kstep(xv[u], yv[u]);
     }
   };
   if (kbeg >= kend) return;
-  cplx<T> xa[KS][NT], ya[KS][NT], xb[KS][NT], yb[KS][NT];
+  cplx<T> xa[KS][NR], ya[KS][NC], xb[KS][NR], yb[KS][NC];
   load(xa, ya);
+  if (kend - kbeg <= 4 * KS) {
+    stage(kbeg, xa, ya);
+    return;
+  }
   for (int k = kbeg; k < kend; k += 8 * KS) {
-    const bool second = k + 4 * KS < kend;
-    if (second) load(xb, yb);
-    steps(k, xa, ya);
-    if (!second) break;
-    if (k + 8 * KS < kend) load(xa, ya);
-    steps(k + 4 * KS, xb, yb);
+    load(xb, yb);
+    stage(k, xa, ya);
+    load(xa, ya);
+    if (k + 4 * KS < kend) stage(k + 4 * KS, xb, yb);
   }
 }
 
-// W wavefronts per workgroup; S workgroups per macro tile.  descs null: the
-// one descriptor `one`.  Otherwise wgdesc[blockIdx.x] names the workgroup's
-// descriptor and tile0 its first workgroup (S = 1).
-template <typename T, typename TO, int NT, int W>
+// W wavefronts per workgroup.  Grouped: wgs[blockIdx.x] names the
+// workgroup's descriptor and its index t within it.  One
+// contraction alone (wgs null): the descriptor `one`, t = blockIdx.x.  The
+// index runs over macro tiles, and per macro tile over the S = ksplit
+// workgroups that share its reduction; with S > 1 each leaves its macro tile
+// in `part` (NT x NT tiles of 256 per workgroup).
+template <typename T, int NT, int W>
 __global__ void __launch_bounds__(64 * W)
-    gc_block(const GcDesc* __restrict__ descs, const int32_t* __restrict__ wgdesc, GcDesc one, int S,
-             const cplx<T>* __restrict__ X0, const cplx<T>* __restrict__ X1, cplx<TO>* O, cplx<TO>* part) {
+    gc_block(const GcDesc* __restrict__ descs, const GcBlockWg* __restrict__ wgs, GcDesc one, int S1,
+             const cplx<T>* __restrict__ X0, const cplx<T>* __restrict__ X1, cplx<T>* O, cplx<T>* part) {
   constexpr int NB = NT > 1 ? 2 : 1;  // LDS buffers: one barrier per tile
-  __shared__ cplx<TO> red[NB * W * 256];
+  __shared__ cplx<T> red[NB * W * 256];
   typedef typename MF<T>::v4 v4;
-  const GcDesc d = descs ? descs[wgdesc[blockIdx.x]] : one;
-  unsigned t = blockIdx.x - (descs ? (unsigned)d.tile0 : 0u);
+  unsigned t = blockIdx.x;
+  int di = 0;
+  int64_t p0 = blockIdx.x;
+  if (wgs) {
+    const GcBlockWg w = wgs[blockIdx.x];
+    di = w.desc;
+    t = (unsigned)w.t;
+    p0 = w.part;
+  }
+  const GcDesc d = wgs ? descs[di] : one;
+  const int S = wgs ? d.ksplit : S1;
   const unsigned s = S > 1 ? t % (unsigned)S : 0u;
   if (S > 1) t /= (unsigned)S;
   const unsigned MJ = (unsigned)(d.nx + 16 * NT - 1) / (16u * NT);
@@ -141,27 +162,32 @@ __global__ void __launch_bounds__(64 * W)
   for (int i = 0; i < NT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) cr[i][j] = ci[i][j] = v4{0, 0, 0, 0};
-  gc_block_product<T, NT, (NT == 1 ? 4 : NT == 2 ? 2 : 1)>(d, j0, l0, nrb, ncb, kbeg, kend, xbase, ybase, cr, ci);
-  const int TJ = (d.nx + 15) >> 4;
+  if constexpr (NT == 1) {
+    gc_block_product<T, 1, 1, 1, 4>(d, j0, l0, kbeg, kend, xbase, ybase, cr, ci);
+  } else {
+    if (nrb == 1 && ncb == 1) gc_block_product<T, NT, 1, 1, 4>(d, j0, l0, kbeg, kend, xbase, ybase, cr, ci);
+    else if (nrb == 1) gc_block_product<T, NT, 1, 2, 2>(d, j0, l0, kbeg, kend, xbase, ybase, cr, ci);
+    else if (ncb == 1) gc_block_product<T, NT, 2, 1, 2>(d, j0, l0, kbeg, kend, xbase, ybase, cr, ci);
+    else gc_block_product<T, NT, 2, 2, 2>(d, j0, l0, kbeg, kend, xbase, ybase, cr, ci);
+  }
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     if (i >= nrb) break;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       if (j >= ncb) break;
-      cplx<TO>* buf = red + (NB > 1 ? ((i * NT + j) & 1) * W * 256 : 0);
+      cplx<T>* buf = red + (NB > 1 ? ((i * NT + j) & 1) * W * 256 : 0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) buf[wave * 256 + q * 64 + lane] = mk<TO>((TO)cr[i][j][q], (TO)ci[i][j][q]);
+      for (int q = 0; q < 4; ++q) buf[wave * 256 + q * 64 + lane] = mk<T>(cr[i][j][q], ci[i][j][q]);
       __syncthreads();
       if (threadIdx.x < 256) {
         const int e = threadIdx.x, el = e & 63, q = e >> 6;
-        cplx<TO> v = buf[e];
+        cplx<T> v = buf[e];
 #pragma unroll
         for (int w = 1; w < W; ++w) v = cadd(v, buf[w * 256 + e]);
         const int row = j0 + i * 16 + MF<T>::drow(el, q), col = l0 + j * 16 + (el & 15);
-        if (part) {
-          const int64_t tile = (int64_t)((l0 >> 4) + j) * TJ + (j0 >> 4) + i;
-          part[(tile * S + s) * 256 + e] = v;
+        if (S > 1) {
+          part[((p0 * NT + j) * NT + i) * 256 + e] = v;
         } else if (row < d.nx && col < d.ny) {
           const int64_t o = d.out + row + (int64_t)col * d.nx;
           if (d.acc) v = cadd(v, O[o]);
@@ -175,28 +201,44 @@ __global__ void __launch_bounds__(64 * W)
   }
 }
 
-// Sums the S partial tiles of every 16 x 16 output tile.  Four workgroups a
-// tile, 64 elements each; a wavefront adds a sixteenth of the partials in
-// order, then the first adds the wavefronts' sums.
+// Sums the S partial macro tiles (2 x 2 tiles) of a macro tile: 16
+// workgroups each, 64 elements a workgroup; a wavefront adds a sixteenth of
+// the partials in order, then the first adds the wavefronts' sums.
+// sums[blockIdx.x / 16]: descriptor, macro tile and its first partial.
 template <typename T>
 __global__ void __launch_bounds__(1024)
-    gc_block_sum(GcDesc d, int S, const cplx<T>* __restrict__ part, cplx<T>* O) {
+    gc_block_sum(const GcDesc* __restrict__ descs, const GcBlockWg* __restrict__ sums, GcDesc one, int S1,
+                 const cplx<T>* __restrict__ part, cplx<T>* O) {
   __shared__ cplx<T> red[15 * 64];
-  const int TJ = (d.nx + 15) >> 4;
-  const unsigned tile = blockIdx.x >> 2;
-  const int lt = (int)(tile / (unsigned)TJ), jt = (int)(tile - (unsigned)lt * TJ);
-  const int lane = threadIdx.x & 63, e = (int)(blockIdx.x & 3) * 64 + lane, g = wave_id();
+  const unsigned b = blockIdx.x >> 4, sub = blockIdx.x & 15u;
+  int di = 0;
+  unsigned macro = b;
+  int64_t p0 = (int64_t)b * S1;
+  if (sums) {
+    const GcBlockWg w = sums[b];
+    di = w.desc;
+    macro = (unsigned)w.t;
+    p0 = w.part;
+  }
+  const GcDesc d = sums ? descs[di] : one;
+  const int S = sums ? d.ksplit : S1;
+  const unsigned MJ = (unsigned)(d.nx + 31) / 32u;
+  const unsigned lm = macro / MJ, jm = macro - lm * MJ;
+  const int tile = (int)(sub >> 2), i = tile & 1, j = tile >> 1;
+  const int lane = threadIdx.x & 63, e = (int)(sub & 3u) * 64 + lane, g = wave_id();
+  const int r0 = (int)jm * 32 + i * 16, c0 = (int)lm * 32 + j * 16;
+  if (r0 >= d.nx || c0 >= d.ny) return;  // the whole workgroup
   const int per = (S + 15) >> 4, s0 = min(S, g * per), s1 = min(S, s0 + per);
-  const cplx<T>* p = part + (int64_t)tile * S * 256 + e;
+  const cplx<T>* p = part + (p0 * 4 + tile) * 256 + e;
   cplx<T> v = czero<T>();
 #pragma unroll 8
-  for (int s = s0; s < s1; ++s) v = cadd(v, p[(int64_t)s * 256]);
+  for (int s = s0; s < s1; ++s) v = cadd(v, p[(int64_t)s * 1024]);
   if (g > 0) red[(g - 1) * 64 + lane] = v;
   __syncthreads();
   if (g > 0) return;
 #pragma unroll
   for (int k = 0; k < 15; ++k) v = cadd(v, red[k * 64 + lane]);
-  const int row = jt * 16 + MF<T>::drow(lane, e >> 6), col = lt * 16 + (lane & 15);
+  const int row = r0 + MF<T>::drow(lane, e >> 6), col = c0 + (lane & 15);
   if (row < d.nx && col < d.ny) {
     const int64_t o = d.out + row + (int64_t)col * d.nx;
     if (d.acc) v = cadd(v, O[o]);
@@ -204,7 +246,186 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
+// ------------------------------------------------------------- mode product
+// out(b,i,a) = alpha sum_l op(M)(i,l) X(b,l,a) (+ out) on RB x CB tiles of
+// 16 rows (flattened (b, a)) x 16 columns i, KS k-steps of four per stage,
+// staged as in gc_block_product.  TR (bef >= 4): accumulated transposed, so a
+// lane holds one row and the 16 lanes of a store write 16 consecutive
+// elements.  Rows and columns past the range are clamped into it (never
+// stored); the last, partial stage masks X past K.
+template <typename T, typename TM, typename TO, int RB, int CB, int KS, bool TR>
+__device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, const cplx<T>* __restrict__ X,
+                                      const cplx<TM>* __restrict__ M, cplx<TO>* O, double sre, double sim) {
+  typedef typename MF<T>::v4 v4;
+  const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
+  const uint32_t bef = (uint32_t)d.bef, R = bef * (uint32_t)d.aft;
+  const int nin = d.nin, nout = d.nout;
+  uint32_t xrow[RB], mrow[CB];
+#pragma unroll
+  for (int t = 0; t < RB; ++t) {
+    const uint32_t r = min(r0 + (uint32_t)(t * 16 + li), R - 1u);
+    const uint32_t a = r / bef;
+    xrow[t] = (r - a * bef) + a * bef * (uint32_t)nin;
+  }
+  const uint32_t mks = d.op == GM_N ? (uint32_t)nout : 1u;
+  const T msign = d.op == GM_H ? (T)-1 : (T)1;
+#pragma unroll
+  for (int t = 0; t < CB; ++t) {
+    const int j = min(c0 + t * 16 + li, nout - 1);
+    mrow[t] = d.op == GM_N ? (uint32_t)j : (uint32_t)j * (uint32_t)nin;
+  }
+  const cplx<T>* xp = X + d.x;
+  const cplx<TM>* mp = M + d.m;
+  v4 cr[RB][CB], ci[RB][CB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) cr[i][j] = ci[i][j] = v4{0, 0, 0, 0};
+  auto load = [&](int k, cplx<T>(&xv)[KS][RB], cplx<TM>(&mv)[KS][CB]) {
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+      const uint32_t kc = (uint32_t)min(k + 4 * u + kk, nin - 1);
+      const uint32_t ox = kc * bef, om = kc * mks;
+#pragma unroll
+      for (int t = 0; t < RB; ++t) xv[u][t] = ld32(xp, xrow[t] + ox);
+#pragma unroll
+      for (int t = 0; t < CB; ++t) mv[u][t] = ld32(mp, mrow[t] + om);
+    }
+  };
+  auto kstep = [&](const cplx<T>(&xv)[RB], const cplx<TM>(&mv)[CB]) {
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      const T mr = (T)mv[j].re, mi = msign * (T)mv[j].im;
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        const T nxi = -xv[i].im;
+        if constexpr (TR) {
+          cr[i][j] = MF<T>::mma(mr, xv[i].re, cr[i][j]);
+          ci[i][j] = MF<T>::mma(mr, xv[i].im, ci[i][j]);
+          cr[i][j] = MF<T>::mma(mi, nxi, cr[i][j]);
+          ci[i][j] = MF<T>::mma(mi, xv[i].re, ci[i][j]);
+        } else {
+          cr[i][j] = MF<T>::mma(xv[i].re, mr, cr[i][j]);
+          ci[i][j] = MF<T>::mma(xv[i].im, mr, ci[i][j]);
+          cr[i][j] = MF<T>::mma(nxi, mi, cr[i][j]);
+          ci[i][j] = MF<T>::mma(xv[i].re, mi, ci[i][j]);
+        }
+      }
+    }
+  };
+  auto stage = [&](int k, cplx<T>(&xv)[KS][RB], const cplx<TM>(&mv)[KS][CB]) {
+    if (k + 4 * KS <= nin) {
+#pragma unroll
+      for (int u = 0; u < KS; ++u) kstep(xv[u], mv[u]);
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+      if (k + 4 * u >= nin) break;
+      const bool kv = k + 4 * u + kk < nin;
+#pragma unroll
+      for (int t = 0; t < RB; ++t) xv[u][t] = mk<T>(kv ? xv[u][t].re : (T)0, kv ? xv[u][t].im : (T)0);
+      kstep(xv[u], mv[u]);
+    }
+  };
+  cplx<T> xa[KS][RB], xb[KS][RB];
+  cplx<TM> ma[KS][CB], mb[KS][CB];
+  load(0, xa, ma);
+  for (int k = 0; k < nin; k += 8 * KS) {
+    load(k + 4 * KS, xb, mb);
+    stage(k, xa, ma);
+    load(k + 8 * KS, xa, ma);
+    if (k + 4 * KS < nin) stage(k + 4 * KS, xb, mb);
+  }
+  const double fre = d.are * sre - d.aim * sim, fim = d.are * sim + d.aim * sre;
+  const bool one = fre == 1.0 && fim == 0.0;
+  const T are = (T)fre, aim = (T)fim;
+  cplx<TO>* ob = O + d.out;
+#pragma unroll
+  for (int i = 0; i < RB; ++i) {
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t r = r0 + (uint32_t)(i * 16 + (TR ? li : MF<T>::drow(lane, q)));
+        const int col = c0 + j * 16 + (TR ? MF<T>::drow(lane, q) : li);
+        if (r < R && col < nout) {
+          const uint32_t a = r / bef;
+          cplx<TO>* o = at32(ob, (r - a * bef) + (uint32_t)col * bef + a * bef * (uint32_t)nout);
+          const T vr = cr[i][j][q], vi = ci[i][j][q];
+          cplx<TO> v = one ? mk<TO>((TO)vr, (TO)vi) : mk<TO>((TO)(are * vr - aim * vi), (TO)(are * vi + aim * vr));
+          if (d.acc) v = cadd(v, *o);
+          *o = v;
+        }
+      }
+    }
+  }
+}
+
+// Four tasks (wavefronts) per workgroup; wgdesc null: one descriptor per
+// task.  A task is 2 x 2 tiles; its last column block may hold one column.
+template <typename T, typename TM, typename TO>
+__global__ void __launch_bounds__(256)
+    gm_block(const GmDesc* __restrict__ descs, const int32_t* __restrict__ wgdesc, int64_t ntasks,
+             const cplx<T>* __restrict__ X0, const cplx<T>* __restrict__ X1, const cplx<TM>* __restrict__ M,
+             cplx<TO>* O, const uint8_t* __restrict__ active, double sre, double sim) {
+  const int64_t task = (int64_t)blockIdx.x * 4 + wave_id();
+  if (task >= ntasks) return;
+  const GmDesc d = descs[wgdesc ? (int64_t)wgdesc[task] : task];
+  if (active && d.node >= 0 && !active[d.node]) return;
+  const uint32_t t = (uint32_t)(task - d.tile0);
+  const uint32_t CT = (uint32_t)(d.nout + 31) / 32u;
+  const uint32_t rt = CT == 1 ? t : t / CT;
+  const int c0 = (int)(t - rt * CT) * 32;
+  const uint32_t r0 = rt * 32u;
+  const bool two = d.nout - c0 > 16;
+  const cplx<T>* X = d.xsel ? X1 : X0;
+  if (d.bef >= 4) {
+    if (two) gm_block_tiles<T, TM, TO, 2, 2, 1, true>(d, r0, c0, X, M, O, sre, sim);
+    else gm_block_tiles<T, TM, TO, 2, 1, 1, true>(d, r0, c0, X, M, O, sre, sim);
+  } else {
+    if (two) gm_block_tiles<T, TM, TO, 2, 2, 1, false>(d, r0, c0, X, M, O, sre, sim);
+    else gm_block_tiles<T, TM, TO, 2, 1, 1, false>(d, r0, c0, X, M, O, sre, sim);
+  }
+}
+
 }  // namespace
+
+template <typename T, typename TM, typename TO>
+int launch_gm_block(const GmDesc* descs, const int32_t* wgdesc, int64_t ntasks, const void* x0, const void* x1,
+                    const void* mbase, void* obase, const uint8_t* active, double sre, double sim, hipStream_t s,
+                    const KernelTiming* kt) {
+  if (ntasks <= 0) return QTG_OK;
+  launch_timed(gm_block<T, TM, TO>, dim3((unsigned)((ntasks + 3) / 4)), dim3(256), 0, s, kt, descs, wgdesc, ntasks,
+               (const cplx<T>*)x0, (const cplx<T>*)x1, (const cplx<TM>*)mbase, (cplx<TO>*)obase, active, sre, sim);
+  QTG_LAUNCH_CHECK();
+  return QTG_OK;
+}
+#define QTG_GM(T, TM, TO)                                                                                       \
+  template int launch_gm_block<T, TM, TO>(const GmDesc*, const int32_t*, int64_t, const void*, const void*,      \
+                                          const void*, void*, const uint8_t*, double, double, hipStream_t,       \
+                                          const KernelTiming*);
+QTG_GM(double, double, double)
+QTG_GM(float, float, float)
+#undef QTG_GM
+
+template <typename T>
+int launch_gc_block(const GcDesc* descs, const GcBlockWg* wgs, int64_t nwg, const GcBlockWg* sums, int64_t nsums,
+                    const void* x0, const void* x1, void* obase, void* part, hipStream_t s) {
+  if (nwg <= 0) return QTG_OK;
+  const GcDesc none{};
+  hipLaunchKernelGGL((gc_block<T, 2, 4>), dim3((unsigned)nwg), dim3(256), 0, s, descs, wgs, none, 1,
+                     (const cplx<T>*)x0, (const cplx<T>*)x1, (cplx<T>*)obase, (cplx<T>*)part);
+  if (nsums > 0)
+    hipLaunchKernelGGL(gc_block_sum<T>, dim3((unsigned)(16 * nsums)), dim3(1024), 0, s, descs, sums, none, 1,
+                       (const cplx<T>*)part, (cplx<T>*)obase);
+  QTG_LAUNCH_CHECK();
+  return QTG_OK;
+}
+template int launch_gc_block<double>(const GcDesc*, const GcBlockWg*, int64_t, const GcBlockWg*, int64_t, const void*,
+                                     const void*, void*, void*, hipStream_t);
+template int launch_gc_block<float>(const GcDesc*, const GcBlockWg*, int64_t, const GcBlockWg*, int64_t, const void*,
+                                    const void*, void*, void*, hipStream_t);
 
 // A reduction of up to kOneWgK elements stays in one workgroup per tile: its
 // 16 wavefronts take 14 us at K = 576 (24 x 24 output), where two launches
@@ -218,22 +439,22 @@ __global__ void __launch_bounds__(1024)
 GcOnePlan plan_gc_one(const GcDesc& d, int64_t max_part_elems) {
   constexpr int64_t kOneWgK = 768;
   const int64_t K = (int64_t)d.bef * d.aft;
+  const int64_t m2 = gc_block_macros(d);
   GcOnePlan p{};
-  p.tiles = (int64_t)((d.nx + 15) / 16) * ((d.ny + 15) / 16);
   p.S = 1;
-  const int64_t m2 = (int64_t)((d.nx + 31) / 32) * ((d.ny + 31) / 32);
   if (K > kOneWgK) {
     int64_t S = std::min<int64_t>((512 + m2 - 1) / m2, K / 128);
-    S = std::min<int64_t>(S, max_part_elems / (p.tiles * 256));
+    S = std::min<int64_t>(S, max_part_elems / (m2 * 1024));
+    // workgroup macro * S + s: with 8 | S the macro tiles of a share, which
+    // read the same operands, land on one XCD (blockIdx mod 8)
+    if (S > 8) S &= ~(int64_t)7;
     if (S > 1) {
-      p.nt = 2;
       p.S = (int)S;
       p.macro = m2;
       return p;
     }
   }
-  p.nt = 1;
-  p.macro = p.tiles;
+  p.macro = (int64_t)((d.nx + 15) / 16) * ((d.ny + 15) / 16);
   return p;
 }
 
@@ -242,21 +463,24 @@ int launch_gc_one(const GcDesc& d, const GcOnePlan& p, const void* x, const void
                   hipStream_t s) {
   const cplx<T>* X = (const cplx<T>*)x;
   const cplx<T>* Y = (const cplx<T>*)y;
-  if (p.nt == 1) {
-    hipLaunchKernelGGL((gc_block<T, T, 1, 16>), dim3((unsigned)p.macro), dim3(1024), 0, s, (const GcDesc*)nullptr,
-                       (const int32_t*)nullptr, d, 1, X, Y, (cplx<T>*)o, (cplx<T>*)nullptr);
+  if (p.S > 1 && !part) {
+    set_error("single hole contraction: a split over workgroups needs its partial tiles");
+    return QTG_EARG;
+  }
+  const GcDesc* nd = nullptr;
+  const GcBlockWg* nw = nullptr;
+  if (p.S == 1 && (int64_t)d.bef * d.aft <= 128) {
+    // short reductions: four wavefronts, the launch itself decides
+    hipLaunchKernelGGL((gc_block<T, 1, 4>), dim3((unsigned)p.macro), dim3(256), 0, s, nd, nw, d, 1, X, Y, (cplx<T>*)o,
+                       (cplx<T>*)nullptr);
+  } else if (p.S == 1) {
+    hipLaunchKernelGGL((gc_block<T, 1, 16>), dim3((unsigned)p.macro), dim3(1024), 0, s, nd, nw, d, 1, X, Y,
+                       (cplx<T>*)o, (cplx<T>*)nullptr);
   } else {
-    const bool split = p.S > 1;
-    if (split && !part) {
-      set_error("single hole contraction: a split over workgroups needs its partial tiles");
-      return QTG_EARG;
-    }
-    hipLaunchKernelGGL((gc_block<T, T, 2, 4>), dim3((unsigned)(p.macro * p.S)), dim3(256), 0, s,
-                       (const GcDesc*)nullptr, (const int32_t*)nullptr, d, p.S, X, Y, (cplx<T>*)o,
-                       split ? (cplx<T>*)part : (cplx<T>*)nullptr);
-    if (split)
-      hipLaunchKernelGGL(gc_block_sum<T>, dim3((unsigned)(4 * p.tiles)), dim3(1024), 0, s, d, p.S, (const cplx<T>*)part,
-                         (cplx<T>*)o);
+    hipLaunchKernelGGL((gc_block<T, 2, 4>), dim3((unsigned)(p.macro * p.S)), dim3(256), 0, s, nd, nw, d, p.S, X, Y,
+                       (cplx<T>*)o, (cplx<T>*)part);
+    hipLaunchKernelGGL(gc_block_sum<T>, dim3((unsigned)(16 * p.macro)), dim3(1024), 0, s, nd, nw, d, p.S,
+                       (const cplx<T>*)part, (cplx<T>*)o);
   }
   QTG_LAUNCH_CHECK();
   return QTG_OK;

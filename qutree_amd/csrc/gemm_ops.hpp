@@ -160,15 +160,42 @@ int launch_gm_single(const GmDesc& d, const void* x, const void* m, void* o, hip
 template <typename T>
 int launch_gc_single(const GcDesc& d, const void* x, const void* y, void* o, hipStream_t s);
 
+// Register-blocked forms (gemm_block.hip) for launches that fill the card;
+// every descriptor passes gm_lean_ok / gc_lean_ok and is no GM_COPY.
+// Mode product: 32 x 32 outputs a wavefront, no K split; tile0 and the table
+// count wavefront tasks.
+inline int64_t gm_block_tasks(const GmDesc& d) {
+  const int64_t R = (int64_t)d.bef * d.aft;
+  return ((R + 31) / 32) * ((d.nout + 31) / 32);
+}
+template <typename T, typename TM, typename TO>
+int launch_gm_block(const GmDesc* descs, const int32_t* wgdesc, int64_t ntasks, const void* x0, const void* x1,
+                    const void* mbase, void* obase, const uint8_t* active, double sre, double sim, hipStream_t s,
+                    const KernelTiming* kt = nullptr);
+// Hole contraction: a workgroup per 32 x 32 macro tile and share of the
+// reduction (ksplit shares, workgroups t = macro * ksplit + share of the
+// descriptor).  A workgroup with shares writes 1024 elements at 1024 * part;
+// sums[] then holds a macro tile each (t: macro tile, part: its first
+// partial; the shares' partials follow one another).
+struct GcBlockWg {
+  int32_t desc, t, part, pad;
+};
+inline int64_t gc_block_macros(const GcDesc& d) {
+  return (int64_t)((d.nx + 31) / 32) * ((d.ny + 31) / 32);
+}
+template <typename T>
+int launch_gc_block(const GcDesc* descs, const GcBlockWg* wgs, int64_t nwg, const GcBlockWg* sums, int64_t nsums,
+                    const void* x0, const void* x1, void* obase, void* part, hipStream_t s);
+
 // One hole contraction alone on the card (gemm_block.hip), for descriptors
-// with gc_lean_ok.  nt 1: a workgroup of 16 wavefronts per 16 x 16 tile, each
-// on a sixteenth of K.  nt 2: 32 x 32 macro tiles, four wavefronts, K split
-// over S workgroups as well when S > 1; the S partial tiles (part_elems()
-// complex elements, caller's buffer) are then summed by a second launch.
+// with gc_lean_ok.  S 1: a workgroup of 16 wavefronts per 16 x 16 tile, each
+// on a sixteenth of K.  S > 1: S workgroups per 32 x 32 macro tile; their
+// partial tiles (part_elems() complex elements, caller's buffer) are then
+// summed by a second launch.
 struct GcOnePlan {
-  int nt, S;
-  int64_t macro, tiles;  // macro tiles, 16 x 16 tiles
-  int64_t part_elems() const { return S > 1 ? tiles * S * 256 : 0; }
+  int S;
+  int64_t macro;  // workgroups per share
+  int64_t part_elems() const { return S > 1 ? macro * S * 1024 : 0; }
 };
 GcOnePlan plan_gc_one(const GcDesc& d, int64_t max_part_elems);
 template <typename T>

@@ -8,6 +8,8 @@
 // their workgroup, in chunk order (deterministic).
 #include <algorithm>
 #include <climits>
+#include <cmath>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -95,16 +97,34 @@ int mode_product_one(const qtg_mode_product_desc& d, cplx<R>* C, const cplx<R>* 
   return launch_gm_single<R>(g, B, M, C, s);
 }
 
+// A plan: descriptors [0, nblock) run in a register-blocked kernel
+// (gemm_block.hip), the rest in a general grouped kernel.
 struct Plan {
   int kind = 0;  // 0 mode product, 1 hole contraction
   bool c64 = false;
-  int64_t ndesc = 0, ntasks = 0;
+  int64_t nblock = 0, block_tasks = 0, nsums = 0;
+  int64_t ngen = 0, gen_tasks = 0;
+  bool gen_lean = false;  // every general descriptor takes the lean form
   void* d_descs = nullptr;
-  void* d_wg = nullptr;  // first descriptor of every workgroup
+  void* d_block = nullptr;  // gm_block: descriptor of every task; gc_block: GcBlockWg of every workgroup, then the sums
+  void* d_wg = nullptr;     // general kernel: descriptor of every task
   double flops = 0, bytes = 0;
+  // Shared reductions (nsums > 0): their partial macro tiles, which an
+  // execution uses from its first launch to its last.  Executions are ordered
+  // by `done`, recorded behind each, so one on another stream waits; under
+  // capture the plan runs unshared (d_descs1, d_block1: a workgroup per macro
+  // tile), since a replay could not be ordered.
+  void* d_part = nullptr;
+  void* d_descs1 = nullptr;
+  void* d_block1 = nullptr;
+  int64_t block_tasks1 = 0;
+  std::mutex mu;
+  hipEvent_t done = nullptr;
+  bool used = false;
   ~Plan() {
-    for (void* p : {d_descs, d_wg})
+    for (void* p : {d_descs, d_block, d_wg, d_part, d_descs1, d_block1})
       if (p) (void)hipFree(p);
+    if (done) (void)hipEventDestroy(done);
   }
 };
 
@@ -117,14 +137,179 @@ int upload(void** dst, const std::vector<X>& v) {
   return QTG_OK;
 }
 
+// The descriptors of the blocked kernel come first; uploads all tables.
+template <typename D>
+int finish_plan(Plan& p, std::vector<D>& block, std::vector<D>& gen, int64_t (*tasks)(const D&),
+                bool (*lean_ok)(const D&)) {
+  std::vector<int32_t> wg;
+  p.nblock = (int64_t)block.size();
+  p.ngen = (int64_t)gen.size();
+  p.gen_tasks = order_tasks(gen, tasks);
+  p.gen_lean = std::all_of(gen.begin(), gen.end(), lean_ok);
+  gemm_wg_table(gen.data(), p.ngen, p.gen_tasks, wg);
+  block.insert(block.end(), gen.begin(), gen.end());
+  int rc = upload(&p.d_descs, block);
+  if (!rc) rc = upload(&p.d_wg, wg);
+  return rc;
+}
+
+// Mode products of more than 16 columns take 32 x 32 outputs a wavefront
+// when the plan then still has kMinBlockTasks wavefronts (eight a SIMD):
+// 500 tensors of legs 17-48 221 -> 195 us, 49-64 1300 -> 1023 us (complex128),
+// 852 -> 643 us (complex64).  Below, and for up to 16 columns, one 16 x 16
+// tile a wavefront is the faster form: 16 tensors of legs 8-64 14.5 against
+// 19.5 us, 2000 of legs 3-20 25.9 against 33 us.
+constexpr int64_t kMinBlockTasks = 8192;
+bool gm_blocked(const GmDesc& g) { return gm_lean_ok(g) && g.nout > 16; }
+
+// A hole contraction of a plan: blocked where its offsets fit 32 bits.
+void add_gc(GcDesc& g, std::vector<GcDesc>& block, std::vector<GcDesc>& gen) {
+  if (gc_lean_ok(g)) {
+    block.push_back(g);
+    return;
+  }
+  const int64_t K = (int64_t)g.bef * g.aft;
+  if (K > 2 * kSplitK) g.ksplit = split_chunks(K, kGemmWaves, 1);
+  gen.push_back(g);
+}
+
+// The workgroups of the blocked hole contractions: every reduction in
+// `ksplit` shares, toward about kTargetWgs workgroups of equal work in all
+// (two per CU) and at least kMinShare elements each (a share costs a 16 KB
+// partial tile where it reads 64 columns).  The macro tiles of a share read
+// the same operands, so they go to one XCD (workgroup index mod 8), where
+// they meet in its L2: 1204 -> 1086 us for 4096 tensors of legs 8-64, 1279
+// -> 984 us for 1000 of legs 33-48.  The shares are dealt to the XCD with the
+// least work so far, the heaviest first, so the launch also ends with its
+// short workgroups; where a queue has run out the others close up, which
+// moves only the lightest units.
+struct GcBlockPlan {
+  std::vector<GcBlockWg> wgs, sums;
+  int64_t parts = 0;  // partial macro tiles
+};
+constexpr int64_t kTargetWgs = 512;
+GcBlockPlan plan_gc_blocks(std::vector<GcDesc>& v, int64_t targetWgs = kTargetWgs) {
+  constexpr int kXcds = 8;
+  constexpr int64_t kMinShare = 256;
+  GcBlockPlan p;
+  auto work = [](const GcDesc& d) {
+    return (double)d.bef * d.aft * ((d.nx + 15) / 16) * ((d.ny + 15) / 16);
+  };
+  double total = 0.0;
+  for (auto& d : v) total += work(d);
+  struct Unit {
+    double w;
+    int32_t desc, share, part;
+  };
+  std::vector<Unit> units;
+  for (size_t i = 0; i < v.size(); ++i) {
+    GcDesc& d = v[i];
+    const int64_t K = (int64_t)d.bef * d.aft, m = gc_block_macros(d);
+    // m shares of more than total / kTargetWgs each: the partial tiles of a
+    // plan stay below 2 kTargetWgs
+    const int64_t want = (int64_t)std::ceil(work(d) / (double)m * (double)targetWgs / total);
+    d.ksplit = (int32_t)std::max<int64_t>(1, std::min(want, K / kMinShare));
+    for (int32_t s = 0; s < d.ksplit; ++s) units.push_back({work(d) / d.ksplit, (int32_t)i, s, (int32_t)p.parts});
+    if (d.ksplit > 1) {
+      for (int64_t t = 0; t < m; ++t) p.sums.push_back({(int32_t)i, (int32_t)t, (int32_t)(p.parts + t * d.ksplit), 0});
+      p.parts += m * d.ksplit;
+    }
+  }
+  std::stable_sort(units.begin(), units.end(), [](const Unit& a, const Unit& b) { return a.w > b.w; });
+  std::vector<GcBlockWg> q[kXcds];
+  double load[kXcds] = {};
+  for (const Unit& u : units) {
+    const int x = (int)(std::min_element(load, load + kXcds) - load);
+    load[x] += u.w;
+    const GcDesc& d = v[u.desc];
+    const int64_t m = gc_block_macros(d);
+    for (int64_t t = 0; t < m; ++t)
+      q[x].push_back({u.desc, (int32_t)(t * d.ksplit + u.share), (int32_t)(u.part + t * d.ksplit + u.share), 0});
+  }
+  size_t len = 0;
+  for (auto& x : q) len = std::max(len, x.size());
+  for (size_t k = 0; k < len; ++k)
+    for (auto& x : q)
+      if (k < x.size()) p.wgs.push_back(x[k]);
+  return p;
+}
+
+int upload_gc_blocks(Plan& p, std::vector<GcDesc>& v) {
+  if (v.empty()) return QTG_OK;
+  GcBlockPlan g = plan_gc_blocks(v);
+  p.block_tasks = (int64_t)g.wgs.size();
+  p.nsums = (int64_t)g.sums.size();
+  g.wgs.insert(g.wgs.end(), g.sums.begin(), g.sums.end());
+  if (g.parts > 0) {
+    const size_t es = p.c64 ? sizeof(cplx<float>) : sizeof(cplx<double>);
+    if (hipMalloc(&p.d_part, (size_t)g.parts * 1024 * es) != hipSuccess) {
+      (void)hipGetLastError();
+      p.d_part = nullptr;
+      set_error("plan: device allocation of the partial tiles failed");
+      return QTG_ENOMEM;
+    }
+    QTG_HIP_TRY(hipEventCreateWithFlags(&p.done, hipEventDisableTiming));
+    std::vector<GcDesc> one = v;
+    const GcBlockPlan g1 = plan_gc_blocks(one, 0);
+    p.block_tasks1 = (int64_t)g1.wgs.size();
+    int rc = upload(&p.d_descs1, one);
+    if (!rc) rc = upload(&p.d_block1, g1.wgs);
+    if (rc) return rc;
+  }
+  return upload(&p.d_block, g.wgs);
+}
+
+// (a query that fails counts as a capture: the launches then need no ordering)
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+template <typename T>
+int run_plan(Plan& p, void* out, const void* first, const void* second, hipStream_t s) {
+  int rc = QTG_OK;
+  if (p.kind == 0) {
+    // first = M base, second = B base
+    const GmDesc* g = (const GmDesc*)p.d_descs;
+    rc = launch_gm_block<T, T, T>(g, (const int32_t*)p.d_block, p.block_tasks, second, second, first, out, nullptr,
+                                  1.0, 0.0, s);
+    if (rc) return rc;
+    return launch_gm<T, T, T>(g + p.nblock, (const int32_t*)p.d_wg, p.ngen, p.gen_tasks, second, second, first, out,
+                              nullptr, 1.0, 0.0, s, nullptr, kGemmWaves, p.gen_lean);
+  }
+  // X (bra) from the first base, Y (ket) from the second: sel = 2 on every descriptor
+  const GcDesc* g = (const GcDesc*)p.d_descs;
+  const GcBlockWg* wgs = (const GcBlockWg*)p.d_block;
+  if (p.nsums == 0) {
+    rc = launch_gc_block<T>(g, wgs, p.block_tasks, wgs, 0, first, second, out, nullptr, s);
+  } else if (capturing(s)) {
+    const GcBlockWg* w1 = (const GcBlockWg*)p.d_block1;
+    rc = launch_gc_block<T>((const GcDesc*)p.d_descs1, w1, p.block_tasks1, w1, 0, first, second, out, nullptr, s);
+  } else {
+    std::lock_guard<std::mutex> lock(p.mu);
+    if (p.used) QTG_HIP_TRY(hipStreamWaitEvent(s, p.done, 0));
+    p.used = true;
+    rc = launch_gc_block<T>(g, wgs, p.block_tasks, wgs + p.block_tasks, p.nsums, first, second, out, p.d_part, s);
+    QTG_HIP_TRY(hipEventRecord(p.done, s));
+  }
+  if (rc) return rc;
+  return launch_gc<T, T>(g + p.nblock, (const int32_t*)p.d_wg, p.ngen, p.gen_tasks, first, second, out, nullptr, s,
+                         nullptr, p.gen_lean);
+}
+
 // ------------------------------------------------ no-allocation variant
 // Device-resident staging of qtg_hole_contraction_grouped_noalloc_z: the
-// converted descriptors, then the per-task descriptor index table.  Each GPU
-// holds its own copy for the life of the process.
+// converted descriptors, then the tables of a plan: the workgroups of the
+// blocked kernel (at most one per 16 x 16 tile and 2 kTargetWgs shares) and
+// its sums, or, for descriptors beyond the blocked kernel's 32-bit offsets,
+// the descriptor of every task.  Each GPU holds its own copy for the life of
+// the process.
 constexpr int64_t kNoAllocMaxDescs = 4096;
 constexpr int64_t kNoAllocMaxTasks = 1 << 18;
 constexpr size_t kNoAllocTableOff = (size_t)kNoAllocMaxDescs * sizeof(GcDesc);
-constexpr size_t kNoAllocBytes = kNoAllocTableOff + (size_t)kNoAllocMaxTasks * sizeof(int32_t);
+constexpr size_t kNoAllocBytes = kNoAllocTableOff + (size_t)(kNoAllocMaxTasks + 4 * kTargetWgs) * sizeof(GcBlockWg);
 static_assert(kNoAllocTableOff % 256 == 0, "table alignment");
 
 }  // namespace
@@ -217,6 +402,21 @@ int hole_split(const GcDesc& g, const GcOnePlan& p, const cplx<R>* A, const cplx
   return rc;
 }
 
+// launch(base) with the slots as one buffer, behind their last uses; launch
+// returns when its work on the device is done.
+template <typename F>
+int with_all_parts(hipStream_t s, F&& launch) {
+  int dev = 0;
+  QTG_HIP_TRY(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(g_parts.mu);
+  void* base = nullptr;
+  int rc = symbol_address(HIP_SYMBOL(part_scratch), dev, g_parts.base, "hole contraction", &base);
+  if (rc) return rc;
+  for (int i = 0; i < kPartSlots; ++i)
+    if (g_parts.used[dev][i]) QTG_HIP_TRY(hipStreamWaitEvent(s, g_parts.ev[dev][i], 0));
+  return launch(base);
+}
+
 // Reductions long enough for it split over workgroups (plan_gc_one), except
 // under stream capture: a replayed graph would use its slot unordered with
 // other calls.
@@ -231,13 +431,7 @@ int hole_one(const qtg_hole_contraction_desc& d, cplx<R>* Sm, const cplx<R>* A, 
   if (rc) return rc;
   if (!gc_lean_ok(g)) return launch_gc_single<R>(g, A, B, Sm, s);
   GcOnePlan p = plan_gc_one(g, (int64_t)(kPartBytes / sizeof(cplx<R>)));
-  if (p.S > 1) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      p = plan_gc_one(g, 0);
-    }
-  }
+  if (p.S > 1 && capturing(s)) p = plan_gc_one(g, 0);
   if (p.S > 1) return hole_split<R>(g, p, A, B, Sm, s);
   return launch_gc_one<R>(g, p, A, B, Sm, nullptr, s);
 }
@@ -320,37 +514,35 @@ int qtg_mode_product_plan_create(qtg_plan* plan, const qtg_mode_product_desc* de
     set_error("plan: bad arguments");
     return QTG_EARG;
   }
-  auto* p = new Plan();
+  std::unique_ptr<Plan> p(new Plan());
   p->kind = 0;
   p->c64 = complex64 != 0;
   const double es = p->c64 ? 8.0 : 16.0;
-  std::vector<GmDesc> gv;
-  int64_t tasks = 0;
+  std::vector<GmDesc> block, gen;
   for (int64_t i = 0; i < count; ++i) {
     GmDesc g;
     int rc = to_gm(descs[i], g);
-    if (rc) {
-      delete p;
-      return rc;
-    }
-    g.tile0 = tasks;
-    tasks += gm_tasks(g);
-    gv.push_back(g);
+    if (rc) return rc;
+    (gm_blocked(g) ? block : gen).push_back(g);
     const auto& d = descs[i];
     p->flops += 8.0 * d.before * d.after * d.nB * d.nC;
     p->bytes += es * (d.before * d.after * (d.nB + d.nC * (d.add ? 2 : 1)) + d.nB * d.nC);
   }
-  std::vector<int32_t> wg;
-  gemm_wg_table(gv.data(), (int64_t)gv.size(), tasks, wg);
-  int rc = upload(&p->d_descs, gv);
-  if (!rc) rc = upload(&p->d_wg, wg);
-  if (rc) {
-    delete p;
-    return rc;
+  for (auto& g : block) {
+    g.tile0 = p->block_tasks;
+    p->block_tasks += gm_block_tasks(g);
   }
-  p->ndesc = count;
-  p->ntasks = tasks;
-  *plan = p;
+  if (p->block_tasks < kMinBlockTasks) {
+    gen.insert(gen.begin(), block.begin(), block.end());
+    block.clear();
+    p->block_tasks = 0;
+  }
+  std::vector<int32_t> wg;
+  gemm_wg_table(block.data(), (int64_t)block.size(), p->block_tasks, wg);
+  int rc = upload(&p->d_block, wg);
+  if (!rc) rc = finish_plan<GmDesc>(*p, block, gen, gm_tasks, gm_lean_ok);
+  if (rc) return rc;
+  *plan = p.release();
   return QTG_OK;
 }
 
@@ -360,37 +552,25 @@ int qtg_hole_contraction_plan_create(qtg_plan* plan, const qtg_hole_contraction_
     set_error("plan: bad arguments");
     return QTG_EARG;
   }
-  auto* p = new Plan();
+  std::unique_ptr<Plan> p(new Plan());
   p->kind = 1;
   p->c64 = complex64 != 0;
   const double es = p->c64 ? 8.0 : 16.0;
-  std::vector<GcDesc> gv;
+  std::vector<GcDesc> block, gen;
   for (int64_t i = 0; i < count; ++i) {
     GcDesc g;
     int rc = to_gc(descs[i], g);
-    if (rc) {
-      delete p;
-      return rc;
-    }
-    const int64_t K = (int64_t)g.bef * g.aft;
-    if (K > 2 * kSplitK) g.ksplit = split_chunks(K, kGemmWaves, 1);
-    gv.push_back(g);
+    if (rc) return rc;
+    add_gc(g, block, gen);
     const auto& d = descs[i];
+    const int64_t K = d.before * d.after;
     p->flops += 8.0 * K * d.nA * d.nB;
     p->bytes += es * (K * (d.nA + d.nB) + d.nA * d.nB * (d.accumulate ? 2 : 1));
   }
-  const int64_t tasks = order_tasks(gv, gc_tasks);
-  std::vector<int32_t> wg;
-  gemm_wg_table(gv.data(), (int64_t)gv.size(), tasks, wg);
-  int rc = upload(&p->d_descs, gv);
-  if (!rc) rc = upload(&p->d_wg, wg);
-  if (rc) {
-    delete p;
-    return rc;
-  }
-  p->ndesc = count;
-  p->ntasks = tasks;
-  *plan = p;
+  int rc = upload_gc_blocks(*p, block);
+  if (!rc) rc = finish_plan<GcDesc>(*p, block, gen, gc_tasks, gc_lean_ok);
+  if (rc) return rc;
+  *plan = p.release();
   return QTG_OK;
 }
 
@@ -401,22 +581,8 @@ int qtg_plan_execute(qtg_plan plan, void* out_base, const void* first_base, cons
     set_error("plan execute: null argument");
     return QTG_EARG;
   }
-  if (p->ntasks == 0) return QTG_OK;
-  hipStream_t s = S(stream);
-  if (p->kind == 0) {
-    // first = M base, second = B base
-    const auto* g = (const GmDesc*)p->d_descs;
-    const auto* wg = (const int32_t*)p->d_wg;
-    return p->c64 ? launch_gm<float, float, float>(g, wg, p->ndesc, p->ntasks, second_base, second_base,
-                                                   first_base, out_base, nullptr, 1.0, 0.0, s)
-                  : launch_gm<double, double, double>(g, wg, p->ndesc, p->ntasks, second_base, second_base,
-                                                      first_base, out_base, nullptr, 1.0, 0.0, s);
-  }
-  const auto* g = (const GcDesc*)p->d_descs;
-  // X (bra) from the first base, Y (ket) from the second: sel = 2 on every descriptor
-  const auto* wg = (const int32_t*)p->d_wg;
-  return p->c64 ? launch_gc<float, float>(g, wg, p->ndesc, p->ntasks, first_base, second_base, out_base, nullptr, s)
-                : launch_gc<double, double>(g, wg, p->ndesc, p->ntasks, first_base, second_base, out_base, nullptr, s);
+  return p->c64 ? run_plan<float>(*p, out_base, first_base, second_base, S(stream))
+                : run_plan<double>(*p, out_base, first_base, second_base, S(stream));
 }
 
 int qtg_hole_contraction_grouped_noalloc_z(const qtg_hole_contraction_desc* descs, int64_t count, double* S_base,
@@ -430,37 +596,61 @@ int qtg_hole_contraction_grouped_noalloc_z(const qtg_hole_contraction_desc* desc
     return QTG_ESHAPE;
   }
   if (count == 0) return QTG_OK;
-  // the same descriptors, K splits and task order as a plan of these descs
-  std::vector<GcDesc> gv;
-  gv.reserve((size_t)count);
+  // the same descriptors, K shares and kernels as a plan of these descs
+  std::vector<GcDesc> block, gen;
+  int64_t tiles = 0;
   for (int64_t i = 0; i < count; ++i) {
     GcDesc g;
     int rc = to_gc(descs[i], g);
     if (rc) return rc;
-    const int64_t K = (int64_t)g.bef * g.aft;
-    if (K > 2 * kSplitK) g.ksplit = split_chunks(K, kGemmWaves, 1);
-    gv.push_back(g);
+    add_gc(g, block, gen);
+    tiles += (int64_t)((g.nx + 15) / 16) * ((g.ny + 15) / 16) *
+             ((int64_t)g.bef * g.aft > 2 * kSplitK ? kGemmWaves : 1);
   }
-  const int64_t tasks = order_tasks(gv, gc_tasks);
-  if (tasks > kNoAllocMaxTasks) {
+  if (tiles > kNoAllocMaxTasks) {
     set_error("no-allocation contraction: more than " + std::to_string(kNoAllocMaxTasks) + " 16 x 16 tiles");
     return QTG_ESHAPE;
   }
-  std::vector<int32_t> wg;
-  gemm_wg_table(gv.data(), (int64_t)gv.size(), tasks, wg);
   void* base = nullptr;
   int rc = scratch_address(&base);
   if (rc) return rc;
   hipStream_t s = S(stream);
   GcDesc* d_descs = reinterpret_cast<GcDesc*>(base);
-  int32_t* d_wg = reinterpret_cast<int32_t*>(static_cast<unsigned char*>(base) + kNoAllocTableOff);
-  QTG_HIP_TRY(hipMemcpyAsync(d_descs, gv.data(), sizeof(GcDesc) * gv.size(), hipMemcpyHostToDevice, s));
-  QTG_HIP_TRY(hipMemcpyAsync(d_wg, wg.data(), sizeof(int32_t) * wg.size(), hipMemcpyHostToDevice, s));
-  rc = launch_gc<double, double>(d_descs, d_wg, count, tasks, A_base, B_base, S_base, nullptr, s);
-  if (rc) return rc;
+  unsigned char* d_table = static_cast<unsigned char*>(base) + kNoAllocTableOff;
   // the staging tables are host temporaries and the device copy is shared by
-  // every call on this GPU: the call returns with the result written
-  QTG_HIP_TRY(hipStreamSynchronize(s));
+  // every call on this GPU: each part returns with its result written
+  if (!block.empty()) {
+    GcBlockPlan p = plan_gc_blocks(block);
+    const int64_t nwg = (int64_t)p.wgs.size(), nsums = (int64_t)p.sums.size();
+    p.wgs.insert(p.wgs.end(), p.sums.begin(), p.sums.end());
+    if (p.wgs.size() * sizeof(GcBlockWg) > kNoAllocBytes - kNoAllocTableOff ||
+        (size_t)p.parts * 1024 * sizeof(cplx<double>) > kPartSlots * kPartBytes) {
+      set_error("no-allocation contraction: tables exceed the fixed array");
+      return QTG_ESHAPE;
+    }
+    QTG_HIP_TRY(hipMemcpyAsync(d_descs, block.data(), sizeof(GcDesc) * block.size(), hipMemcpyHostToDevice, s));
+    QTG_HIP_TRY(hipMemcpyAsync(d_table, p.wgs.data(), sizeof(GcBlockWg) * p.wgs.size(), hipMemcpyHostToDevice, s));
+    const GcBlockWg* wgs = reinterpret_cast<const GcBlockWg*>(d_table);
+    auto launch = [&](void* part) -> int {
+      int e = launch_gc_block<double>(d_descs, wgs, nwg, wgs + nwg, nsums, A_base, B_base, S_base, part, s);
+      if (e) return e;
+      QTG_HIP_TRY(hipStreamSynchronize(s));
+      return QTG_OK;
+    };
+    rc = p.parts > 0 ? with_all_parts(s, launch) : launch(nullptr);
+    if (rc) return rc;
+  }
+  if (!gen.empty()) {
+    const int64_t tasks = order_tasks(gen, gc_tasks);
+    std::vector<int32_t> wg;
+    gemm_wg_table(gen.data(), (int64_t)gen.size(), tasks, wg);
+    QTG_HIP_TRY(hipMemcpyAsync(d_descs, gen.data(), sizeof(GcDesc) * gen.size(), hipMemcpyHostToDevice, s));
+    QTG_HIP_TRY(hipMemcpyAsync(d_table, wg.data(), sizeof(int32_t) * wg.size(), hipMemcpyHostToDevice, s));
+    rc = launch_gc<double, double>(d_descs, reinterpret_cast<const int32_t*>(d_table), (int64_t)gen.size(), tasks,
+                                   A_base, B_base, S_base, nullptr, s);
+    if (rc) return rc;
+    QTG_HIP_TRY(hipStreamSynchronize(s));
+  }
   return QTG_OK;
 }
 

@@ -78,3 +78,77 @@ def test_single_hole_contraction_streams():
         assert np.array_equal(out[i].download(np.complex128).reshape(n, n), first[i])
     for s in streams:
         Q.check(L.qtg_stream_destroy(s))
+
+
+def _plan_case(rng, shapes, c64):
+    """Operands of a plan over (before, n, after) tensors, back to back."""
+    es = np.complex64 if c64 else np.complex128
+    N = [b * n * a for b, n, a in shapes]
+    oT = np.concatenate([[0], np.cumsum(N)]).astype(np.int64)
+    oM = np.concatenate([[0], np.cumsum([n * n for _, n, _ in shapes])]).astype(np.int64)
+    return rand(rng, oT[-1], c64), rand(rng, oT[-1], c64), rand(rng, oM[-1], c64), oT, oM, es
+
+
+# one tensor of a long reduction (shared by many workgroups), a few of very
+# different work, many of edge sizes: each chooses shares, XCD queues and the
+# sums over partial tiles differently
+HOLE_PLANS = {
+    "one_long": [(64, 40, 250)],
+    "mixed": [(1, 1, 1), (64, 64, 64), (3, 33, 700), (1, 17, 16), (40, 65, 30), (5, 16, 5), (2, 100, 900)],
+    "many": [(1 + i % 5, 1 + (7 * i) % 67, 3 + (11 * i) % 90) for i in range(200)],
+}
+
+
+@pytest.mark.parametrize("c64", [False, True])
+@pytest.mark.parametrize("name", sorted(HOLE_PLANS))
+def test_hole_plan(name, c64):
+    print(f"case hole plan {name} c64={c64}", flush=True)
+    shapes = HOLE_PLANS[name]
+    rng = np.random.default_rng(len(shapes))
+    A, B, S0, oT, oM, es = _plan_case(rng, shapes, c64)
+    d = np.zeros(len(shapes), Q.HC_DESC)
+    d["offS"], d["offA"], d["offB"] = oM[:-1], oT[:-1], oT[:-1]
+    d["before"], d["after"] = [s[0] for s in shapes], [s[2] for s in shapes]
+    d["nA"] = d["nB"] = [s[1] for s in shapes]
+    d["accumulate"] = np.arange(len(shapes)) % 2
+    plan = Q.Plan("hole_contraction", d, complex64=c64)
+    dA, dB, dS = (Q.DeviceBuffer.from_array(x) for x in (A, B, S0))
+    plan.execute(dS, dA, dB)
+    got = dS.download(es)
+    for i, (b, n, a) in enumerate(shapes):
+        x, y = (v[oT[i]:oT[i + 1]].reshape(a, n, b).astype(np.complex128) for v in (A, B))
+        ref = np.einsum("ajb,alb->lj", x.conj(), y, optimize=True).ravel()
+        if i % 2:
+            ref = ref + S0[oM[i]:oM[i + 1]]
+        close(got[oM[i]:oM[i + 1]], ref, b * a, c64)
+
+
+@pytest.mark.parametrize("c64", [False, True])
+def test_product_plan(c64):
+    """Enough tensors for the blocked product, among them ones it leaves to
+    the tile kernel: rows around 32, bef below and above 4, columns around 16
+    and 32, every op, plain and accumulating."""
+    print(f"case product plan c64={c64}", flush=True)
+    shapes = [(1 + (5 * i) % 37, (15, 16, 17, 31, 32, 33, 48, 61)[i % 8], 1 + (13 * i) % 70) for i in range(700)]
+    rng = np.random.default_rng(9)
+    B, C0, M, oT, oM, es = _plan_case(rng, shapes, c64)
+    d = np.zeros(len(shapes), Q.MP_DESC)
+    d["offC"], d["offM"], d["offB"] = oT[:-1], oM[:-1], oT[:-1]
+    d["before"], d["after"] = [s[0] for s in shapes], [s[2] for s in shapes]
+    d["nB"] = d["nC"] = [s[1] for s in shapes]
+    d["op"] = np.arange(len(shapes)) % 3
+    d["add"] = (np.arange(len(shapes)) // 3) % 2
+    # the blocked kernel's share of the plan: 32 x 32 outputs a wavefront
+    assert sum(-(-b * a // 32) * -(-n // 32) for b, n, a in shapes if n > 16) >= 8192
+    plan = Q.Plan("mode_product", d, complex64=c64)
+    dB, dC, dM = (Q.DeviceBuffer.from_array(x) for x in (B, C0, M))
+    plan.execute(dC, dM, dB)
+    got = dC.download(es)
+    for i, (b, n, a) in enumerate(shapes):
+        x = B[oT[i]:oT[i + 1]].reshape(a, n, b).astype(np.complex128)
+        m = M[oM[i]:oM[i + 1]].reshape(n, n).T.astype(np.complex128)  # column-major
+        m = (m, m.T, m.conj().T)[d["op"][i]]
+        ref = np.einsum("kl,alb->akb", m, x, optimize=True).ravel()
+        if d["add"][i]:
+            ref = ref + C0[oT[i]:oT[i + 1]]
+        close(got[oT[i]:oT[i + 1]], ref, n, c64)
