@@ -220,7 +220,10 @@ int qtg_engine_get_dpsi(qtg_engine engine, double* host, int which, qtg_stream s
  * states at the top node this is the state average trace(H) / trace(S); the
  * levels of each state come from qtg_cmf_eigenstates. */
 int qtg_engine_energy(qtg_engine engine, double* energy, qtg_stream stream);
-/* which: 0 rho[node], 1 rho^-1[node], 2 h-matrix[term][node], 3 hole[term][node] */
+/* which: 0 rho[node], 1 rho^-1[node], 2 h-matrix[term][node], 3 hole[term][node]
+ * of the last build (or derivative).  A compressed engine may form a term's
+ * matrices only inside sums; the first call with which 2 or 3 after a build
+ * then forms all of them at that build's state, in buffers of their own. */
 int qtg_engine_get_matrix(qtg_engine engine, int which, int64_t term, int64_t node, double* out,
                           qtg_stream stream);
 /* FLOPs of one H|Psi> sweep of the reference algorithm (8 per complex

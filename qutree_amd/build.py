@@ -10,7 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libqutree_amd.so")
-SOURCES = ["runtime.cpp", "gemm_ops.hip", "gemm_block.hip", "node_ops.hip", "tree_ops.hip", "cmf_ops.hip", "model.cpp", "engine.cpp", "engine_gemm.cpp", "launch_set.cpp", "ttno.cpp", "cmf.cpp",
+SOURCES = ["runtime.cpp", "gemm_ops.hip", "gemm_block.hip", "node_ops.hip", "tree_ops.hip", "cmf_ops.hip", "model.cpp", "engine.cpp", "engine_gemm.cpp", "engine_reduce.cpp", "launch_set.cpp", "ttno.cpp", "cmf.cpp",
            "capi_engine.cpp", "formats.cpp", "seam.cpp", "smallmat.hip", "grad_ops.hip", "gradient.cpp", "tuning.cpp",
            "scf.cpp", "scf_ops.hip", "tree_prog.cpp", "apply_fit.cpp"]
 # -amdgpu-mfma-vgpr-form: MFMA accumulators in ordinary VGPRs (gfx950 has

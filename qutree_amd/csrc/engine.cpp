@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 
 namespace qtg {
@@ -59,6 +60,9 @@ void Engine::invalidate_graph() {
 }
 
 void Engine::release() {
+  full_.reset();
+  fullBuild_ = -1;
+  builds_ = 0;
   for (void* p : device_buffers_)
     if (p) (void)hipFree(p);
   device_buffers_.clear();
@@ -143,6 +147,7 @@ int Engine::set_hamiltonian(int64_t nterms, const double* coeff, const int64_t* 
     return QTG_EARG;
   }
   apply_tuning();
+  planSmall_ = false;
   return plan();
 }
 
@@ -425,6 +430,16 @@ int Engine::plan() {
   combTerm2.clear();
   double combFlops = 0.0;
   int64_t part = 0;
+  sums_.clear();
+  sumOf_.clear();
+  sumKey_.clear();
+  hWant_.assign(NN, {});
+  qWant_.assign(NN, {});
+  gsumm_.clear();
+  fused_.clear();
+  leafSums_.clear();
+  h_combA_.clear();
+  h_combtA_.clear();
   summ_.assign(NN, {});
   smode_.assign(NN, {});
   sdim_.assign(NN, {});
@@ -463,7 +478,14 @@ int Engine::plan() {
       if (!v.top()) g.ids.push_back(holeslot_[l][v.addr]);
       tl.push_back(g);
     }
-    std::vector<Summand> groups = compress_ ? aggregate(tl, sdim, off, combFlops) : tl;
+    std::vector<Summand> groups;
+    if (reduced()) {
+      std::vector<int> sd;
+      const std::vector<SlotRef> slots = node_slots(v, sd);
+      groups = take_groups(merge_groups(tl, S), slots, sdim, off);
+    } else {
+      groups = compress_ ? aggregate(tl, sdim, off, combFlops) : tl;
+    }
     summ_[v.addr] = groups;
     smode_[v.addr] = smode;
     sdim_[v.addr] = sdim;
@@ -497,6 +519,54 @@ int Engine::plan() {
     terms.insert(terms.end(), vt.begin(), vt.end());
     fn.nchunk = nch;
     fin.push_back(fn);
+  }
+  keep_.assign(items.size(), 1);
+  // A plan whose single matrices cost less than kReduceFlops keeps them all:
+  // there the launches decide, and the summed contractions add one (the sums
+  // of h-matrices) and fuse no hole layer.  Sweeps measured on both sides:
+  // 0.03 and 0.2 GFLOP 0.99 and 0.97 times as fast reduced, 0.94 GFLOP 1.08,
+  // 3.3 GFLOP (the 64-mode tree) 1.15, 532 GFLOP (the 128-mode tree) 3.3.
+  // (QTG_REDUCE_MIN_FLOPS moves the line, for tests.)
+  constexpr double kReduceFlops = 5e8;
+  const char* rmin = std::getenv("QTG_REDUCE_MIN_FLOPS");
+  if (reduced() && flops_ < (rmin ? std::atof(rmin) : kReduceFlops)) {
+    planSmall_ = true;
+    return plan();
+  }
+  if (reduced()) {
+    // the gradient's summands (the terms active at the parent and inactive
+    // at the node) use the sums of Apply at the parent
+    if (precision_ == 0 && tree_.nodes.back().n == 1) {
+      gsumm_.assign(NN, {});
+      for (auto& v : tree_.nodes) {
+        if (v.top()) continue;
+        const HNode& p = tree_.nodes[v.parent];
+        std::vector<Summand> tl;
+        for (int l = 0; l < L; ++l) {
+          if (!active_[l][p.addr] || active_[l][v.addr]) continue;
+          Summand g;
+          g.coef = sop_.terms[l].coeff;
+          for (int c : p.children) g.ids.push_back(active_[l][c] ? hslot_[l][c] : -1);
+          if (!p.top()) g.ids.push_back(holeslot_[l][p.addr]);
+          tl.push_back(g);
+        }
+        std::vector<int> sd;
+        const std::vector<SlotRef> slots = node_slots(p, sd);
+        gsumm_[v.addr] = take_groups(merge_groups(tl, (int)slots.size()), slots, sd, off);
+      }
+    }
+    reduce_plan(hent, qent, off);
+    for (size_t i = 0; i < items.size(); ++i) {
+      const SwItem& it = items[i];
+      const HNode& nd = tree_.nodes[it.node];
+      if (it.k == nd.order() - 1 && hWant_[it.node].single.count(it.out)) continue;
+      const bool hole = it.k < (int)nd.children.size() && !nd.bottom;
+      if (hole) {
+        const int v = nd.children[it.k];
+        if (it.out == rhoslot_[v] || qWant_[v].single.count(it.out)) continue;
+      }
+      keep_[i] = 0;
+    }
   }
   poolSize_ = off;
   nChunks_ = (int64_t)chunks.size();
@@ -543,8 +613,10 @@ int Engine::plan() {
   release();
   int rc = materialize();
   if (rc) return rc;
-  if ((rc = up(&d_sw_, items))) return rc;
-  device_buffers_.push_back(d_sw_);
+  if (path_ == 0) {
+    if ((rc = up(&d_sw_, items))) return rc;
+    device_buffers_.push_back(d_sw_);
+  }
   if ((rc = up(&d_eig_, eig))) return rc;
   device_buffers_.push_back(d_eig_);
   if ((rc = up(&d_terms_, terms))) return rc;
@@ -570,6 +642,16 @@ int Engine::plan() {
     device_buffers_.push_back(d_hk_);
     if ((rc = up(&d_hi_, h_hi_))) return rc;
     device_buffers_.push_back(d_hi_);
+    if ((rc = up(&d_gs_, h_gs_))) return rc;
+    device_buffers_.push_back(d_gs_);
+    if ((rc = up(&d_seg_, h_seg_))) return rc;
+    device_buffers_.push_back(d_seg_);
+    if ((rc = up(&d_combA_, h_combA_))) return rc;
+    device_buffers_.push_back(d_combA_);
+    if ((rc = up(&d_combtA_, h_combtA_))) return rc;
+    device_buffers_.push_back(d_combtA_);
+    if (partElems_ > 0 && (rc = alloc(&d_part_, 16 * (size_t)partElems_))) return rc;
+    if (reduced() && (rc = alloc((void**)&d_psiBuilt_, sizeof(double) * 2 * tree_.total))) return rc;
     if ((rc = up(&d_solve_, h_solve_))) return rc;
     device_buffers_.push_back(d_solve_);
     if ((rc = up(&d_combOut3_, h_comb3_))) return rc;
@@ -622,6 +704,14 @@ int Engine::plan() {
     std::vector<double> e(2 * (size_t)id.second * id.second, 0.0);
     for (int i = 0; i < id.second; ++i) e[2 * ((size_t)i + (size_t)i * id.second)] = 1.0;
     if ((rc = put(id.first, e))) return rc;
+  }
+  for (auto& ls : leafSums_) {
+    std::vector<double> e;
+    for (auto& z : ls.second) {
+      e.push_back(z.real());
+      e.push_back(z.imag());
+    }
+    if ((rc = put(ls.first, e))) return rc;
   }
   planned_ = true;
   return QTG_OK;
@@ -939,6 +1029,7 @@ int Engine::derivative(hipStream_t s, double ph_re, double ph_im) {
   }
   QTG_HIP_TRY(hipGraphLaunch(graph_exec_, s));
   built_ = true;
+  ++builds_;
   return QTG_OK;
 }
 
@@ -950,6 +1041,40 @@ int Engine::energy(hipStream_t s, double* out) {
   // <A_top|Apply(A_top)> / <A_top|A_top>
   const cd num(e[0], e[1]), den(e[2], e[3]);
   *out = (num / den).real();
+  return QTG_OK;
+}
+
+// The engine that forms every matrix of every term, at the state of the last
+// build.
+int Engine::full_engine(hipStream_t s) {
+  if (builds_ == 0) {
+    set_error("engine: build() first");
+    return QTG_ESTATE;
+  }
+  int rc;
+  if (!full_) {
+    std::unique_ptr<Engine> e(new Engine());
+    if ((rc = e->create(treeText_, precision_))) return rc;
+    e->reduce_ = false;
+    e->graph_ = false;
+    e->tuning_ = false;
+    e->splitWaves_ = splitWaves_;
+    e->splitMinK_ = splitMinK_;
+    e->gmSplitK_ = gmSplitK_;
+    e->gcLongK_ = gcLongK_;
+    e->fuseHoles_ = fuseHoles_;
+    e->sop_ = sop_;
+    if ((rc = e->plan())) return rc;
+    full_ = std::move(e);
+  }
+  if (fullBuild_ == builds_) return QTG_OK;
+  if (heevPending_) QTG_HIP_TRY(hipStreamWaitEvent(s, evHeev_, 0));  // the copy runs before it
+  QTG_HIP_TRY(hipStreamSynchronize(s));
+  full_->eps_ = eps_;
+  if ((rc = full_->set_psi_device(d_psiBuilt_, full_->stream_))) return rc;
+  if ((rc = full_->build(full_->stream_))) return rc;
+  if ((rc = full_->synchronize())) return rc;
+  fullBuild_ = builds_;
   return QTG_OK;
 }
 
@@ -966,6 +1091,10 @@ int Engine::get_matrix(int which, int term, int node, double* out, hipStream_t s
     off = (which == 2) ? hslot_[term][node] : holeslot_[term][node];
   }
   if (off < 0) return QTG_EARG;
+  if (which >= 2 && reduced()) {
+    const int rc = full_engine(s);
+    return rc ? rc : full_->get_matrix(which, term, node, out, full_->stream_);
+  }
   if (heevPending_) QTG_HIP_TRY(hipStreamWaitEvent(s, evHeev_, 0));  // rho^-1 of the side stream
   if (from64 || !c64_ || path_ == 1) {
     const void* base = from64 ? (const void*)d_pool64_ : d_pool_;

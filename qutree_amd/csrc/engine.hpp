@@ -1,8 +1,10 @@
 // Device-resident tree engine (see engine.cpp).
 #pragma once
 #include <map>
+#include <memory>
 #include <set>
 #include <string>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -148,7 +150,7 @@ class Engine {
   // mode product writing FP64 (the stacked Apply sum)
   enum Prec { P64 = 0, P32 = 1, P32W = 2 };
   struct GLaunch {
-    int kind;    // 0 mode products, 1 hole contractions, 2 solve
+    int kind;    // 0 mode products, 1 hole contractions, 2 solve, 3 fused hole layer, 4 summed contractions
     int prec;    // Prec
     int64_t d0, nd, ntasks;
     int64_t wg0;       // first entry of the workgroup -> descriptor table
@@ -159,6 +161,8 @@ class Engine {
     int waves;     // mode products: tasks per workgroup (0: kGemmWaves)
     bool lean;     // every descriptor takes the lean kernel form
     int64_t lds;   // fused hole layers (kind 3): dynamic LDS bytes per workgroup
+    int64_t nsums; // summed contractions (kind 4): macro tiles whose workgroups leave partial tiles
+    int nt;        // and their macro tile (launch_gc_sum)
   };
   bool gramInSolve_ = false;  // the solve launch forms S, A^H Y and the energy terms
   int run_launches(const std::vector<GLaunch>& L, void* const* bases, const uint8_t* active, double sre, double sim,
@@ -182,6 +186,7 @@ class Engine {
   bool c64_ = false, planned_ = false, built_ = false, host_only_ = false;
   int precision_ = 0;  // 0 complex128, 1 complex64 bulk, 2 complex64 bulk with FP64 for large terms
   std::vector<SwItem> h_items_;
+  std::vector<char> keep_;  // items the reduced sweep forms
   std::vector<EigItem> h_eig_;
   std::vector<ApTerm> h_terms_;
   std::vector<ApChunk> h_chunks_;
@@ -194,6 +199,65 @@ class Engine {
     std::vector<int64_t> ids;  // matrix per slot (-1: identity)
   };
   std::vector<std::vector<Summand>> summ_;    // Apply summands per node
+  // Reduced sweep (engine_reduce.cpp): which matrices are formed
+  struct SlotRef {
+    int node;
+    enum Kind { LEAF, H, HOLE } kind;
+  };
+  struct Group {  // merged summands: slot fs (-1: none) carries the weighted list `terms`
+    cd coef = cd(1.0, 0.0);
+    std::vector<int64_t> ids;
+    int fs = -1;
+    std::vector<std::pair<int64_t, cd>> terms;
+  };
+  struct MatSum {  // sum of coefficient times matrix (-1: identity) at one slot
+    SlotRef slot;
+    int d;
+    std::vector<std::pair<int64_t, cd>> terms;
+    int64_t out;
+    bool early = false;  // read by a hole: combined from single h-matrices
+    bool hard = false;   // read by a hole below: formed as a contraction
+    bool fused = false;  // formed as a contraction (fused_)
+  };
+  struct Fused {  // out = sum_g coef_g <A| factors_g |A> over the legs of `node` but k
+    int node, k, level = 0, d = 0;
+    int64_t out, add = -1;  // add: a matrix of an earlier layer to add (-1: none)
+    std::vector<SlotRef> slots;
+    std::vector<Summand> groups;
+  };
+  struct Want {
+    std::set<int64_t> single;
+    std::set<int> sums;
+  };
+  bool reduce_ = true;        // with compress on the grouped path
+  bool planSmall_ = false;    // this plan is too small for it (plan())
+  bool reduced() const { return reduce_ && !planSmall_ && compress_ && path_ == 1; }
+  std::vector<MatSum> sums_;
+  std::map<int64_t, int> sumOf_;
+  std::map<std::tuple<int, int, std::vector<std::pair<int64_t, std::pair<double, double>>>>, int> sumKey_;
+  std::vector<Want> hWant_, qWant_;
+  std::vector<Fused> fused_;
+  std::vector<std::vector<Summand>> gsumm_;  // gradient summands at a node's parent
+  std::vector<std::pair<int64_t, std::vector<cd>>> leafSums_;
+  std::vector<CombOut> h_combA_;
+  std::vector<CombTerm> h_combtA_;
+  CombOut* d_combA_ = nullptr;
+  CombTerm* d_combtA_ = nullptr;
+  std::vector<Group> merge_groups(const std::vector<Summand>& tl, int S) const;
+  int matrix_sum(const SlotRef& slot, int d, const std::vector<std::pair<int64_t, cd>>& terms, int64_t& off);
+  std::vector<Summand> take_groups(const std::vector<Group>& groups, const std::vector<SlotRef>& slots,
+                                   const std::vector<int>& sdim, int64_t& off);
+  std::vector<SlotRef> node_slots(const HNode& v, std::vector<int>& sdim) const;
+  void want(const SlotRef& slot, int64_t id, bool early, bool hard);
+  void reduce_plan(const std::vector<std::vector<std::pair<int64_t, int>>>& hent,
+                   const std::vector<std::vector<std::pair<int64_t, int>>>& qent, int64_t& off);
+  // Matrices of single terms for get_matrix: an engine of the same tree and
+  // Hamiltonian that forms all of them, run on the state of the last build
+  // (d_psiBuilt_, copied beside the eigensolver) when one is asked for.
+  std::unique_ptr<Engine> full_;
+  double* d_psiBuilt_ = nullptr;
+  int64_t builds_ = 0, fullBuild_ = -1;
+  int full_engine(hipStream_t s);
   std::vector<Summand> aggregate(const std::vector<Summand>& tl, const std::vector<int>& sdim, int64_t& off,
                                  double& combFlops);
   std::vector<CombOut> h_comb1_, h_comb2_;  // aggregated slots: partial sums, sums of partials
@@ -229,6 +293,12 @@ class Engine {
   std::vector<HoleKet> h_hk_;   // fused hole layers: kets and their items
   std::vector<HoleItem> h_hi_;
   HoleKet* d_hk_ = nullptr;
+  std::vector<GcSum> h_gs_;     // summed contractions: one per output tile and share, then one per tile to add up
+  std::vector<GcSeg> h_seg_;
+  GcSum* d_gs_ = nullptr;
+  GcSeg* d_seg_ = nullptr;
+  int64_t partElems_ = 0;
+  void* d_part_ = nullptr;      // partial tiles of the summed contractions
   HoleItem* d_hi_ = nullptr;
   std::vector<int32_t> h_gmwg_, h_gcwg_;
   int32_t* d_gmwg_ = nullptr;

@@ -32,6 +32,7 @@
 #include <tuple>
 
 #include "engine.hpp"
+#include "grad_ops.hpp"
 
 namespace qtg {
 
@@ -82,6 +83,9 @@ int Engine::plan_gemm() {
   idSlots_.clear();
   h_comb3_.clear();
   h_combt3_.clear();
+  h_gs_.clear();
+  h_seg_.clear();
+  partElems_ = 0;
   int64_t poolOff = poolSize_;
   int64_t pool64Off = pool64Size_;
   workSize_ = 0;
@@ -205,9 +209,16 @@ int Engine::plan_gemm() {
   struct LayerLists {
     std::vector<GmDesc> lv0[2], lv1[2];
     std::vector<GcDesc> con[2];
+    // summed contractions: per output its view and segments
+    struct Sum {
+      GcSum d;
+      std::vector<GcSeg> segs;
+    };
+    std::vector<Sum> sums[2];
   };
-  auto sandwich_layer = [&](const std::pair<int64_t, int64_t>& r, int rho, LayerLists& out) {
-    if (r.second == r.first) return;
+  auto sandwich_layer = [&](const std::pair<int64_t, int64_t>& r, int rho, LayerLists& out,
+                            const std::vector<const Fused*>& fused = {}) {
+    if (r.second == r.first && fused.empty()) return;
     struct Side {
       std::map<std::tuple<int, int, int64_t>, int64_t> zbra;  // (node, leg, mat) -> work offset
       std::map<std::vector<int64_t>, int64_t> zket1, zket2;   // (node, leg, mat[, leg, mat])
@@ -217,63 +228,91 @@ int Engine::plan_gemm() {
     } sd[2];  // [0] FP32, [1] FP64
     sd[0].w = wbase32;
     sd[1].w = wbase;
-    for (int64_t i = r.first; i < r.second; ++i) {
-      const SwItem& it = h_items_[i];
-      if (rho >= 0 && (int)is_rho(it) != rho) continue;
-      Side& S = sd[item_hi(it.out) ? 1 : 0];
-      const HNode& p = tree_.nodes[it.node];
-      const int k = it.k;
+    // the bra and ket tensors of <F x .. |A| .. x G> at node p contracted over
+    // all legs but k; equal tensors of a layer once
+    struct XY {
+      int64_t x, y;
+      int sel;
+    };
+    // (coef: a group's coefficient, carried by its first product, or by a
+    // copy of the ket where it has none)
+    auto operands = [&](Side& S, const HNode& p, int k, const std::vector<std::pair<int, int64_t>>& fac,
+                        cd coef = cd(1.0, 0.0)) {
+      const bool scaled = coef != cd(1.0, 0.0);
       const int braleg = (k == 0) ? 1 : 0;
-      int64_t xoff = p.off;
-      int xsel = 0;
+      XY o{p.off, p.off, 0};
       std::vector<std::pair<int, int64_t>> ket;
-      for (int f = 0; f < it.nf; ++f) {
-        if (it.fmode[f] == braleg) {
-          auto key = std::make_tuple((int)it.node, braleg, it.fmat[f]);
+      for (auto& f : fac) {
+        if (f.first == braleg) {
+          auto key = std::make_tuple(p.addr, braleg, f.second);
           auto z = S.zbra.find(key);
           if (z == S.zbra.end()) {
-            S.lv0.push_back(gm_desc(p, braleg, p.off, 0, it.fmat[f], S.w, GM_H, it.node));
+            S.lv0.push_back(gm_desc(p, braleg, p.off, 0, f.second, S.w, GM_H, p.addr));
             z = S.zbra.emplace(key, S.w).first;
             S.w += p.N;
           }
-          xoff = z->second;
-          xsel = 1;
+          o.x = z->second;
+          o.sel |= 1;
         } else {
-          ket.push_back({it.fmode[f], it.fmat[f]});
+          ket.push_back(f);
         }
       }
       std::sort(ket.begin(), ket.end(), [](auto& a, auto& b) { return a.first > b.first; });
-      int64_t yoff = p.off;
-      int ysel = 0;
-      if (!ket.empty()) {
-        std::vector<int64_t> key1 = {it.node, ket[0].first, ket[0].second};
+      if (scaled) {
+        // not shared: the ket of this group alone
+        GmDesc g = ket.empty() ? gm_desc(p, p.order() - 1, p.off, 0, 0, S.w, GM_COPY, p.addr)
+                               : gm_desc(p, ket[0].first, p.off, 0, ket[0].second, S.w, GM_N, p.addr);
+        g.are = coef.real();
+        g.aim = coef.imag();
+        S.lv0.push_back(g);
+        o.y = S.w;
+        o.sel |= 2;
+        S.w += p.N;
+        if (ket.size() > 1) {
+          S.lv1.push_back(gm_desc(p, ket[1].first, o.y, 1, ket[1].second, S.w, GM_N, p.addr));
+          o.y = S.w;
+          S.w += p.N;
+        }
+      } else if (!ket.empty()) {
+        std::vector<int64_t> key1 = {p.addr, ket[0].first, ket[0].second};
         auto z = S.zket1.find(key1);
         if (z == S.zket1.end()) {
-          S.lv0.push_back(gm_desc(p, ket[0].first, p.off, 0, ket[0].second, S.w, GM_N, it.node));
+          S.lv0.push_back(gm_desc(p, ket[0].first, p.off, 0, ket[0].second, S.w, GM_N, p.addr));
           z = S.zket1.emplace(key1, S.w).first;
           S.w += p.N;
         }
-        yoff = z->second;
-        ysel = 1;
+        o.y = z->second;
+        o.sel |= 2;
         if (ket.size() > 1) {
           std::vector<int64_t> key2 = key1;
           key2.push_back(ket[1].first);
           key2.push_back(ket[1].second);
           auto z2 = S.zket2.find(key2);
           if (z2 == S.zket2.end()) {
-            S.lv1.push_back(gm_desc(p, ket[1].first, yoff, 1, ket[1].second, S.w, GM_N, it.node));
+            S.lv1.push_back(gm_desc(p, ket[1].first, o.y, 1, ket[1].second, S.w, GM_N, p.addr));
             z2 = S.zket2.emplace(key2, S.w).first;
             S.w += p.N;
           }
-          yoff = z2->second;
+          o.y = z2->second;
         }
       }
+      return o;
+    };
+    for (int64_t i = r.first; i < r.second; ++i) {
+      const SwItem& it = h_items_[i];
+      if (!keep_[i]) continue;
+      if (rho >= 0 && (int)is_rho(it) != rho) continue;
+      Side& S = sd[item_hi(it.out) ? 1 : 0];
+      const HNode& p = tree_.nodes[it.node];
+      std::vector<std::pair<int, int64_t>> fac;
+      for (int f = 0; f < it.nf; ++f) fac.push_back({it.fmode[f], it.fmat[f]});
+      const XY o = operands(S, p, it.k, fac);
       GcDesc g{};
       int64_t bef, aft;
       int nk;
-      view(p, k, bef, nk, aft);
-      g.x = xoff;
-      g.y = yoff;
+      view(p, it.k, bef, nk, aft);
+      g.x = o.x;
+      g.y = o.y;
       g.out = it.out;
       g.bef = (int32_t)bef;
       g.nx = g.ny = nk;
@@ -281,8 +320,34 @@ int Engine::plan_gemm() {
       g.acc = 0;
       g.node = it.node;
       g.ksplit = 1;
-      g.sel = xsel | (ysel << 1);
+      g.sel = o.sel;
       S.con.push_back(g);
+    }
+    for (const Fused* f : fused) {
+      const int hp = item_hi(f->out) ? 1 : 0;
+      Side& S = sd[hp];
+      const HNode& p = tree_.nodes[f->node];
+      LayerLists::Sum sm{};
+      int64_t bef, aft;
+      int nk;
+      view(p, f->k, bef, nk, aft);
+      sm.d.out = f->out;
+      sm.d.add = f->add;
+      sm.d.bef = (int32_t)bef;
+      sm.d.n = nk;
+      sm.d.aft = (int32_t)aft;
+      for (const Summand& g : f->groups) {
+        std::vector<std::pair<int, int64_t>> fac;
+        for (size_t q = 0; q < f->slots.size(); ++q) {
+          if (g.ids[q] < 0) continue;
+          // a child's h-matrix on the child's leg, the node's own hole on the last
+          const bool own = f->slots[q].kind == SlotRef::HOLE;
+          fac.push_back({own ? p.order() - 1 : tree_.nodes[f->slots[q].node].childIdx, g.ids[q]});
+        }
+        const XY o = operands(S, p, f->k, fac, g.coef);
+        sm.segs.push_back({o.x, o.y, o.sel, 0});
+      }
+      out.sums[hp].push_back(sm);
     }
     wmax32 = std::max(wmax32, sd[0].w);
     wmax = std::max(wmax, sd[1].w);
@@ -293,6 +358,64 @@ int Engine::plan_gemm() {
       app(out.con[hp], sd[hp].con);
     }
   };
+  // The summed contractions of a layer and precision, one launch for the
+  // matrices of up to 16 x 16 and one for the larger.  A reduction beyond
+  // `whole` elements is shared by workgroups of `share` each, whose partial
+  // tiles a further launch adds: the top's children of the 64-mode tree
+  // (K = 18 x 196) would hold one CU for 23 us.
+  auto push_sum = [&](std::vector<GLaunch>& L, std::vector<LayerLists::Sum>& v, int prec, int x0, int x1) {
+    // 32 x 32 macro tiles where the launch has workgroups to spare: they read
+    // an operand once per 32 columns, but hold 2 x 2 tiles' work on one CU
+    // (24 x 24 matrices, K = 1152, 40 of them: 43 us against 9)
+    int64_t fine = 0;
+    for (auto& sm : v) {
+      const int64_t T1 = (sm.d.n + 15) / 16;
+      fine += T1 * T1 * std::max<int64_t>(1, (int64_t)sm.d.bef * sm.d.aft * (int64_t)sm.segs.size() / 512);
+    }
+    for (int nt = 1; nt <= 2; ++nt) {
+      const int64_t whole = nt == 1 ? 768 : 1536, share = nt == 1 ? 512 : 1024;
+      GLaunch gl{};
+      gl.kind = 4;
+      gl.prec = prec;
+      gl.nt = nt;
+      gl.d0 = (int64_t)h_gs_.size();
+      gl.x0 = x0;
+      gl.x1 = x1;
+      gl.m = -1;
+      gl.o = B_POOL;
+      std::vector<GcSum> tasks, sums;
+      int64_t parts = 0;
+      for (auto& sm : v) {
+        GcSum d = sm.d;
+        if ((d.n <= 16 || fine <= 1024 ? 1 : 2) != nt) continue;
+        const int64_t Kt = (int64_t)d.bef * d.aft * (int64_t)sm.segs.size();
+        d.seg0 = (int32_t)h_seg_.size();
+        h_seg_.insert(h_seg_.end(), sm.segs.begin(), sm.segs.end());
+        d.seg1 = (int32_t)h_seg_.size();
+        d.S = Kt > whole ? (int32_t)((Kt + share - 1) / share) : 1;
+        const int T1 = (d.n + 16 * nt - 1) / (16 * nt);
+        for (d.tile = 0; d.tile < T1 * T1; ++d.tile) {
+          d.part = (int32_t)parts;
+          for (d.share = 0; d.share < d.S; ++d.share) tasks.push_back(d);
+          if (d.S > 1) {
+            d.share = 0;
+            sums.push_back(d);
+            parts += d.S;
+          }
+        }
+        gl.flops += 8.0 * (double)Kt * d.n * d.n;
+        gl.bytes += (prec == P64 ? 16.0 : 8.0) * 2.0 * (double)Kt * d.n + 16.0 * d.n * (double)d.n;
+      }
+      if (tasks.empty()) continue;
+      flops += gl.flops;
+      partElems_ = std::max(partElems_, 256 * nt * nt * parts);
+      gl.nd = gl.ntasks = (int64_t)tasks.size();
+      gl.nsums = (int64_t)sums.size();
+      h_gs_.insert(h_gs_.end(), tasks.begin(), tasks.end());
+      h_gs_.insert(h_gs_.end(), sums.begin(), sums.end());
+      L.push_back(gl);
+    }
+  };
   auto push_layer = [&](LayerLists& x, std::vector<GLaunch>& L) {
     push_gm(L, x.lv0[1], P64, B_PSI64, B_WORK64, B_POOL, B_WORK64, false);
     push_gm(L, x.lv0[0], P32, B_PSI32, B_WORK32, B_POOL, B_WORK32, false);
@@ -300,6 +423,8 @@ int Engine::plan_gemm() {
     push_gm(L, x.lv1[0], P32, B_PSI32, B_WORK32, B_POOL, B_WORK32, false);
     push_gc(L, x.con[1], P64, B_PSI64, B_WORK64, B_POOL);
     push_gc(L, x.con[0], P32, B_PSI32, B_WORK32, B_POOL);
+    push_sum(L, x.sums[1], P64, B_PSI64, B_WORK64);
+    push_sum(L, x.sums[0], P32, B_PSI32, B_WORK32);
   };
   // Represent (bottom-up) and the density tree (top-down) are independent
   // chains of the same depth: layer j of each runs in the same launches
@@ -307,9 +432,16 @@ int Engine::plan_gemm() {
   // ready when represent ends.  The holes of the terms (top-down), which
   // use the densities as the parent factor of terms acting only below a
   // node, follow; the eigensolver of rho^-1 runs on a side stream beside them.
-  std::vector<LayerLists> rep(repRange_.size()), hol(holeRange_.size()), rho(holeRange_.size());
+  size_t nhol = holeRange_.size();
+  for (const Fused& f : fused_) nhol = std::max(nhol, (size_t)f.level + 1);
+  std::vector<LayerLists> rep(repRange_.size()), hol(nhol), rho(holeRange_.size());
   for (size_t i = 0; i < repRange_.size(); ++i) sandwich_layer(repRange_[i], -1, rep[i]);
-  for (size_t dd = 1; dd < holeRange_.size(); ++dd) sandwich_layer(holeRange_[dd], 0, hol[dd]);
+  for (size_t dd = 1; dd < nhol; ++dd) {
+    std::vector<const Fused*> fs;
+    for (const Fused& f : fused_)
+      if (f.level == (int)dd) fs.push_back(&f);
+    sandwich_layer(dd < holeRange_.size() ? holeRange_[dd] : std::make_pair((int64_t)0, (int64_t)0), 0, hol[dd], fs);
+  }
   wbase = wmax;
   wbase32 = wmax32;
   for (size_t dd = 1; dd < holeRange_.size(); ++dd) sandwich_layer(holeRange_[dd], 1, rho[dd]);
@@ -353,7 +485,7 @@ int Engine::plan_gemm() {
     const int64_t bw0 = std::max(wmax, workSize_);  // bras after every other work tensor of the sweep
     int64_t bw = bw0;
     // the first layer keeps two launches: its mode products carry the bras
-    for (size_t dd = 2; fuseHoles_ && precision_ == 0 && dd < holeRange_.size(); ++dd) {
+    for (size_t dd = 2; fuseHoles_ && fused_.empty() && precision_ == 0 && dd < holeRange_.size(); ++dd) {
       std::map<std::tuple<int, int, int64_t>, std::vector<HoleItem>> byKet;  // (node, leg, matrix)
       bool ok = true;
       std::vector<GmDesc> lb;  // this layer's new bras
@@ -362,7 +494,7 @@ int Engine::plan_gemm() {
       double fl_ = 0.0, by_ = 0.0;
       for (int64_t i = holeRange_[dd].first; i < holeRange_[dd].second && ok; ++i) {
         const SwItem& it = h_items_[i];
-        if (is_rho(it)) continue;
+        if (is_rho(it) || !keep_[i]) continue;
         const HNode& p = tree_.nodes[it.node];
         const int k = it.k, braleg = (k == 0) ? 1 : 0;
         int64_t bmat = -1, kmat = -1;
@@ -754,6 +886,7 @@ int Engine::plan_gemm() {
   }
   // combine flops (aggregated slots; sums over them and stacked blocks)
   double comb = 0.0;
+  for (auto& co : h_combA_) comb += 8.0 * co.n * co.n * (double)(co.t1 - co.t0);
   for (auto& co : h_comb1_) comb += 8.0 * co.n * co.n * (double)(co.t1 - co.t0);
   for (auto& co : h_comb3_) comb += 8.0 * co.n * co.n * (double)(co.t1 - co.t0);
   phaseFlops_[5] = comb;
@@ -817,7 +950,12 @@ int Engine::plan_gemm() {
         if (!p.top()) g.ids.push_back(holeslot_[l][p.addr]);
         tl.push_back(g);
       }
-      std::vector<Summand> sm = compress_ ? aggregate(tl, sdim_[p.addr], poolOff, gcomb) : tl;
+      std::vector<Summand> sm;
+      if (reduced()) {
+        if (!gsumm_.empty()) sm = gsumm_[v.addr];
+      } else {
+        sm = compress_ ? aggregate(tl, sdim_[p.addr], poolOff, gcomb) : tl;
+      }
       const int64_t yv = gw;  // Y_v (N_p elements)
       gw += p.N;
       if (sm.empty()) {
@@ -1070,6 +1208,7 @@ void Engine::dump_plan() const {
                    name, i, g.kind, g.prec, (long long)g.ntasks, outs, kmin, kmax, g.flops, g.bytes);
     }
   };
+  std::fprintf(stderr, "plan single-matrix flops %.3e, summed contractions %zu\n", lflops_, fused_.size());
   one("build", gBuild_);
   one("hole", gHole_);
   one("apply", gApply_);
@@ -1134,6 +1273,15 @@ int Engine::run_launches(const std::vector<GLaunch>& L, size_t i0, size_t i1, vo
                                   gl.lds, active, s, kt)))
         return rc;
       if (timing_) tfl_[9] += gl.flops, tby_[9] += gl.bytes;
+    } else if (gl.kind == 4) {
+      if ((rc = kernel_mark(7, &kt))) return rc;
+      const GcSum* t = d_gs_ + gl.d0;
+      rc = gl.prec == P64 ? launch_gc_sum<double>(gl.nt, t, gl.ntasks, t + gl.ntasks, gl.nsums, d_seg_, bases[gl.x0],
+                                                  bases[gl.x1], bases[gl.o], d_part_, s, kt)
+                          : launch_gc_sum<float>(gl.nt, t, gl.ntasks, t + gl.ntasks, gl.nsums, d_seg_, bases[gl.x0],
+                                                 bases[gl.x1], bases[gl.o], d_part_, s, kt);
+      if (rc) return rc;
+      if (timing_) tfl_[7] += gl.flops, tby_[7] += gl.bytes;
     } else {
       if ((rc = kernel_mark(8, &kt))) return rc;
       if ((rc = launch_solve(d_solve_, gl.nd, (cplx<double>*)bases[B_POOL64], nspf_, active, s, kt,
@@ -1152,12 +1300,18 @@ int Engine::build_gemm(hipStream_t s) {
   void* bases[B_COUNT] = {d_psi32_, d_work32_, d_pool_, d_psi64_, d_apply64_, d_dpsi64_, d_pool64_, d_work_};
   // represent and the density tree, layer by layer in shared launches
   if ((rc = run_launches(gBuild_, bases, nullptr, 1.0, 0.0, s))) return rc;
+  // the state that get_matrix forms single terms' matrices from (full_engine)
+  auto keep_state = [&](hipStream_t t) {
+    return d_psiBuilt_ ? launch_copy_vec(d_psi64_, d_psiBuilt_, 2 * tree_.total, t) : (int)QTG_OK;
+  };
+  ++builds_;
   if (heevSide_) {
     // side stream: the eigensolver (it only feeds the solve of the finish,
     // which apply_gemm makes wait for it); engine stream: the holes, the
     // combinations and Apply
     QTG_HIP_TRY(hipEventRecord(evFork_, s));
     QTG_HIP_TRY(hipStreamWaitEvent(side_, evFork_, 0));
+    if ((rc = keep_state(side_))) return rc;
     if ((rc = begin_mark(1, side_))) return rc;
     if ((rc = launch_heev<double>(d_eig_, nEig_, d_pool_, d_pool64_, eps_, nspf_, side_))) return rc;
     if ((rc = end_mark(side_))) return rc;
@@ -1165,8 +1319,15 @@ int Engine::build_gemm(hipStream_t s) {
     heevPending_ = true;
   } else {
     // in line on the engine stream
+    if ((rc = keep_state(s))) return rc;
     if ((rc = begin_mark(1, s))) return rc;
     if ((rc = launch_heev<double>(d_eig_, nEig_, d_pool_, d_pool64_, eps_, nspf_, s))) return rc;
+    if ((rc = end_mark(s))) return rc;
+  }
+  // sums of single h-matrices, which the mean fields read
+  if (!h_combA_.empty()) {
+    if ((rc = begin_mark(5, s))) return rc;
+    if ((rc = launch_combine<double>(d_combA_, (int64_t)h_combA_.size(), d_combtA_, d_pool_, s))) return rc;
     if ((rc = end_mark(s))) return rc;
   }
   if ((rc = run_launches(gHole_, bases, nullptr, 1.0, 0.0, s))) return rc;

@@ -246,6 +246,103 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
+// ----------------------------------------------------- summed contractions
+// One workgroup per macro tile and share: its wavefronts split the
+// concatenated reduction of all segments evenly, so a sum over many small
+// contractions (the summed matrices of a sweep) is as wide as one long one
+// and needs neither a matrix per segment nor a pass to add them.
+template <typename T, int NT, int W>
+__global__ void __launch_bounds__(64 * W)
+    gc_sum_kernel(const GcSum* __restrict__ tasks, const GcSeg* __restrict__ segs, const cplx<T>* __restrict__ X0,
+                  const cplx<T>* __restrict__ X1, cplx<double>* O, cplx<double>* part) {
+  typedef typename MF<T>::v4 v4;
+  constexpr int NB = NT > 1 ? 2 : 1;
+  __shared__ cplx<double> red[NB * W * 256];
+  const GcSum d = tasks[blockIdx.x];
+  const int wave = wave_id(), lane = threadIdx.x & 63;
+  const int TJ = (d.n + 16 * NT - 1) / (16 * NT), lt = d.tile / TJ, jt = d.tile - lt * TJ;
+  const int j0 = jt * 16 * NT, l0 = lt * 16 * NT;
+  const int nrb = min(NT, (d.n - j0 + 15) >> 4), ncb = min(NT, (d.n - l0 + 15) >> 4);
+  const int K = d.bef * d.aft, nseg = d.seg1 - d.seg0;
+  const int64_t Kt = (int64_t)K * nseg;
+  const int64_t nch = (int64_t)W * d.S;
+  const int64_t chunk = ((Kt + nch - 1) / nch + 3) & ~(int64_t)3;
+  const int64_t kb = min(Kt, ((int64_t)d.share * W + wave) * chunk), ke = min(Kt, kb + chunk);
+  GcDesc g{};
+  g.bef = d.bef;
+  g.nx = g.ny = d.n;
+  g.aft = d.aft;
+  v4 cr[NT][NT], ci[NT][NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) cr[i][j] = ci[i][j] = v4{0, 0, 0, 0};
+  int sg = kb < ke ? (int)(kb / K) : nseg;
+  for (; sg < nseg && (int64_t)sg * K < ke; ++sg) {
+    const int64_t s0 = (int64_t)sg * K;
+    const GcSeg e = segs[d.seg0 + sg];
+    g.x = e.x;
+    g.y = e.y;
+    const int lo = (int)(max(kb, s0) - s0), hi = (int)(min(ke, s0 + K) - s0);
+    const cplx<T>* X = (e.sel & 1) ? X1 : X0;
+    const cplx<T>* Y = (e.sel & 2) ? X1 : X0;
+    if constexpr (NT == 1) {
+      gc_block_product<T, 1, 1, 1, 4>(g, j0, l0, lo, hi, X, Y, cr, ci);
+    } else {
+      if (nrb == 1 && ncb == 1) gc_block_product<T, NT, 1, 1, 4>(g, j0, l0, lo, hi, X, Y, cr, ci);
+      else if (nrb == 1) gc_block_product<T, NT, 1, 2, 2>(g, j0, l0, lo, hi, X, Y, cr, ci);
+      else if (ncb == 1) gc_block_product<T, NT, 2, 1, 2>(g, j0, l0, lo, hi, X, Y, cr, ci);
+      else gc_block_product<T, NT, 2, 2, 2>(g, j0, l0, lo, hi, X, Y, cr, ci);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    if (i >= nrb) break;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      if (j >= ncb) break;
+      cplx<double>* buf = red + (NB > 1 ? ((i * NT + j) & 1) * W * 256 : 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) buf[wave * 256 + q * 64 + lane] = mk<double>((double)cr[i][j][q], (double)ci[i][j][q]);
+      __syncthreads();
+      if (threadIdx.x < 256) {
+        const int e = threadIdx.x, el = e & 63;
+        cplx<double> v = buf[e];
+#pragma unroll
+        for (int w = 1; w < W; ++w) v = cadd(v, buf[w * 256 + e]);
+        const int row = j0 + i * 16 + MF<T>::drow(el, e >> 6), col = l0 + j * 16 + (el & 15);
+        if (d.S > 1) {
+          part[((((int64_t)d.part + d.share) * NT + j) * NT + i) * 256 + e] = v;
+        } else if (row < d.n && col < d.n) {
+          const int64_t o = row + (int64_t)col * d.n;
+          if (d.add >= 0) v = cadd(v, O[d.add + o]);
+          O[d.out + o] = v;
+        }
+      }
+    }
+    if (NB > 1 && (ncb & 1) && i + 1 < nrb) __syncthreads();  // as in gc_block
+  }
+}
+
+// The shares of a macro tile, added in order: one workgroup per 16 x 16 tile.
+template <typename T, int NT>
+__global__ void __launch_bounds__(256)
+    gc_sum_add(const GcSum* __restrict__ sums, const cplx<double>* __restrict__ part, cplx<double>* O) {
+  const GcSum d = sums[blockIdx.x / (NT * NT)];
+  const int sub = blockIdx.x % (NT * NT), i = sub % NT, j = sub / NT;
+  const int TJ = (d.n + 16 * NT - 1) / (16 * NT), lt = d.tile / TJ, jt = d.tile - lt * TJ;
+  const int e = threadIdx.x, el = e & 63;
+  const int row = (jt * NT + i) * 16 + MF<T>::drow(el, e >> 6), col = (lt * NT + j) * 16 + (el & 15);
+  if (row >= d.n || col >= d.n) return;
+  const cplx<double>* p = part + (((int64_t)d.part * NT + j) * NT + i) * 256 + e;
+  cplx<double> v = czero<double>();
+#pragma unroll 8
+  for (int s = 0; s < d.S; ++s) v = cadd(v, p[(int64_t)s * (NT * NT * 256)]);
+  const int64_t o = row + (int64_t)col * d.n;
+  if (d.add >= 0) v = cadd(v, O[d.add + o]);
+  O[d.out + o] = v;
+}
+
 // ------------------------------------------------------------- mode product
 // out(b,i,a) = alpha sum_l op(M)(i,l) X(b,l,a) (+ out) on RB x CB tiles of
 // 16 rows (flattened (b, a)) x 16 columns i, KS k-steps of four per stage,
@@ -390,6 +487,30 @@ __global__ void __launch_bounds__(256)
 }
 
 }  // namespace
+
+template <typename T>
+int launch_gc_sum(int nt, const GcSum* tasks, int64_t ntasks, const GcSum* sums, int64_t nsums, const GcSeg* segs,
+                  const void* x0, const void* x1, void* obase, void* part, hipStream_t s, const KernelTiming* kt) {
+  if (ntasks <= 0) return QTG_OK;
+#define QTG_GCS(NT, W)                                                                                              \
+  launch_timed(gc_sum_kernel<T, NT, W>, dim3((unsigned)ntasks), dim3(64 * W), 0, s, kt, tasks, segs,                \
+               (const cplx<T>*)x0, (const cplx<T>*)x1, (cplx<double>*)obase, (cplx<double>*)part);                  \
+  if (nsums > 0)                                                                                                    \
+    hipLaunchKernelGGL((gc_sum_add<T, NT>), dim3((unsigned)(nsums * NT * NT)), dim3(256), 0, s, sums,               \
+                       (const cplx<double>*)part, (cplx<double>*)obase)
+  if (nt == 1) {
+    QTG_GCS(1, 8);
+  } else {
+    QTG_GCS(2, 4);
+  }
+#undef QTG_GCS
+  QTG_LAUNCH_CHECK();
+  return QTG_OK;
+}
+template int launch_gc_sum<double>(int, const GcSum*, int64_t, const GcSum*, int64_t, const GcSeg*, const void*,
+                                   const void*, void*, void*, hipStream_t, const KernelTiming*);
+template int launch_gc_sum<float>(int, const GcSum*, int64_t, const GcSum*, int64_t, const GcSeg*, const void*,
+                                  const void*, void*, void*, hipStream_t, const KernelTiming*);
 
 template <typename T, typename TM, typename TO>
 int launch_gm_block(const GmDesc* descs, const int32_t* wgdesc, int64_t ntasks, const void* x0, const void* x1,

@@ -202,6 +202,29 @@ template <typename T>
 int launch_gc_one(const GcDesc& d, const GcOnePlan& p, const void* x, const void* y, void* o, void* part,
                   hipStream_t s);
 
+// Summed hole contraction (gemm_block.hip): out(j, l) = add(j, l) + sum over
+// segments of sum_{b,a} conj(X(b,j,a)) Y(b,l,a), X and Y (bef, n, aft) at
+// the segment's offsets.  A GcSum is one macro tile of nt x nt 16 x 16 tiles
+// (of ceil(n / (16 nt))^2) and one of its S shares of the concatenated
+// reduction; with S > 1 the share leaves nt^2 256 elements at that many times
+// (part + share) and a second launch over one GcSum per macro tile adds them
+// in order.  nt 1: 8 wavefronts a workgroup, for n <= 16; nt 2: 4 (twice as
+// many spill registers).
+struct GcSeg {
+  int64_t x, y;
+  int32_t sel, pad;  // as GcDesc::sel
+};
+struct GcSum {
+  int64_t out, add;  // add < 0: none
+  int32_t bef, n, aft, tile;
+  int32_t seg0, seg1, share, S;
+  int32_t part, pad;
+};
+template <typename T>
+int launch_gc_sum(int nt, const GcSum* tasks, int64_t ntasks, const GcSum* sums, int64_t nsums, const GcSeg* segs,
+                  const void* x0, const void* x1, void* obase, void* part, hipStream_t s,
+                  const KernelTiming* kt = nullptr);
+
 // Real FP64 mode product (op GM_N or GM_T; one descriptor, no K split).
 int launch_gm_real(const GmDesc& d, const double* x, const double* m, double* o, hipStream_t s);
 

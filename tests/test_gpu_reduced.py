@@ -1,0 +1,135 @@
+"""The reduced sweep (engine_reduce.cpp: sums of h-matrices and holes formed
+as contractions) against the oracle and against the sweep that forms every
+matrix, on trees and Hamiltonians that its choices depend on.  Small plans are
+left alone by its rule, so the tests move the line to zero."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import qutree_amd as Q
+from qutree_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(rng, d):
+    A = rng.normal(size=(d, d)) + 1j * rng.normal(size=(d, d))
+    return A + A.conj().T
+
+
+def _three_body(f, d, seed):
+    """One-, two- and three-mode products of explicit matrices with complex
+    coefficients (not Hermitian as a whole), repeated factors among them."""
+    rng = np.random.default_rng(seed)
+    H = W.Hamiltonian()
+    mats = [_rand(rng, d) for _ in range(4)]
+    for i in range(f):
+        H.add_term(0.3 + 0.1j * i, [(i, W.FACTOR_MATRIX, mats[i % 4])])
+        H.add_term(0.05, [(i, W.FACTOR_X), ((i + 1) % f, W.FACTOR_X), ((i + 3) % f, W.FACTOR_MATRIX, mats[i % 4])])
+        H.add_term(0.2j, [(i, W.FACTOR_X2), ((i + 2) % f, W.FACTOR_KIN)])
+    H.add_term(0.7, [(j, W.FACTOR_MATRIX, mats[j % 4]) for j in range(f)])
+    H.add_term(-0.4, [(0, W.FACTOR_MATRIX, mats[0])])  # the first term's factor again
+    return H
+
+
+def _models():
+    return {
+        "f4": (W.balanced_tree_text(4, 3, [2, 3]), W.coupled_ho(4, 11, c_sigma=0.1)),
+        "cmf8": W.cmf8_model(),
+        "quartic16": (W.balanced_tree_text(16, 6, [4, 6, 8, 8]), W.coupled_quartic(16, 5, c_sigma=0.01)),
+        "wide8": (W.balanced_tree_text(8, 8, [8, 18, 33]), W.coupled_quartic(8, 5, c_sigma=0.05)),
+        "three8": (W.balanced_tree_text(8, 5, [4, 7, 9]), _three_body(8, 5, 3)),
+        "one_mode": (W.balanced_tree_text(8, 5, [4, 6, 6]), _one_mode(8)),
+    }
+
+
+def _one_mode(f):
+    H = W.Hamiltonian()
+    for i in range(f):
+        H.add_term(1.0, [(i, W.FACTOR_KIN)])
+        H.add_term(0.5 + 0.1 * i, [(i, W.FACTOR_X2)])
+    return H
+
+
+@pytest.fixture
+def every_size(monkeypatch):
+    monkeypatch.setenv("QTG_REDUCE_MIN_FLOPS", "0")
+
+
+def _err(x, y):
+    return np.linalg.norm(x - y) / np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("heev_side", [1, 0])
+@pytest.mark.parametrize("name", sorted(_models()))
+def test_reduced_sweep_matches_oracle(name, heev_side, every_size):
+    text, H = _models()[name]
+    print(f"case reduced sweep {name} heev_side={heev_side}", flush=True)
+    om = O.OracleModel(text, H)
+    psi = om.fill_random(5, delta_lowest=False)
+    ref = om.derivative(psi)
+    # rho^-1 amplifies rounding by the smallest density eigenvalue (wide8: a
+    # random 33 x 33 top node): the sweep that forms every matrix shows by how
+    # much on this state
+    full = Q.Engine(text, H, compress=False)
+    full.set_psi(psi)
+    full.derivative()
+    lim = max(1e-12, 4 * _err(full.get(0), ref))
+    eng = Q.Engine(text, H, heev_side=heev_side)
+    for _ in range(2):  # captured, then replayed
+        eng.set_psi(psi)
+        eng.derivative()
+        got = eng.get(0)
+        print(f"  derivative rel err {_err(got, ref):.2e} limit {lim:.2e}", flush=True)
+        assert _err(got, ref) < lim
+    e = om.energy(psi)
+    assert abs(eng.energy() - e) < 1e-12 * abs(e)
+
+
+@pytest.mark.parametrize("name", sorted(_models()))
+def test_reduced_sweep_matrices_of_single_terms(name, every_size):
+    """get_matrix after a reduced sweep forms the terms' matrices at the state
+    of the last build, also when the state has been replaced since."""
+    text, H = _models()[name]
+    print(f"case reduced matrices {name}", flush=True)
+    om = O.OracleModel(text, H)
+    eng = Q.Engine(text, H)
+    for seed in (1, 2):
+        psi = om.fill_random(seed, delta_lowest=False)
+        om.build(psi)
+        eng.set_psi(psi)
+        eng.derivative()
+        if seed == 2:
+            eng.set_psi(om.fill_random(3, delta_lowest=False))
+        for l in range(0, H.nterms, max(1, H.nterms // 7)):
+            for a in om.sparse_tree(l):
+                if a == om.nnodes - 1:
+                    continue
+                h, g = om.hmat(l, a), om.hole(l, a)
+                assert np.max(np.abs(eng.matrix(2, l, a) - h)) < 1e-11 * max(1, np.max(np.abs(h)))
+                assert np.max(np.abs(eng.matrix(3, l, a) - g)) < 1e-11 * max(1, np.max(np.abs(g)))
+
+
+@pytest.mark.parametrize("name", ["f4", "cmf8", "quartic16", "wide8"])
+def test_reduced_gradient_and_split_precision(name, every_size):
+    text, H = _models()[name]
+    print(f"case reduced gradient, split {name}", flush=True)
+    om = O.OracleModel(text, H)
+    psi = om.fill_random(21, delta_lowest=False)
+    ref, e_ref = om.gradient(psi)
+    eng = Q.Engine(text, H)
+    eng.set_psi(psi)
+    got, e = eng.gradient()
+    print(f"  gradient rel err {_err(got, ref):.2e}", flush=True)
+    assert _err(got, ref) < 1e-11 and abs(e - e_ref) < 1e-12 * abs(e_ref)
+    dref = om.derivative(psi)
+    full = Q.Engine(text, H, precision=2, compress=False)
+    red = Q.Engine(text, H, precision=2)
+    errs = []
+    for g in (full, red):
+        g.set_psi(psi)
+        g.derivative()
+        errs.append(_err(g.get(0), dref))
+        assert abs(g.energy() - e_ref) < 1e-9 * abs(e_ref)
+    print(f"  split derivative err, every matrix {errs[0]:.2e} reduced {errs[1]:.2e}", flush=True)
+    assert errs[1] < max(4 * errs[0], 1e-7)
