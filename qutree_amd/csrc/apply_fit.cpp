@@ -354,6 +354,7 @@ int ApplyFit::init() {
         qr_item(tmp[i], nd.off, nd.N / nd.n, nd.n);
       }
       q.n = (int64_t)nodes.size();
+      qr_extent(q);
       iter_.push_back(q);
       std::vector<GcDesc> gcs;
       for (size_t i = 0; i < nodes.size(); ++i) {

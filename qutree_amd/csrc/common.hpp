@@ -56,6 +56,28 @@ __host__ __device__ inline cplx<T> cconj(const cplx<T>& a) {
   return mk<T>(a.re, -a.im);
 }
 
+// Sum over the 64 lanes, the same value in every lane, on the vector ALU
+// alone: neighbours, quads, half rows and rows by lane permutations within a
+// row of 16, then the row totals broadcast upward (row_bcast 15 and 31) and
+// lane 63 read.  Six cross-lane steps through LDS (__shfl) take about five
+// times as long, which is most of a serial chain of reductions.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+  return v + __hiloint2double(hi, lo);
+}
+__device__ inline double wave_total(double v) {
+  v = dpp_add<0xB1, 0xf>(v);   // quad_perm [1,0,3,2]
+  v = dpp_add<0x4E, 0xf>(v);   // quad_perm [2,3,0,1]
+  v = dpp_add<0x141, 0xf>(v);  // row_half_mirror
+  v = dpp_add<0x140, 0xf>(v);  // row_mirror: every lane its row's total
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast31 into rows 2 and 3
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
 // per-thread last error of the C ABI
 void set_error(const std::string& msg);
 const char* get_error();

@@ -13,6 +13,8 @@
 // No reference counterpart; rho^-1 (1 - P) of the gradient is the
 // reference's imaginary-time LayerDerivative (HamiltonianRepresentation.cpp:
 // 45-72 with phase -i, Eigenstates.cpp:75).
+#include <algorithm>
+
 #include "engine.hpp"
 #include "grad_ops.hpp"
 #include "smallmat.hpp"
@@ -93,9 +95,15 @@ int Engine::canonicalize(hipStream_t s) {
   int rc;
   for (size_t d = 0; d < canonRange_.size(); ++d) {
     const auto& r = canonRange_[d];
+    int64_t mmax = 0;
+    int nmax = 0;
+    for (int64_t i = r.first; i < r.second; ++i) {
+      mmax = std::max<int64_t>(mmax, h_canon_[i].m);
+      nmax = std::max(nmax, h_canon_[i].n);
+    }
     if (r.second > r.first &&
-        (rc = launch_qr_batch(d_canon_ + r.first, SmItem{}, SmItem{}, r.second - r.first, d_psi64_, d_psi64_, s,
-                              d_pool_)))
+        (rc = launch_qr_batch(d_canon_ + r.first, SmItem{}, SmItem{}, r.second - r.first, mmax, nmax, d_psi64_,
+                              d_psi64_, s, d_pool_)))
       return rc;
     if ((rc = run_launches(gCanon_[d], bases, nullptr, 1.0, 0.0, s))) return rc;
   }

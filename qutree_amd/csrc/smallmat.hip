@@ -41,10 +41,7 @@ __device__ inline SmItem item_of(const SmItem* __restrict__ items, const SmItem&
   return it;
 }
 
-__device__ inline double wsum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+__device__ inline double wsum(double v) { return wave_total(v); }
 
 __global__ void __launch_bounds__(EW)
     heev_batch_kernel(const SmItem* __restrict__ items, SmItem u, SmItem st, const z* __restrict__ in, z* U,
@@ -306,6 +303,183 @@ __global__ void __launch_bounds__(kQrThreads)
   qr_inplace(W, m, n, tau, (Rb && it.e >= 0) ? Rb + it.e : nullptr);
 }
 
+// The same QR with the matrix in registers: wavefront w of W holds columns
+// w, w + W, ... (at most CW), a lane rows lane + 64 t (t < RT).  The
+// owner of column j forms the reflector and leaves v in LDS; after one
+// barrier every wavefront applies it to its own columns, each a dot product
+// over the lanes' rows and a wavefront sum.  qr_inplace walks the same columns
+// in global memory with two dependent passes and two barriers a column: one
+// 576 x 24 matrix (221 KB, more than LDS) takes 617 us there and 78 us here,
+// 64 x 64 741 and 190, 196 x 16 138 and 32, 8 x 8 26 and 11.
+// pos: column signs with R's diagonal positive (the Q of Gram-Schmidt).
+template <int RT, int CW, int W>
+__global__ void __launch_bounds__(64 * W)
+    qr_reg_kernel(const SmItem* __restrict__ items, SmItem u, SmItem st, const z* in, z* out, z* Rb, int pos) {
+  __shared__ z vb[2][64 * RT];
+  __shared__ z tau[64];
+  const SmItem it = item_of(items, u, st);
+  const int m = (int)it.m, n = it.n;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const z* A = in + it.a;
+  z a[CW][RT];
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    const int k = c * W + wave;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      const int r = lane + 64 * t;
+      a[c][t] = (k < n && r < m) ? A[r + (int64_t)k * m] : czero<double>();
+    }
+  }
+  int buf = 0;
+  // reflectors in order; column c W + w belongs to wavefront w
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    for (int w = 0; w < W; ++w) {
+      const int j = c * W + w;
+      if (j >= n) break;
+      if (wave == w) {
+        double s = 0.0;
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+          if (lane + 64 * t > j) s += a[c][t].re * a[c][t].re + a[c][t].im * a[c][t].im;
+        s = wsum(s);
+        const z alpha = mk<double>(__shfl(a[c][0].re, j, 64), __shfl(a[c][0].im, j, 64));
+        z t1 = czero<double>(), sc = mk<double>(1.0, 0.0);
+        double beta = alpha.re;
+        if (!(s == 0.0 && alpha.im == 0.0)) {
+          const double nr = sqrt(alpha.re * alpha.re + alpha.im * alpha.im + s);
+          beta = alpha.re >= 0.0 ? -nr : nr;
+          t1 = mk<double>((beta - alpha.re) / beta, -alpha.im / beta);
+          const z dlt = mk<double>(alpha.re - beta, alpha.im);
+          const double dd = dlt.re * dlt.re + dlt.im * dlt.im;
+          sc = mk<double>(dlt.re / dd, -dlt.im / dd);
+        }
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          const int r = lane + 64 * t;
+          if (r > j) a[c][t] = cmul(a[c][t], sc);
+          else if (r == j) a[c][t] = mk<double>(beta, 0.0);
+          vb[buf][r] = r > j ? a[c][t] : mk<double>(r == j ? 1.0 : 0.0, 0.0);
+        }
+        if (lane == 0) tau[j] = t1;
+      }
+      __syncthreads();
+      const z t1 = tau[j];
+      if (t1.re != 0.0 || t1.im != 0.0) {
+        z v[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) v[t] = vb[buf][lane + 64 * t];
+        // all dot products, then all their sums side by side
+        double sr[CW], si[CW];
+#pragma unroll
+        for (int d = c; d < CW; ++d) {
+          sr[d] = si[d] = 0.0;
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+            sr[d] += v[t].re * a[d][t].re + v[t].im * a[d][t].im;
+            si[d] += v[t].re * a[d][t].im - v[t].im * a[d][t].re;
+          }
+        }
+#pragma unroll
+        for (int d = c; d < CW; ++d) {
+          sr[d] = wsum(sr[d]);
+          si[d] = wsum(si[d]);
+        }
+#pragma unroll
+        for (int d = c; d < CW; ++d) {
+          if (d == c && wave <= w) continue;  // a column that is done
+          const z f = mk<double>(t1.re * sr[d] + t1.im * si[d], t1.re * si[d] - t1.im * sr[d]);  // conj(tau) s
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+            a[d][t].re -= v[t].re * f.re - v[t].im * f.im;
+            a[d][t].im -= v[t].re * f.im + v[t].im * f.re;
+          }
+        }
+      }
+      buf ^= 1;
+    }
+  }
+  // R: the diagonal and above (rows below 64 are the t = 0 elements); sgn:
+  // whether a column changes sign for a positive diagonal
+  z* R = (Rb && it.e >= 0) ? Rb + it.e : nullptr;
+  bool neg[CW];
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    const int k = c * W + wave;
+    neg[c] = pos && __shfl(a[c][0].re, min(k, 63), 64) < 0.0;
+    if (R && k < n && lane < n) R[lane + k * n] = lane <= k ? a[c][0] : czero<double>();
+  }
+  // thin Q, backward.  A buffer is written two barriers after its last read.
+#pragma unroll
+  for (int c = CW - 1; c >= 0; --c) {
+    for (int w = W - 1; w >= 0; --w) {
+      const int i = c * W + w;
+      if (i >= n) continue;
+      if (wave == w) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          const int r = lane + 64 * t;
+          vb[buf][r] = r > i ? a[c][t] : mk<double>(r == i ? 1.0 : 0.0, 0.0);
+        }
+      }
+      __syncthreads();
+      const z t1 = tau[i];
+      z v[RT];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) v[t] = vb[buf][lane + 64 * t];
+      double sr[CW], si[CW];
+#pragma unroll
+      for (int d = c; d < CW; ++d) {
+        sr[d] = si[d] = 0.0;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          sr[d] += v[t].re * a[d][t].re + v[t].im * a[d][t].im;
+          si[d] += v[t].re * a[d][t].im - v[t].im * a[d][t].re;
+        }
+      }
+#pragma unroll
+      for (int d = c; d < CW; ++d) {
+        sr[d] = wsum(sr[d]);
+        si[d] = wsum(si[d]);
+      }
+#pragma unroll
+      for (int d = c; d < CW; ++d) {
+        if (d == c && wave <= w) continue;
+        const z f = mk<double>(t1.re * sr[d] - t1.im * si[d], t1.re * si[d] + t1.im * sr[d]);  // tau s
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          a[d][t].re -= v[t].re * f.re - v[t].im * f.im;
+          a[d][t].im -= v[t].re * f.im + v[t].im * f.re;
+        }
+      }
+      if (wave == w) {
+        const z mt = mk<double>(-t1.re, -t1.im);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          const int r = lane + 64 * t;
+          if (r < i) a[c][t] = czero<double>();
+          else if (r == i) a[c][t] = mk<double>(1.0 - t1.re, -t1.im);
+          else a[c][t] = cmul(mt, a[c][t]);
+        }
+      }
+      buf ^= 1;
+    }
+  }
+  z* Q = out + it.q;
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    const int k = c * W + wave;
+    if (k >= n) continue;
+    const double g = neg[c] ? -1.0 : 1.0;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      const int r = lane + 64 * t;
+      if (r < m) Q[r + (int64_t)k * m] = mk<double>(g * a[c][t].re, g * a[c][t].im);
+    }
+  }
+}
+
 }  // namespace
 
 int launch_heev_batch(const SmItem* items, const SmItem& u, const SmItem& st, int64_t count, int nmax,
@@ -336,11 +510,30 @@ int launch_inverse_batch(const SmItem* items, const SmItem& u, const SmItem& st,
   return QTG_OK;
 }
 
-int launch_qr_batch(const SmItem* items, const SmItem& u, const SmItem& st, int64_t count, const void* in, void* out,
-                    hipStream_t s, void* R) {
+int launch_qr_batch(const SmItem* items, const SmItem& u, const SmItem& st, int64_t count, int64_t mmax, int nmax,
+                    const void* in, void* out, hipStream_t s, void* R, bool positive) {
   if (count <= 0) return QTG_OK;
-  hipLaunchKernelGGL(qr_batch_kernel, dim3((unsigned)count), dim3(kQrThreads), 0, s, items, u, st, (const z*)in,
-                     (z*)out, (z*)R);
+  const dim3 grid((unsigned)count);
+#define QTG_QR(RT, CW, W)                                                                                        \
+  hipLaunchKernelGGL((qr_reg_kernel<RT, CW, W>), grid, dim3(64 * W), 0, s, items, u, st, (const z*)in, (z*)out,   \
+                     (z*)R, positive ? 1 : 0)
+  // the smallest register form that holds the largest matrix: 64 RT rows,
+  // CW W columns
+  if (mmax <= 64 && nmax <= 8) QTG_QR(1, 1, 8);
+  else if (mmax <= 64 && nmax <= 24) QTG_QR(1, 3, 8);
+  else if (mmax <= 64) QTG_QR(1, 4, 16);
+  else if (mmax <= 128 && nmax <= 24) QTG_QR(2, 3, 8);
+  else if (mmax <= 256 && nmax <= 16) QTG_QR(4, 2, 8);
+  else if (mmax <= 256 && nmax <= 24) QTG_QR(4, 3, 8);
+  else if (mmax <= 256) QTG_QR(4, 4, 16);
+  else if (mmax <= 576 && nmax <= 24) QTG_QR(9, 3, 8);
+  else if (positive) {
+    set_error("qr: a positive diagonal is formed by the register kernels only");
+    return QTG_ESHAPE;
+  } else {
+    hipLaunchKernelGGL(qr_batch_kernel, grid, dim3(kQrThreads), 0, s, items, u, st, (const z*)in, (z*)out, (z*)R);
+  }
+#undef QTG_QR
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }
@@ -408,7 +601,7 @@ int qtg_qr_batch_z(const double* A, double* Q, int64_t m, int64_t n, int64_t cou
   if (rc) return rc;
   SmItem u = uniform(m, n);
   u.e = -1;  // no R
-  return launch_qr_batch(nullptr, u, strides(m * n, m * n, 0), count, A, Q, S(stream), nullptr);
+  return launch_qr_batch(nullptr, u, strides(m * n, m * n, 0), count, m, (int)n, A, Q, S(stream), nullptr);
 }
 
 }  // extern "C"

@@ -21,10 +21,15 @@ int launch_heev_batch(const SmItem* items, const SmItem& u, const SmItem& st, in
                       const void* in, void* U, double* ev, void* R, double eps, hipStream_t s);
 int launch_inverse_batch(const SmItem* items, const SmItem& u, const SmItem& st, int64_t count, int nmax,
                          const void* in, void* out, hipStream_t s);
-// thin Q of every (m x n) item, n <= 64, m >= n; in and out may alias.
-// With R non-null, an item with e >= 0 also writes its n x n upper
-// triangular R (A = Q R) at R + e.
-int launch_qr_batch(const SmItem* items, const SmItem& u, const SmItem& st, int64_t count, const void* in, void* out,
-                    hipStream_t s, void* R = nullptr);
+// thin Q of every (m x n) item, n <= 64, m >= n, none larger than mmax x
+// nmax; in and out may alias.  With R non-null, an item with e >= 0 also
+// writes its n x n upper triangular R (A = Q R) at R + e.  positive: the Q
+// whose R has a positive diagonal (R itself is not adjusted), for matrices
+// that qr_in_registers.
+int launch_qr_batch(const SmItem* items, const SmItem& u, const SmItem& st, int64_t count, int64_t mmax, int nmax,
+                    const void* in, void* out, hipStream_t s, void* R = nullptr, bool positive = false);
+inline bool qr_in_registers(int64_t m, int n) {
+  return m <= 256 || (m <= 576 && n <= 24);
+}
 
 }  // namespace qtg

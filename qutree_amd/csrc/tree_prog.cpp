@@ -278,6 +278,15 @@ int TreeProg::emit_stack(std::vector<Step>& comb, std::vector<Step>& body, int a
   return QTG_OK;
 }
 
+// the largest matrix of a batch, for its kernel's choice
+void TreeProg::qr_extent(Step& st) const {
+  st.bef = st.nn = 0;
+  for (int64_t i = 0; i < st.n; ++i) {
+    st.bef = std::max<int64_t>(st.bef, h_qr_[st.d0 + i].m);
+    st.nn = std::max<int64_t>(st.nn, h_qr_[st.d0 + i].n);
+  }
+}
+
 int64_t TreeProg::qr_item(int64_t a, int64_t q, int64_t rows, int n) {
   SmItem it{};
   it.a = a;
@@ -454,12 +463,12 @@ int TreeProg::run_steps(const std::vector<Step>& P, hipStream_t s) {
         u.e = -1;
         u.m = st.bef;
         u.n = (int32_t)st.nn;
-        rc = launch_qr_batch(nullptr, u, zero, 1, st.abuf ? (void*)work_ : (void*)psi_,
+        rc = launch_qr_batch(nullptr, u, zero, 1, u.m, u.n, st.abuf ? (void*)work_ : (void*)psi_,
                              st.cbuf ? (void*)work_ : (void*)psi_, s);
         break;
       }
       case K_QRB:
-        rc = launch_qr_batch(d_qr_ + st.d0, zero, zero, st.n, st.abuf ? (void*)work_ : (void*)psi_,
+        rc = launch_qr_batch(d_qr_ + st.d0, zero, zero, st.n, st.bef, (int)st.nn, st.abuf ? (void*)work_ : (void*)psi_,
                              st.cbuf ? (void*)work_ : (void*)psi_, s);
         break;
       default:

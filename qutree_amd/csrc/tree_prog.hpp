@@ -81,6 +81,7 @@ class TreeProg {
   int emit_stack(std::vector<Step>& comb, std::vector<Step>& body, int a, int inbuf, int64_t in,
                  std::vector<StackEntry>& entries, bool entry0_is_input, int64_t stack_base, int64_t out);
   int64_t qr_item(int64_t a, int64_t q, int64_t rows, int n);
+  void qr_extent(Step& st) const;
   int run_steps(const std::vector<Step>& P, hipStream_t s);
   virtual int run_extra(const Step& st, hipStream_t s);
   int validate_steps(const std::vector<Step>& P) const;
