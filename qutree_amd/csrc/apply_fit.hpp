@@ -29,6 +29,7 @@ class ApplyFit : public TreeProg {
   using Key = std::vector<std::pair<int, int>>;
   Key restrict_key(int l, int a, bool inside) const;
   Chain r_chain(int l, int a, int skip) const;
+  void plan_start();
   int run_extra(const Step& st, hipStream_t s) override;
   int validate_extra(const Step& st, std::vector<Span>& rd, std::vector<Span>& wr) const override;
 
@@ -39,7 +40,8 @@ class ApplyFit : public TreeProg {
   std::vector<std::map<Key, int64_t>> hmat_, hole_;
   bool single_ = false;  // one product: applied to the bottom tensors directly
   int64_t ketOff_ = 0;   // the state (ket) in work
-  std::vector<Step> first_, iter_;
+  std::vector<char> startOnDevice_;  // node of the start orthonormalised by start_
+  std::vector<Step> start_, first_, iter_;
   double* fid_ = nullptr;
   hipGraphExec_t exec_ = nullptr;
   bool ready_ = false;

@@ -340,11 +340,13 @@ struct CountingGen {
 };
 }  // namespace
 
-void fill_random(const HTree& tree, uint64_t seed, bool delta_lowest, std::vector<cd>& psi) {
-  fill_random_stream(tree, seed, 0, delta_lowest, psi);
+void fill_random(const HTree& tree, uint64_t seed, bool delta_lowest, std::vector<cd>& psi,
+                 const std::vector<char>* drawn_only) {
+  fill_random_stream(tree, seed, 0, delta_lowest, psi, drawn_only);
 }
 
-int64_t fill_random_stream(const HTree& tree, uint64_t seed, int64_t discard, bool delta_lowest, std::vector<cd>& psi) {
+int64_t fill_random_stream(const HTree& tree, uint64_t seed, int64_t discard, bool delta_lowest, std::vector<cd>& psi,
+                           const std::vector<char>* drawn_only) {
   std::mt19937 mt((std::mt19937::result_type)seed);
   mt.discard((unsigned long long)discard);
   CountingGen gen{mt};
@@ -369,7 +371,7 @@ int64_t fill_random_stream(const HTree& tree, uint64_t seed, int64_t discard, bo
         A[0] = 1.0;
       }
     }
-    gram_schmidt(A, L, n.n);
+    if (!drawn_only || !(*drawn_only)[n.addr]) gram_schmidt(A, L, n.n);
   }
   return gen.n;
 }

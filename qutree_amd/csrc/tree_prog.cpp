@@ -469,7 +469,7 @@ int TreeProg::run_steps(const std::vector<Step>& P, hipStream_t s) {
       }
       case K_QRB:
         rc = launch_qr_batch(d_qr_ + st.d0, zero, zero, st.n, st.bef, (int)st.nn, st.abuf ? (void*)work_ : (void*)psi_,
-                             st.cbuf ? (void*)work_ : (void*)psi_, s);
+                             st.cbuf ? (void*)work_ : (void*)psi_, s, nullptr, st.dir == 1);
         break;
       default:
         rc = run_extra(st, s);

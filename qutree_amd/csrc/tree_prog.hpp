@@ -29,7 +29,7 @@ class TreeProg {
   enum Kind { K_GM, K_GC, K_COMB, K_LBEGIN, K_LSTEP, K_HEEV, K_KCOMB, K_PERM, K_QR, K_QRB, K_NORM };
   struct Step {
     int kind = K_GM;
-    int64_t d0 = 0, n = 0;  // descriptor range (GM, GC: tasks; COMB: outputs; QRB: items)
+    int64_t d0 = 0, n = 0;  // descriptor range (GM, GC: tasks; COMB: outputs; QRB: items, dir 1: R's diagonal positive)
     int obuf = 1;           // GM output base: 0 psi, 1 work
     int waves = 0;
     int64_t a = 0, b = 0, c = 0, d = 0;  // offsets (see the launching code)

@@ -6,7 +6,10 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import oracle_lib as O
 import qutree_amd as Q
+import test_oracle_apply_fit as TA
+from qutree_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -79,3 +82,23 @@ def test_a_column_of_nan_leaves_the_columns_before_it():
     # a column of Q depends on the columns of A up to it and on no later one
     assert np.max(np.abs(got[:, :11] - _householder(X[0, :, :11]))) < 2e-15 * 20 * 10
     assert np.isnan(got[:, 11]).any()
+
+
+@pytest.mark.parametrize("spf", [[4, 16, 18], [8, 20, 28], [5, 24, 24]])
+def test_fit_start_at_the_edges_of_the_device_orthonormalisation(spf):
+    """The fit's random start (Gram-Schmidt in the oracle): square nodes, 256
+    rows, 576 x 24, and nodes (400 x 28, a top node of 784) left to the host."""
+    print(f"case fit start {spf}", flush=True)
+    text, H = W.balanced_tree_text(8, spf[0] + 1, spf), TA.contraction_sop(8, spf[0] + 1, 4, 2)
+    om = O.OracleModel(text, H)
+    psi = om.fill_random(21, delta_lowest=False)
+    ref = om.apply_fit(psi, 5, 1)
+    got = Q.ApplyFit(Q.Engine(text, H)).run(psi, 5, 1)
+    # both starts are the exact one up to eps times a random node's condition
+    # number (square ones: some 1e2), and one iteration is a product and a QR
+    assert abs(got["fidelities"][0] / ref["fidelities"][0] - 1.0) < 1e-11
+    ov = om.overlap(ref["psi"], got["psi"])
+    n2 = om.overlap(ref["psi"], ref["psi"]).real * om.overlap(got["psi"], got["psi"]).real
+    assert abs(1.0 - abs(ov) ** 2 / n2) < 1e-11
+    top = om.nnodes - 1
+    assert np.max(np.abs(om.node_tensor(got["psi"], top) - om.node_tensor(ref["psi"], top))) < 1e-11
