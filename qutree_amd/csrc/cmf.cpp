@@ -621,7 +621,7 @@ int Cmf::cmfstep_dev(cplx<double>* P, double t0, double t1, double eps) {
     slot = slot_;
     slot_ = (slot_ + 1) % kBsRing;
     return launch_bs_tick(d_bs_, NN_, bb, E.d_nodes_, pool, rhoslot_, err_, d_rec_ + slot * recB, init, t0, t1, eps,
-                          s_);
+                          E.nmax_, s_);
   };
   int rc = boundary(1);
   if (rc) return rc;

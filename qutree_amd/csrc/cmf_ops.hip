@@ -17,15 +17,28 @@ __device__ inline cd2 cdiv(const cd2& a, const cd2& b) {
   return mk<double>((a.re * b.re + a.im * b.im) / d, (a.im * b.re - a.re * b.im) / d);
 }
 
+// Threads of the vector-op kernels: a workgroup has one node, and the largest
+// nodes set a tick's time.  With 256 threads a node of 3136 elements took 12
+// dependent memory round trips in its final op (a tick up to 43 us, with 1024 up
+// to 27 us).
+constexpr int TV = 1024;
+
+// Orders the workgroup's LDS accesses; global stores on their way are not
+// waited for.
+__device__ inline void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 __device__ inline double block_sum_d(double v, double* red) {
-  red[threadIdx.x] = v;
-  __syncthreads();
-  for (int s = TB / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  const double r = red[0];
-  __syncthreads();
+  v = wave_total(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  lds_barrier();
+  double r = 0.0;
+#pragma unroll
+  for (int w = 0; w < TV / 64; ++w) r += red[w];
+  lds_barrier();
   return r;
 }
 
@@ -50,20 +63,19 @@ static_assert(kCmfBufs == 17, "bp() covers every buffer");
 // Op::store(e, v) writes its results.  The buffers of one op are different
 // arenas, but the compiler cannot prove it, so a store would order every later
 // load behind it: a pass loads up to P elements per thread (the tail
-// predicated) before storing any, so a node of up to P * TB elements takes
-// one memory round trip per op.  P shrinks with the operands per element
-// (16 for one complex value, 8 for three) to stay in registers.
+// predicated) before storing any, so a node of up to P * TV = 4096 elements
+// takes one memory round trip per op.
 template <class Op>
 __device__ __forceinline__ void elementwise(int N, const Op& op) {
-  constexpr int P = sizeof(typename Op::Val) <= 16 ? 16 : sizeof(typename Op::Val) <= 32 ? 12 : 8;
-  for (int e0 = threadIdx.x; e0 < N; e0 += P * TB) {
+  constexpr int P = 4;
+  for (int e0 = threadIdx.x; e0 < N; e0 += P * TV) {
     typename Op::Val v[P];
 #pragma unroll
     for (int u = 0; u < P; ++u)
-      if (e0 + u * TB < N) v[u] = op.load(e0 + u * TB);
+      if (e0 + u * TV < N) v[u] = op.load(e0 + u * TV);
 #pragma unroll
     for (int u = 0; u < P; ++u)
-      if (e0 + u * TB < N) op.store(e0 + u * TB, v[u]);
+      if (e0 + u * TV < N) op.store(e0 + u * TV, v[u]);
   }
 }
 
@@ -132,6 +144,9 @@ struct StartOp {  // v = src; P <- v (when wp); y0, y3, x <- v; ytab[1..6] <- 0
     for (int k = 0; k < 6; ++k) yt[k][e] = czero<double>();
   }
 };
+// In the two ops below x and y2w are null where they are the arenas of y1
+// (which gets the same values) and of the derivative (which the Apply that
+// follows writes).
 struct MmidBeginOp {  // y0 <- y3; t = y3 + h y4; y1 <- t; x <- t
   cd2 *y0, *y1, *x;
   const cd2 *y3, *y4;
@@ -144,11 +159,13 @@ struct MmidBeginOp {  // y0 <- y3; t = y3 + h y4; y1 <- t; x <- t
     y0[e] = v.b;
     const cd2 t = mk<double>(v.b.re + h * v.c.re, v.b.im + h * v.c.im);
     y1[e] = t;
-    x[e] = t;
+    if (x) x[e] = t;
   }
 };
 struct MmidStepXOp {  // t = y0 + 2h y2; y0 <- y1; y1 <- t; y2 <- t; x <- t
-  cd2 *y0, *y1, *y2, *x;
+  cd2 *y0, *y1;
+  const cd2* y2;
+  cd2 *y2w, *x;
   double h;
   struct Val {
     cd2 a, b, c;
@@ -158,8 +175,8 @@ struct MmidStepXOp {  // t = y0 + 2h y2; y0 <- y1; y1 <- t; y2 <- t; x <- t
     const cd2 t = mk<double>(v.a.re + 2.0 * h * v.c.re, v.a.im + 2.0 * h * v.c.im);
     y0[e] = v.b;
     y1[e] = t;
-    y2[e] = t;
-    x[e] = t;
+    if (y2w) y2w[e] = t;
+    if (x) x[e] = t;
   }
 };
 struct PostExtrOp {  // y0 <- y1; y1 <- y1 + y2
@@ -175,15 +192,79 @@ struct PostExtrOp {  // y0 <- y1; y1 <- y1 + y2
   }
 };
 
+// a double that is the same in every lane, in scalar registers
+__device__ inline double uniform(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// sum over this thread's share of Re( conj(d(i,nn)) rho(nn,m) d(i,m) ), d(o)
+// being element o of the L x n difference: a row i and four columns nn a step
+template <class Diff>
+__device__ __forceinline__ double rho_norm(const Diff& d, const cd2* rho, int n, int L) {
+  double delta = 0.0;
+  const int quads = (n + 3) / 4;
+  for (int o = threadIdx.x; o < L * quads; o += TV) {
+    const int i = o % L, q0 = 4 * (o / L);
+    double tr[4] = {}, ti[4] = {};
+    cd2 dn[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const cd2 v = d(i + min(q0 + u, n - 1) * L);
+      dn[u] = q0 + u < n ? v : czero<double>();
+    }
+#pragma unroll 4
+    for (int m = 0; m < n; ++m) {
+      const cd2 v = d(i + m * L);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const cd2 r = rho[min(q0 + u, n - 1) + m * n];
+        tr[u] += r.re * v.re - r.im * v.im;
+        ti[u] += r.re * v.im + r.im * v.re;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) delta += dn[u].re * tr[u] + dn[u].im * ti[u];
+  }
+  return delta;
+}
+
+// What a tick holds for a node's error op beside the op itself: an LDS array
+// for the difference y0 - y1 that the final op before it forms (null for nodes
+// beyond it), the node's rho, loaded ahead (element threadIdx.x, n <= 16), and
+// where the error goes besides err.
+struct ErrLocal {
+  cd2* diff;
+  cd2 rho;
+  double* out;
+};
+
 // One vector op on one node (the whole workgroup; the caller synchronises
-// the workgroup before the next op).
+// the workgroup before the next op).  kTick: the ops and forms of the device
+// integrators only.
+template <bool kTick>
 __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, const DNode* __restrict__ nodes,
                                         const cd2* __restrict__ pool, const int64_t* __restrict__ rhoslot,
-                                        double* err, int node, const DNode& nd, double* red, cd2* rhos) {
+                                        double* err, int node, const DNode& nd, double* red, cd2* rhos,
+                                        const ErrLocal& el) {
   const int N = nd.N;
   const int64_t off = nd.off;
-  const VecOp op = *opp;
-  switch (op.code) {
+  // the op's words are uniform: keep them scalar
+  struct {
+    int a, b, c, i, mi;
+    double h;
+  } op;
+  op.a = __builtin_amdgcn_readfirstlane(opp->a);
+  op.b = __builtin_amdgcn_readfirstlane(opp->b);
+  op.c = __builtin_amdgcn_readfirstlane(opp->c);
+  op.i = __builtin_amdgcn_readfirstlane(opp->i);
+  op.mi = __builtin_amdgcn_readfirstlane(opp->mi);
+  op.h = uniform(opp->h);
+  const int code = __builtin_amdgcn_readfirstlane(opp->code);
+  if (kTick && (code == V_AXPY || code == V_ZERO || code == V_MMID_STEP || code == V_MMID_FINAL ||
+                code == V_RZEXTR || code == V_POST_EXTR))
+    __builtin_unreachable();
+  switch (code) {
     case V_COPY:
       elementwise(N, CopyOp{bp(bufs, op.a) + off, bp(bufs, op.b) + off});
       break;
@@ -192,7 +273,7 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
       break;
     case V_ZERO: {
       cd2* A = bp(bufs, op.a) + off;
-      for (int e = threadIdx.x; e < N; e += TB) A[e] = czero<double>();
+      for (int e = threadIdx.x; e < N; e += TV) A[e] = czero<double>();
       break;
     }
     case V_MMID_STEP:
@@ -211,12 +292,12 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
       const int mi = op.mi < kTab ? op.mi : kTab;
       double fx[kTab];
 #pragma unroll
-      for (int k2 = 1; k2 < kTab; ++k2) fx[k2] = opp->fx[k2];
+      for (int k2 = 1; k2 < kTab; ++k2) fx[k2] = uniform(opp->fx[k2]);
       cd2* yt[kTab];
 #pragma unroll
       for (int k2 = 0; k2 < kTab; ++k2) yt[k2] = bp(bufs, B_YT0 + k2) + off;
       if (op.i == 0) {
-        for (int e = threadIdx.x; e < N; e += TB) {
+        for (int e = threadIdx.x; e < N; e += TV) {
           const cd2 v = yest[e];
           ysav[e] = v;
           dy[e] = v;
@@ -224,54 +305,36 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
         }
         break;
       }
-      // two elements per pass: both tableau columns are loaded before any
-      // store, and the two extrapolation chains are independent
-      for (int e0 = threadIdx.x; e0 < N; e0 += 2 * TB) {
-        const int e1 = e0 + TB;
-        const bool has1 = e1 < N;
-        const int ee[2] = {e0, has1 ? e1 : e0};
-        cd2 col[2][kTab], yy[2], v[2];
+      // every tableau column of the element is loaded before any store
+      for (int e = threadIdx.x; e < N; e += TV) {
+        cd2 col[kTab], v = yt0[e];
+        const cd2 yst = yest[e];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-          for (int k2 = 1; k2 < kTab; ++k2) col[h][k2] = yt[k2 < mi ? k2 : 0][ee[h]];
-          yy[h] = yest[ee[h]];
-          v[h] = yt0[ee[h]];
-        }
-        const cd2 yst[2] = {yy[0], yy[1]};
-        cd2 ddy[2] = {czero<double>(), czero<double>()}, c[2] = {yy[0], yy[1]};
+        for (int k2 = 1; k2 < kTab; ++k2) col[k2] = yt[k2 < mi ? k2 : 0][e];
+        cd2 ddy = czero<double>(), c = yst, yy = yst;
 #pragma unroll
         for (int k2 = 1; k2 < kTab; ++k2) {
           if (k2 < mi) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const cd2 bi = mk<double>(fx[k2] * v[h].re, fx[k2] * v[h].im);
-              cd2 b = mk<double>(bi.re - c[h].re, bi.im - c[h].im);
-              if (b.re != 0.0 || b.im != 0.0) {
-                b = cdiv(mk<double>(c[h].re - v[h].re, c[h].im - v[h].im), b);
-                ddy[h] = cmul(c[h], b);
-                c[h] = cmul(bi, b);
-              } else {
-                ddy[h] = v[h];
-              }
-              v[h] = col[h][k2];
-              col[h][k2] = ddy[h];
-              yy[h] = mk<double>(yy[h].re + ddy[h].re, yy[h].im + ddy[h].im);
+            const cd2 bi = mk<double>(fx[k2] * v.re, fx[k2] * v.im);
+            cd2 b = mk<double>(bi.re - c.re, bi.im - c.im);
+            if (b.re != 0.0 || b.im != 0.0) {
+              b = cdiv(mk<double>(c.re - v.re, c.im - v.im), b);
+              ddy = cmul(c, b);
+              c = cmul(bi, b);
+            } else {
+              ddy = v;
             }
+            v = col[k2];
+            col[k2] = ddy;
+            yy = mk<double>(yy.re + ddy.re, yy.im + ddy.im);
           }
         }
+        yt0[e] = yst;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (h == 0 || has1) {
-            const int e = ee[h];
-            yt0[e] = yst[h];
-#pragma unroll
-            for (int k2 = 1; k2 < kTab; ++k2)
-              if (k2 < mi) yt[k2][e] = col[h][k2];
-            dy[e] = ddy[h];
-            ysav[e] = yy[h];
-          }
-        }
+        for (int k2 = 1; k2 < kTab; ++k2)
+          if (k2 < mi) yt[k2][e] = col[k2];
+        dy[e] = ddy;
+        ysav[e] = yy;
       }
       break;
     }
@@ -286,14 +349,18 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
       elementwise(N, so);
       break;
     }
-    case V_MMID_BEGIN:
-      elementwise(N, MmidBeginOp{bp(bufs, B_Y0) + off, bp(bufs, B_Y0 + 1) + off, bp(bufs, B_X) + off,
-                                 bp(bufs, B_Y0 + 3) + off, bp(bufs, B_Y0 + 4) + off, op.h});
+    case V_MMID_BEGIN: {
+      cd2 *y1 = bp(bufs, B_Y0 + 1) + off, *x = bp(bufs, B_X) + off;
+      elementwise(N, MmidBeginOp{bp(bufs, B_Y0) + off, y1, x == y1 ? nullptr : x, bp(bufs, B_Y0 + 3) + off,
+                                 bp(bufs, B_Y0 + 4) + off, op.h});
       break;
-    case V_MMID_STEP_X:
-      elementwise(N, MmidStepXOp{bp(bufs, B_Y0) + off, bp(bufs, B_Y0 + 1) + off, bp(bufs, B_Y0 + 2) + off,
-                                 bp(bufs, B_X) + off, op.h});
+    }
+    case V_MMID_STEP_X: {
+      cd2 *y1 = bp(bufs, B_Y0 + 1) + off, *y2 = bp(bufs, B_Y0 + 2) + off, *x = bp(bufs, B_X) + off;
+      elementwise(N, MmidStepXOp{bp(bufs, B_Y0) + off, y1, y2, y2 == bp(bufs, B_D) + off ? nullptr : y2,
+                                 x == y1 ? nullptr : x, op.h});
       break;
+    }
     case V_FINAL_EXTR: {
       // y2 <- d; y0 <- (y0 + y1 + h y2) / 2 (the midpoint estimate yest);
       // rzextr at step i; then y0 <- ysav, y1 <- ysav + dy
@@ -306,11 +373,11 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
       const double h = op.h;
       double fx[kTab];
 #pragma unroll
-      for (int k2 = 1; k2 < kTab; ++k2) fx[k2] = opp->fx[k2];
+      for (int k2 = 1; k2 < kTab; ++k2) fx[k2] = uniform(opp->fx[k2]);
       cd2* yt[kTab];
 #pragma unroll
       for (int k2 = 0; k2 < kTab; ++k2) yt[k2] = bp(bufs, B_YT0 + k2) + off;
-      for (int e = threadIdx.x; e < N; e += TB) {
+      for (int e = threadIdx.x; e < N; e += TV) {
         const cd2 d = dd[e], a = y0[e], b = y1[e];
         cd2 col[kTab], v = czero<double>();
         if (op.i > 0) {
@@ -347,8 +414,10 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
         }
         yt[0][e] = yest;
         y2[e] = dy;
+        const cd2 ye = mk<double>(ysav.re + dy.re, ysav.im + dy.im);
         y0[e] = ysav;
-        y1[e] = mk<double>(ysav.re + dy.re, ysav.im + dy.im);
+        y1[e] = ye;
+        if (kTick && el.diff) el.diff[e] = mk<double>(ysav.re - ye.re, ysav.im - ye.im);
       }
       break;
     }
@@ -359,7 +428,7 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
       const int64_t rs = rhoslot[node];
       double delta = 0.0, nrm = 0.0;
       if (rs < 0) {
-        for (int e = threadIdx.x; e < N; e += TB) {
+        for (int e = threadIdx.x; e < N; e += TV) {
           const double dr = Phi[e].re - Chi[e].re, di = Phi[e].im - Chi[e].im;
           delta += dr * dr + di * di;
           nrm += Phi[e].re * Phi[e].re + Phi[e].im * Phi[e].im;
@@ -370,35 +439,24 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
         const cd2* rho = pool + rs;
         // Delta = sum_{i,n,m} Re( conj(d(i,n)) rho(n,m) d(i,m) )
         if (n <= 16) {
-          // a thread per row i: d(i, :) in registers, rho in LDS
-          for (int o = threadIdx.x; o < n * n; o += TB) rhos[o] = rho[o];
-          __syncthreads();
-          for (int i = threadIdx.x; i < L; i += TB) {
-            cd2 d[16];
-#pragma unroll
-            for (int m = 0; m < 16; ++m) {
-              const int mm = m < n ? m : 0;
-              const cd2 p = Phi[i + mm * L], q = Chi[i + mm * L];
-              d[m] = mk<double>(p.re - q.re, p.im - q.im);
-            }
-#pragma unroll
-            for (int nn = 0; nn < 16; ++nn) {
-              if (nn < n) {
-                double tr = 0.0, ti = 0.0;
-#pragma unroll
-                for (int m = 0; m < 16; ++m) {
-                  if (m < n) {
-                    const cd2 r = rhos[nn + m * n];
-                    tr += r.re * d[m].re - r.im * d[m].im;
-                    ti += r.re * d[m].im + r.im * d[m].re;
-                  }
-                }
-                delta += d[nn].re * tr + d[nn].im * ti;
-              }
-            }
+          if (kTick) {
+            if ((int)threadIdx.x < n * n) rhos[threadIdx.x] = el.rho;
+          } else {
+            for (int o = threadIdx.x; o < n * n; o += TV) rhos[o] = rho[o];
+          }
+          lds_barrier();
+          if (kTick && el.diff) {
+            delta = rho_norm([&](int o) { return el.diff[o]; }, rhos, n, L);
+          } else {
+            delta = rho_norm(
+                [&](int o) {
+                  const cd2 p = Phi[o], q = Chi[o];
+                  return mk<double>(p.re - q.re, p.im - q.im);
+                },
+                rhos, n, L);
           }
         } else {
-          for (int e = threadIdx.x; e < N; e += TB) {
+          for (int e = threadIdx.x; e < N; e += TV) {
             const int i = e % L, nn = e / L;
             const double dr = Phi[e].re - Chi[e].re, di = Phi[e].im - Chi[e].im;
             double tr = 0.0, ti = 0.0;
@@ -414,13 +472,19 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
         }
         delta = block_sum_d(delta, red);
         double t = 0.0, tim = 0.0;
+        const cd2* rd = n <= 16 ? rhos : rho;
+#pragma unroll 4
         for (int m = 0; m < n; ++m) {
-          t += rho[m + m * n].re;
-          tim += rho[m + m * n].im;
+          t += rd[m + m * n].re;
+          tim += rd[m + m * n].im;
         }
         nrm = sqrt(t * t + tim * tim);
       }
-      if (threadIdx.x == 0) err[node] = sqrt(fabs(delta / nrm));
+      if (threadIdx.x == 0) {
+        const double e = sqrt(fabs(delta / nrm));
+        err[node] = e;
+        if (kTick) *el.out = e;
+      }
       break;
     }
     default:
@@ -428,11 +492,11 @@ __device__ __forceinline__ void exec_op(const VecOp* opp, const CmfBufs& bufs, c
   }
 }
 
-__global__ void __launch_bounds__(TB)
+__global__ void __launch_bounds__(TV)
     program_kernel(const NodeProg* __restrict__ progs, const VecOp* __restrict__ ops, CmfBufs bufs,
                    const DNode* __restrict__ nodes, const cd2* __restrict__ pool, const int64_t* __restrict__ rhoslot,
                    double* err, uint8_t* mask) {
-  __shared__ double red[TB];
+  __shared__ double red[TV / 64];
   __shared__ cd2 rhos[16 * 16];
   const NodeProg pg = progs[blockIdx.x];
   int op0 = pg.op0, op1 = pg.op1;
@@ -451,10 +515,12 @@ __global__ void __launch_bounds__(TB)
   if (op0 >= op1) return;  // an empty program (the whole workgroup)
   const DNode nd = nodes[pg.node];
   for (int k = op0; k < op1; ++k) {
-    exec_op(&ops[k], bufs, nodes, pool, rhoslot, err, pg.node, nd, red, rhos);
+    exec_op<false>(&ops[k], bufs, nodes, pool, rhoslot, err, pg.node, nd, red, rhos, ErrLocal{});
     __syncthreads();
   }
 }
+
+constexpr int OW = 8, OT = 64 * OW;  // wavefronts and threads of orthogonal()
 
 // The transposed square root SW(j,k) = S^(1/2)(k,j) of a near-identity
 // S = Phi^H Phi (n <= 16, rho = n max|S - I| < 1/2: the node tensors after
@@ -462,15 +528,16 @@ __global__ void __launch_bounds__(TB)
 // Newton-Schulz iteration T = (3I - Z Y) / 2, Y <- Y T, Z <- T Z from
 // Y = S, Z = I (Y -> S^(1/2), Z -> S^(-1/2), quadratically: the error is
 // below 1e-17 after the steps chosen).  It is the principal square root the
-// eigendecomposition gives, to rounding.  One wavefront; returns false (and
-// writes nothing) when S is not near enough the identity.
+// eigendecomposition gives, to rounding.  By OT threads; returns false (and
+// writes nothing) when S is not near enough the identity, the same in every
+// thread.
 __device__ bool ortho_sqrt_ns(const cd2* A, int ld, int n, cd2* sw) {
   __shared__ cd2 nsb[5][256];
   static_assert(sizeof(nsb) == kOrthoNsElems * sizeof(cd2), "Newton-Schulz buffers");
   if (n > 16) return false;
   const int nn = n * n;
   double e = 0.0;
-  for (int o = threadIdx.x; o < nn; o += EW) {
+  for (int o = threadIdx.x & 63; o < nn; o += 64) {  // every wavefront the whole of it
     const int i = o % n, j = o / n;
     const cd2 v = A[i + j * ld];
     e = fmax(e, fabs((i == j ? 1.0 : 0.0) - v.re) + fabs(v.im));
@@ -481,29 +548,26 @@ __device__ bool ortho_sqrt_ns(const cd2* A, int ld, int n, cd2* sw) {
   int nsk = 1;  // one step beyond the estimate
   for (double r = rho; r > 1e-17 && nsk < 9; r *= r) ++nsk;
   cd2 *Y = nsb[0], *Z = nsb[1], *T = nsb[2], *Yn = nsb[3], *Zn = nsb[4];
-  for (int o = threadIdx.x; o < nn; o += EW) {
+  for (int o = threadIdx.x; o < nn; o += OT) {
     const int i = o % n, j = o / n;
     Y[o] = A[i + j * ld];
     Z[o] = mk<double>(i == j ? 1.0 : 0.0, 0.0);
   }
   __syncthreads();
   for (int k = 0; k < nsk; ++k) {
-    for (int o = threadIdx.x; o < nn; o += EW) {
+    for (int o = threadIdx.x; o < nn; o += OT) {
       const int i = o % n, j = o / n;
       cd2 acc = czero<double>();
       for (int l = 0; l < n; ++l) cfma(acc, Z[i + l * n], Y[l + j * n]);
       T[o] = mk<double>(0.5 * ((i == j ? 3.0 : 0.0) - acc.re), -0.5 * acc.im);
     }
     __syncthreads();
-    for (int o = threadIdx.x; o < nn; o += EW) {
-      const int i = o % n, j = o / n;
-      cd2 y = czero<double>(), z = czero<double>();
-      for (int l = 0; l < n; ++l) {
-        cfma(y, Y[i + l * n], T[l + j * n]);
-        cfma(z, T[i + l * n], Z[l + j * n]);
-      }
-      Yn[o] = y;
-      Zn[o] = z;
+    for (int o2 = threadIdx.x; o2 < 2 * nn; o2 += OT) {  // Y T, then T Z
+      const int o = o2 < nn ? o2 : o2 - nn, i = o % n, j = o / n;
+      const cd2 *l0 = o2 < nn ? Y : T, *r0 = o2 < nn ? T : Z;
+      cd2 acc = czero<double>();
+      for (int l = 0; l < n; ++l) cfma(acc, l0[i + l * n], r0[l + j * n]);
+      (o2 < nn ? Yn : Zn)[o] = acc;
     }
     __syncthreads();
     cd2* t = Y;
@@ -513,179 +577,133 @@ __device__ bool ortho_sqrt_ns(const cd2* A, int ld, int n, cd2* sw) {
     Z = Zn;
     Zn = t;
   }
-  for (int o = threadIdx.x; o < nn; o += EW) {
+  for (int o = threadIdx.x; o < nn; o += OT) {
     const int j = o % n, k = o / n;
     sw[j + k * n] = Y[k + j * n];
   }
   return true;
 }
 
+// sum_i conj(a_i) b_i of two columns by one wavefront
+__device__ __forceinline__ cd2 column_overlap(const cd2* a, const cd2* b, int L, int lane) {
+  double re = 0.0, im = 0.0;
+  for (int i = lane; i < L; i += 64) {
+    re += a[i].re * b[i].re + a[i].im * b[i].im;
+    im += a[i].re * b[i].im - a[i].im * b[i].re;
+  }
+  return mk<double>(wave_total(re), wave_total(im));
+}
+
 // ------------------------------------------------------------- orthogonal()
 // S = Phi^H Phi, SW(j,k) = sum_l U(k,l) sqrt(max(l_l,0)) conj(U(j,l)) (the
 // transposed square root), then iterated Gram-Schmidt of Phi in place
-// (Tensor_Implementation.h:806-853).  One wavefront per node.  Items with
-// sw < 0 take the Gram-Schmidt only (orthonormal(),
-// TensorTree_Implementation.h:190-195).
-__global__ void __launch_bounds__(EW)
+// (Tensor_Implementation.h:806-853).  One workgroup per node; Phi is staged in
+// LDS (kLds), or read and written in place for node tensors that LDS does not
+// hold (which take the eigendecomposition always).  Items with sw < 0 take the
+// Gram-Schmidt only (orthonormal(), TensorTree_Implementation.h:190-195).
+//
+// Bound by the chain of the n columns' dependent reductions.  A wavefront
+// takes every OW-th overlap of column k with those before it (all against the
+// same column: classical, iterated until they vanish as the reference does),
+// a thread the rows i, i + OT, ... of the update.  One wavefront alone, an
+// overlap and an update after the other, took 246 us for 196 x 16 columns; this
+// form takes 75 us (16 wavefronts 72, but 29 to 34 instead of 28 for 100 x 11).
+template <bool kLds>
+__global__ void __launch_bounds__(OT)
     ortho_kernel(const OrthoItem* __restrict__ items, const DNode* __restrict__ nodes, cd2* P, cd2* sw,
                  int nmax, int nspf) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  cd2* Phi = reinterpret_cast<cd2*>(smem_raw);
-  cd2* A = Phi + nmax;
+  cd2* A = reinterpret_cast<cd2*>(smem_raw) + (kLds ? nmax : 0);
   cd2* U = A + jacobi_elems(nspf);
   __shared__ JacobiScratch js;
-  __shared__ double lam[64];
+  __shared__ double lam[64], oab[64], red[OW];
+  __shared__ cd2 ovl[64];
   const OrthoItem it = items[blockIdx.x];
   const DNode nd = nodes[it.node];
   const int N = nd.N, n = nodes[it.node].dims[nd.order - 1], L = N / n, ld = jacobi_ld(n);
-  stage_to_lds<EW>(Phi, P + nd.off, N);
-  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  cd2* Phi = kLds ? reinterpret_cast<cd2*>(smem_raw) : P + nd.off;
+  if (kLds) {
+    stage_to_lds<OT>(Phi, P + nd.off, N);
+    __syncthreads();
+  }
   if (it.sw >= 0) {  // uniform per workgroup
-    for (int o = threadIdx.x; o < n * n; o += EW) {
-      const int j = o % n, k = o / n;
-      cd2 acc = czero<double>();
-      for (int i = 0; i < L; ++i) cfmac(acc, Phi[i + j * L], Phi[i + k * L]);
-      A[j + k * ld] = acc;
-    }
-    __syncthreads();
-    if (ortho_sqrt_ns(A, ld, n, sw + it.sw)) goto gram_schmidt;
-    jacobi_eig(A, U, n, ld, js);
-    for (int i = threadIdx.x; i < n; i += EW) lam[i] = sqrt(fmax(A[i + i * ld].re, 0.0));
-    __syncthreads();
-    for (int o = threadIdx.x; o < n * n; o += EW) {
-      const int j = o % n, k = o / n;
-      cd2 acc = czero<double>();
-      for (int l = 0; l < n; ++l) {
-        const cd2 ukl = U[k + l * ld], ujl = U[j + l * ld];
-        // U(k,l) * s_l * conj(U(j,l))
-        acc.re += lam[l] * (ukl.re * ujl.re + ukl.im * ujl.im);
-        acc.im += lam[l] * (ukl.im * ujl.re - ukl.re * ujl.im);
-      }
-      sw[it.sw + j + k * n] = acc;
-    }
-  }
-gram_schmidt:
-  // Gram-Schmidt: lane owns rows i = lane + 64 t, so every reduction is a
-  // wavefront shuffle sum and no other lane touches its elements.
-  for (int k = 0; k < n; ++k) {
-    double accum = 1.0;
-    for (int iter = 0; iter < 15 && accum > 1e-12; ++iter) {
-      accum = 0.0;
-      for (int m = 0; m < k; ++m) {
-        double ore = 0.0, oim = 0.0;
-        for (int i = threadIdx.x; i < L; i += EW) {
-          const cd2 a = Phi[i + m * L], b = Phi[i + k * L];
-          ore += a.re * b.re + a.im * b.im;
-          oim += a.re * b.im - a.im * b.re;
-        }
-        ore = wave_sum(ore);
-        oim = wave_sum(oim);
-        accum += sqrt(ore * ore + oim * oim);
-        for (int i = threadIdx.x; i < L; i += EW) {
-          const cd2 a = Phi[i + m * L];
-          cd2& b = Phi[i + k * L];
-          b.re -= ore * a.re - oim * a.im;
-          b.im -= ore * a.im + oim * a.re;
-        }
-      }
-      double nr = 0.0;
-      for (int i = threadIdx.x; i < L; i += EW) nr += Phi[i + k * L].re * Phi[i + k * L].re + Phi[i + k * L].im * Phi[i + k * L].im;
-      nr = wave_sum(nr);
-      if (nr != 0.0) {
-        const double s = sqrt(nr);
-        for (int i = threadIdx.x; i < L; i += EW) {
-          Phi[i + k * L].re /= s;
-          Phi[i + k * L].im /= s;
-        }
-      }
-    }
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < N; e += EW) P[nd.off + e] = Phi[e];
-}
-
-// orthogonal() for node tensors too large for LDS: the algorithm of
-// ortho_kernel with Phi read and written in place in global memory (only the
-// n x n Jacobi buffers in LDS).  One wavefront per node; a lane owns rows
-// i = lane + 64 t, so the Gram-Schmidt reductions are shuffle sums.
-__global__ void __launch_bounds__(EW)
-    ortho_global_kernel(const OrthoItem* __restrict__ items, const DNode* __restrict__ nodes, cd2* P, cd2* sw,
-                        int nspf) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  cd2* A = reinterpret_cast<cd2*>(smem_raw);
-  cd2* U = A + jacobi_elems(nspf);
-  __shared__ JacobiScratch js;
-  __shared__ double lam[64];
-  const OrthoItem it = items[blockIdx.x];
-  const DNode nd = nodes[it.node];
-  const int N = nd.N, n = nd.dims[nd.order - 1], L = N / n, ld = jacobi_ld(n);
-  cd2* Phi = P + nd.off;
-  if (it.sw >= 0) {
-    // S(j,k) = sum_i conj(Phi(i,j)) Phi(i,k): lanes split the rows, every
-    // entry is a shuffle sum (coalesced column reads)
     for (int j = 0; j < n; ++j)
-      for (int k = 0; k < n; ++k) {
-        double re = 0.0, im = 0.0;
-        for (int i = threadIdx.x; i < L; i += EW) {
-          const cd2 a = Phi[i + j * L], b = Phi[i + k * L];
-          re += a.re * b.re + a.im * b.im;
-          im += a.re * b.im - a.im * b.re;
+      for (int k = j + wave; k < n; k += OW) {
+        const cd2 v = column_overlap(Phi + j * L, Phi + k * L, L, lane);
+        if (lane == 0) {
+          A[j + k * ld] = v;
+          if (j != k) A[k + j * ld] = cconj(v);
         }
-        re = wave_sum(re);
-        im = wave_sum(im);
-        if (threadIdx.x == 0) A[j + k * ld] = mk<double>(re, im);
       }
     __syncthreads();
-    jacobi_eig(A, U, n, ld, js);
-    for (int i = threadIdx.x; i < n; i += EW) lam[i] = sqrt(fmax(A[i + i * ld].re, 0.0));
-    __syncthreads();
-    for (int o = threadIdx.x; o < n * n; o += EW) {
-      const int j = o % n, k = o / n;
-      cd2 acc = czero<double>();
-      for (int l = 0; l < n; ++l) {
-        const cd2 ukl = U[k + l * ld], ujl = U[j + l * ld];
-        acc.re += lam[l] * (ukl.re * ujl.re + ukl.im * ujl.im);
-        acc.im += lam[l] * (ukl.im * ujl.re - ukl.re * ujl.im);
+    bool done = false;
+    if constexpr (kLds) done = ortho_sqrt_ns(A, ld, n, sw + it.sw);
+    if (!done) {
+      if (wave == 0) {
+        jacobi_eig(A, U, n, ld, js);
+        for (int i = lane; i < n; i += EW) lam[i] = sqrt(fmax(A[i + i * ld].re, 0.0));
       }
-      sw[it.sw + j + k * n] = acc;
+      __syncthreads();
+      for (int o = threadIdx.x; o < n * n; o += OT) {
+        const int j = o % n, k = o / n;
+        cd2 acc = czero<double>();
+        for (int l = 0; l < n; ++l) {
+          const cd2 ukl = U[k + l * ld], ujl = U[j + l * ld];
+          // U(k,l) * s_l * conj(U(j,l))
+          acc.re += lam[l] * (ukl.re * ujl.re + ukl.im * ujl.im);
+          acc.im += lam[l] * (ukl.im * ujl.re - ukl.re * ujl.im);
+        }
+        sw[it.sw + j + k * n] = acc;
+      }
     }
   }
   for (int k = 0; k < n; ++k) {
+    cd2* Ck = Phi + k * L;
     double accum = 1.0;
-    for (int iter = 0; iter < 15 && accum > 1e-12; ++iter) {
-      accum = 0.0;
-      for (int m = 0; m < k; ++m) {
-        double ore = 0.0, oim = 0.0;
-        for (int i = threadIdx.x; i < L; i += EW) {
-          const cd2 a = Phi[i + m * L], b = Phi[i + k * L];
-          ore += a.re * b.re + a.im * b.im;
-          oim += a.re * b.im - a.im * b.re;
-        }
-        ore = wave_sum(ore);
-        oim = wave_sum(oim);
-        accum += sqrt(ore * ore + oim * oim);
-        for (int i = threadIdx.x; i < L; i += EW) {
-          const cd2 a = Phi[i + m * L];
-          cd2 b = Phi[i + k * L];
-          b.re -= ore * a.re - oim * a.im;
-          b.im -= ore * a.im + oim * a.re;
-          Phi[i + k * L] = b;
+    for (int iter = 0; iter < 15 && accum > 1e-12; ++iter) {  // accum is the same in every thread
+      for (int m = wave; m < k; m += OW) {
+        const cd2 v = column_overlap(Phi + m * L, Ck, L, lane);
+        if (lane == 0) {
+          ovl[m] = v;
+          oab[m] = sqrt(v.re * v.re + v.im * v.im);
         }
       }
+      __syncthreads();
+      accum = 0.0;
+      for (int m = 0; m < k; ++m) accum += oab[m];
       double nr = 0.0;
-      for (int i = threadIdx.x; i < L; i += EW) nr += Phi[i + k * L].re * Phi[i + k * L].re + Phi[i + k * L].im * Phi[i + k * L].im;
-      nr = wave_sum(nr);
+      for (int i = threadIdx.x; i < L; i += OT) {
+        cd2 b = Ck[i];
+#pragma unroll 4
+        for (int m = 0; m < k; ++m) {
+          const cd2 o = ovl[m], a = Phi[i + m * L];
+          b.re -= o.re * a.re - o.im * a.im;
+          b.im -= o.re * a.im + o.im * a.re;
+        }
+        Ck[i] = b;
+        nr += b.re * b.re + b.im * b.im;
+      }
+      nr = wave_total(nr);
+      if (lane == 0) red[wave] = nr;
+      __syncthreads();
+      nr = 0.0;
+#pragma unroll
+      for (int w = 0; w < OW; ++w) nr += red[w];
       if (nr != 0.0) {
         const double s = sqrt(nr);
-        for (int i = threadIdx.x; i < L; i += EW) {
-          cd2 b = Phi[i + k * L];
+        for (int i = threadIdx.x; i < L; i += OT) {
+          cd2 b = Ck[i];
           b.re /= s;
           b.im /= s;
-          Phi[i + k * L] = b;
+          Ck[i] = b;
         }
       }
+      __syncthreads();
     }
   }
+  if (kLds)
+    for (int e = threadIdx.x; e < N; e += OT) P[nd.off + e] = Phi[e];
 }
 
 // ------------------------------------------------------ top eigenproblems
@@ -739,27 +757,31 @@ __global__ void __launch_bounds__(EW)
 }
 
 // parent <- SW_c x_{childIdx(c)} parent for its children, in node-address order
-__global__ void __launch_bounds__(TB)
-    apply_sw_kernel(const SwApply* __restrict__ items, const DNode* __restrict__ nodes, cd2* P, const cd2* sw,
+// (NT threads, 1024 for node tensors of at least 1024 elements)
+template <int NT>
+__global__ void __launch_bounds__(NT)
+    apply_sw_kernel(const SwApply* __restrict__ items, const DNode* __restrict__ nodes, cd2* __restrict__ P,
+                    const cd2* __restrict__ sw,
                     int nmax) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cd2* b0 = reinterpret_cast<cd2*>(smem_raw);
   cd2* b1 = b0 + nmax;
-  const SwApply it = items[blockIdx.x];
-  const DNode nd = nodes[it.node];
+  // by reference: the entries indexed at run time stay out of scratch
+  const SwApply& it = items[blockIdx.x];
+  const DNode& nd = nodes[it.node];
   const int N = nd.N;
-  stage_to_lds<TB>(b0, P + nd.off, N);
+  stage_to_lds<NT>(b0, P + nd.off, N);
   __syncthreads();
   cd2* cur = b0;
   cd2* nxt = b1;
   for (int f = 0; f < it.nf; ++f) {
-    mode_apply<double>(nxt, cur, sw + it.fmat[f], nd, it.fmode[f]);
+    mode_apply<NT, double>(nxt, cur, sw + it.fmat[f], nd, it.fmode[f]);
     __syncthreads();
     cd2* t = cur;
     cur = nxt;
     nxt = t;
   }
-  for (int e = threadIdx.x; e < N; e += TB) P[nd.off + e] = cur[e];
+  for (int e = threadIdx.x; e < N; e += NT) P[nd.off + e] = cur[e];
 }
 
 // ------------------------------------------------- device BS integrators
@@ -876,30 +898,43 @@ __device__ bool bs_advance(BsRegs& b, const double* xin, double* xtab, double e,
 }
 }  // namespace
 
-__global__ void __launch_bounds__(TB)
+__global__ void __launch_bounds__(TV)
     bs_tick_kernel(BsNode* __restrict__ st, CmfBufs bufs, const DNode* __restrict__ nodes,
                    const cd2* __restrict__ pool, const int64_t* __restrict__ rhoslot, double* err, uint8_t* rec,
-                   int init, double t0, double t1, double eps) {
-  __shared__ double red[TB];
+                   int init, double t0, double t1, double eps, int dcap) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ double red[TV / 64];
   __shared__ cd2 rhos[16 * 16];
   __shared__ VecOp pre;
   __shared__ int npre;
-  // the node's state up to its post ops, read once for the workgroup (one
-  // round trip, before thread 0 can rewrite it)
-  __shared__ double head[kBsHeadWords];
+  // the node's state with its post ops, read once for the workgroup.  Thread
+  // 0 makes the next state in LDS, and the workgroup writes it, with the
+  // record, after the last op: a store before the barrier would be waited
+  // for there.
+  constexpr int kWords = sizeof(BsNode) / 8;
+  __shared__ double head[kWords], next[kWords];
+  __shared__ double errl;
+  __shared__ uint8_t recl[2];
   const int v = blockIdx.x;
   BsNode* b = st + v;
   const DNode nd = nodes[v];
-  if (threadIdx.x < kBsHeadWords) head[threadIdx.x] = reinterpret_cast<const double*>(b)[threadIdx.x];
+  if (threadIdx.x < kWords) head[threadIdx.x] = next[threadIdx.x] = reinterpret_cast<const double*>(b)[threadIdx.x];
   __syncthreads();
   const BsNode& hd = *reinterpret_cast<const BsNode*>(head);
   const int np = init ? 0 : hd.npost;
+  ErrLocal el{nullptr, czero<double>(), &errl};
+  if (np == 2) {  // the final op and the error
+    const int64_t rs = rhoslot[v];
+    const int n = nodes[v].dims[nd.order - 1];
+    if (nd.N <= dcap && (rs < 0 || n <= 16)) el.diff = reinterpret_cast<cd2*>(smem_raw);
+    if (rs >= 0 && n <= 16 && (int)threadIdx.x < n * n) el.rho = pool[rs + threadIdx.x];
+  }
   // the post ops of the tick that ran, then (k == np) the decisions and the
   // next tick's pre op: one call site of the op code
   for (int k = 0; k <= np; ++k) {
     const VecOp* opp = &pre;
     if (k < np) {
-      opp = &b->post[k];
+      opp = &hd.post[k];
     } else {
       if (threadIdx.x == 0) {
         BsRegs r{hd.st, hd.i, hd.step, hd.nsub, hd.x, hd.xend, hd.h, hd.hh, hd.dt};
@@ -908,43 +943,57 @@ __global__ void __launch_bounds__(TB)
           r.x = t0;
           r.xend = t1;
         }
-        // the node error the post ops just wrote (this thread wrote it)
-        const double e = (r.st == BS_AWAIT_ERR) ? err[v] : 0.0;
+        // the node error of the post ops above (a node awaits it only in the
+        // tick that has it among them)
+        const double e = (r.st == BS_AWAIT_ERR) ? errl : 0.0;
+        BsNode& nx = *reinterpret_cast<BsNode*>(next);
         int nq = 0, lead = 0, n1 = 0;
         bool fail = false;
-        const bool active = bs_advance(r, hd.xtab, b->xtab, e, eps, bufs, &pre, n1, b->post, nq, fail, lead);
-        b->st = r.st;
-        b->i = r.i;
-        b->step = r.step;
-        b->nsub = r.nsub;
-        b->x = r.x;
-        b->xend = r.xend;
-        b->h = r.h;
-        b->hh = r.hh;
-        b->dt = r.dt;
-        b->npost = nq;
+        const bool active = bs_advance(r, hd.xtab, nx.xtab, e, eps, bufs, &pre, n1, nx.post, nq, fail, lead);
+        nx.st = r.st;
+        nx.i = r.i;
+        nx.step = r.step;
+        nx.nsub = r.nsub;
+        nx.x = r.x;
+        nx.xend = r.xend;
+        nx.h = r.h;
+        nx.hh = r.hh;
+        nx.dt = r.dt;
+        nx.npost = nq;
         const bool failed = fail || hd.fail;
-        if (fail) b->fail = 1;
-        if (active) b->nderiv = hd.nderiv + 1;
+        if (fail) nx.fail = 1;
+        if (active) nx.nderiv = hd.nderiv + 1;
         npre = n1;
-        rec[v] = active ? 1 : 0;
-        rec[gridDim.x + v] = failed ? kBsFailed : (uint8_t)(lead < 254 ? lead : 254);
+        recl[0] = active ? 1 : 0;
+        recl[1] = failed ? kBsFailed : (uint8_t)(lead < 254 ? lead : 254);
       }
       __syncthreads();
       if (!npre) break;
     }
-    exec_op(opp, bufs, nodes, pool, rhoslot, err, v, nd, red, rhos);
-    __syncthreads();
+    exec_op<true>(opp, bufs, nodes, pool, rhoslot, err, v, nd, red, rhos, el);
+    if (k < np) {
+      // the error op reads the final op's results from LDS, where that holds
+      // them, and a thread's own elements; the ops that follow the error read
+      // their own elements
+      if (el.diff) lds_barrier();
+      else __syncthreads();
+    }
+  }
+  if (threadIdx.x < kWords) reinterpret_cast<double*>(b)[threadIdx.x] = next[threadIdx.x];
+  if (threadIdx.x == 0) {
+    rec[v] = recl[0];
+    rec[gridDim.x + v] = recl[1];
   }
 }
 
 int launch_bs_tick(BsNode* st, int64_t count, const CmfBufs& bufs, const DNode* nodes, const cplx<double>* pool,
                    const int64_t* rhoslot, double* err, uint8_t* rec, int init, double t0, double t1, double eps,
-                   hipStream_t s) {
-  static_assert(offsetof(BsNode, post) == 8 * kBsHeadWords, "BsNode head");
+                   int nmax, hipStream_t s) {
+  static_assert(sizeof(BsNode) % 8 == 0 && sizeof(BsNode) / 8 <= TV, "BsNode is read a word a thread");
   if (count == 0) return QTG_OK;
-  hipLaunchKernelGGL(bs_tick_kernel, dim3((unsigned)count), dim3(TB), 0, s, st, bufs, nodes, pool, rhoslot, err, rec,
-                     init, t0, t1, eps);
+  const int dcap = nmax < 8192 ? nmax : 8192;  // 128 KB
+  hipLaunchKernelGGL(bs_tick_kernel, dim3((unsigned)count), dim3(TV), dcap * sizeof(cd2), s, st, bufs, nodes, pool,
+                     rhoslot, err, rec, init, t0, t1, eps, dcap);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }
@@ -953,7 +1002,7 @@ int launch_programs(const NodeProg* progs, int64_t count, const VecOp* ops, cons
                     const DNode* nodes, const cplx<double>* pool, const int64_t* rhoslot, double* err,
                     hipStream_t s, uint8_t* mask) {
   if (count == 0) return QTG_OK;
-  hipLaunchKernelGGL(program_kernel, dim3((unsigned)count), dim3(TB), 0, s, progs, ops, bufs, nodes, pool, rhoslot,
+  hipLaunchKernelGGL(program_kernel, dim3((unsigned)count), dim3(TV), 0, s, progs, ops, bufs, nodes, pool, rhoslot,
                      err, mask);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
@@ -963,7 +1012,7 @@ int launch_ortho(const OrthoItem* items, int64_t count, const DNode* nodes, cplx
                  int nmax, int nspf, hipStream_t s) {
   if (count == 0) return QTG_OK;
   const size_t lds = ((size_t)nmax + 2 * (size_t)jacobi_elems(nspf)) * sizeof(cd2);
-  hipLaunchKernelGGL(ortho_kernel, dim3((unsigned)count), dim3(EW), lds, s, items, nodes, P, sw, nmax, nspf);
+  hipLaunchKernelGGL(ortho_kernel<true>, dim3((unsigned)count), dim3(OT), lds, s, items, nodes, P, sw, nmax, nspf);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }
@@ -972,7 +1021,7 @@ int launch_ortho_global(const OrthoItem* items, int64_t count, const DNode* node
                         cplx<double>* sw, int nspf, hipStream_t s) {
   if (count == 0) return QTG_OK;
   const size_t lds = 2 * (size_t)jacobi_elems(nspf) * sizeof(cd2);
-  hipLaunchKernelGGL(ortho_global_kernel, dim3((unsigned)count), dim3(EW), lds, s, items, nodes, P, sw, nspf);
+  hipLaunchKernelGGL(ortho_kernel<false>, dim3((unsigned)count), dim3(OT), lds, s, items, nodes, P, sw, 0, nspf);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }
@@ -992,7 +1041,10 @@ int launch_apply_sw(const SwApply* items, int64_t count, const DNode* nodes, cpl
                     const cplx<double>* sw, int nmax, hipStream_t s) {
   if (count == 0) return QTG_OK;
   const size_t lds = 2 * (size_t)nmax * sizeof(cd2);
-  hipLaunchKernelGGL(apply_sw_kernel, dim3((unsigned)count), dim3(TB), lds, s, items, nodes, P, sw, nmax);
+  if (nmax >= 1024)
+    hipLaunchKernelGGL(apply_sw_kernel<1024>, dim3((unsigned)count), dim3(1024), lds, s, items, nodes, P, sw, nmax);
+  else
+    hipLaunchKernelGGL(apply_sw_kernel<TB>, dim3((unsigned)count), dim3(TB), lds, s, items, nodes, P, sw, nmax);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }

@@ -90,7 +90,6 @@ struct BsNode {
   unsigned long long nderiv;
   VecOp post[2];
 };
-constexpr int kBsHeadWords = 20;  // 8-byte words of BsNode before post
 // The per-tick record of the device integrators, a ring of kBsRing ticks of
 // 2 * nodes bytes: the tick's Apply mask (1: the node takes a derivative),
 // then per node the ticks from that one on in which it surely takes one
@@ -102,10 +101,10 @@ constexpr uint8_t kBsFailed = 255;
 // post ops of the tick that ran (none when init), the accept test on the
 // node error they computed, the next tick's pre op and the node's bytes of
 // record entry rec (2 * count bytes).  init starts every node's interval
-// [t0, t1] (the step size carries over).
+// [t0, t1] (the step size carries over).  nmax: the largest node's elements.
 int launch_bs_tick(BsNode* st, int64_t count, const CmfBufs& bufs, const DNode* nodes, const cplx<double>* pool,
                    const int64_t* rhoslot, double* err, uint8_t* rec, int init, double t0, double t1, double eps,
-                   hipStream_t s);
+                   int nmax, hipStream_t s);
 
 // mask: the Apply mask that programs with kSelect | kMask write (may be null
 // when no program has kMask)

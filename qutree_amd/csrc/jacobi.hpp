@@ -34,6 +34,12 @@ struct JacobiScratch {
   int pp[32], pq[32];
 };
 
+// Orders one wavefront's LDS accesses (its lanes' are served in program order,
+// so only the compiler needs to be told); no other wavefront takes part.
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 __device__ inline double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, EW);
   return v;
@@ -199,6 +205,8 @@ __device__ __forceinline__ void jacobi_block_full(cplx<double>* A, cplx<double>*
   }
 }
 
+// By threads 0..63 of the workgroup alone, on matrices the caller has
+// synchronised; other wavefronts wait at the caller's next barrier.
 // ld must be jacobi_ld(n); the padding row and column (odd n) are set here.
 __device__ __forceinline__ void jacobi_eig(cplx<double>* A, cplx<double>* U, int n, int ld, JacobiScratch& js) {
   const int md = jacobi_dim(n);
@@ -207,7 +215,7 @@ __device__ __forceinline__ void jacobi_eig(cplx<double>* A, cplx<double>* U, int
     U[i + j * ld] = mk<double>(i == j ? 1.0 : 0.0, 0.0);
     if (i >= n || j >= n) A[i + j * ld] = czero<double>();
   }
-  __syncthreads();
+  wave_sync();
   // Hermitise (the input is Hermitian up to rounding)
   for (int o = threadIdx.x; o < n * n; o += EW) {
     const int i = o % n, j = o / n;
@@ -220,7 +228,7 @@ __device__ __forceinline__ void jacobi_eig(cplx<double>* A, cplx<double>* U, int
       A[i + i * ld].im = 0.0;
     }
   }
-  __syncthreads();
+  wave_sync();
   if (n < 2) return;
   const int m = (n + 1) & ~1;  // even player count (a dummy when n is odd)
   const int np = m / 2;
@@ -251,7 +259,7 @@ __device__ __forceinline__ void jacobi_eig(cplx<double>* A, cplx<double>* U, int
         if (!__any(flag)) continue;  // uniform: no pair rotates in this step
         rotated = 1;
         if (mine) jacobi_block_full(A, U, ld, bi == bj, p, q, ci, si, hi, pc, qc, cj, sj, hj);
-        __syncthreads();
+        wave_sync();
       }
       if (!rotated) break;
     }
@@ -275,7 +283,7 @@ __device__ __forceinline__ void jacobi_eig(cplx<double>* A, cplx<double>* U, int
       }
       if (!__any(flag)) continue;  // uniform: no pair rotates in this step
       rotated = 1;
-      __syncthreads();
+      wave_sync();
       // phase 2: every 2x2 block (rows of pair bi, columns of pair bj) gets
       // A <- G_bi^H A G_bj, and U <- U G_bj on the same rows, where
       // G = [[c, s ph], [-s conj(ph), c]] on (p, q)
@@ -284,7 +292,7 @@ __device__ __forceinline__ void jacobi_eig(cplx<double>* A, cplx<double>* U, int
         jacobi_block(A, U, n, ld, bi == bj, js.pp[bi], js.pq[bi], js.pc[bi], js.ps[bi], js.pph[bi], js.pp[bj],
                      js.pq[bj], js.pc[bj], js.ps[bj], js.pph[bj]);
       }
-      __syncthreads();
+      wave_sync();
     }
     if (!rotated) break;
   }

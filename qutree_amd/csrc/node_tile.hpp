@@ -33,20 +33,22 @@ __device__ inline void node_view(const DNode& nd, int k, int& bef, int& nk, int&
   for (int i = k + 1; i < nd.order; ++i) aft *= nd.dims[i];
 }
 
-// dst = M x_f src on an LDS-resident node tensor (M is n_f x n_f).
-template <typename T>
+// dst = M x_f src on an LDS-resident node tensor (M is n_f x n_f) by NT
+// threads; M's elements are loaded four at a time.
+template <int NT, typename T>
 __device__ void mode_apply(cplx<T>* dst, const cplx<T>* src, const cplx<T>* __restrict__ M, const DNode& nd,
                            int f) {
   int bef, nf, aft;
   node_view(nd, f, bef, nf, aft);
   const int N = nd.N;
-  for (int e = threadIdx.x; e < N; e += TB) {
+  for (int e = threadIdx.x; e < N; e += NT) {
     const int b = e % bef;
     const int q = e / bef;
     const int k = q % nf;
     const int a = q / nf;
     const cplx<T>* s = src + b + a * bef * nf;
     cplx<T> acc = czero<T>();
+#pragma unroll 4
     for (int m = 0; m < nf; ++m) cfma(acc, M[k + m * nf], s[m * bef]);
     dst[e] = acc;
   }

@@ -34,16 +34,17 @@
 
 namespace qtg {
 
-// out(j,l) = sum_r conj(X(r,j)) Y(r,l) over all indices but k.  scratch needs TB entries.
-template <typename T>
+// out(j,l) = sum_r conj(X(r,j)) Y(r,l) over all indices but k.  NT threads;
+// scratch needs NT entries.
+template <int NT, typename T>
 __device__ void contract_k(cplx<T>* __restrict__ out, const cplx<T>* X, const cplx<T>* Y, const DNode& nd, int k,
                            cplx<T>* scratch, bool accumulate) {
   int bef, nk, aft;
   node_view(nd, k, bef, nk, aft);
   const int outs = nk * nk;
   const int R = bef * aft;
-  if (outs >= TB) {
-    for (int o = threadIdx.x; o < outs; o += TB) {
+  if (outs >= NT) {
+    for (int o = threadIdx.x; o < outs; o += NT) {
       const int j = o % nk, l = o / nk;
       cplx<T> acc = czero<T>();
       const int jo = j * bef, lo = l * bef, abn = bef * nk;
@@ -57,7 +58,7 @@ __device__ void contract_k(cplx<T>* __restrict__ out, const cplx<T>* X, const cp
     }
     return;
   }
-  const int G = TB / outs;
+  const int G = NT / outs;
   const int o = threadIdx.x % outs, g = threadIdx.x / outs;
   const int j = o % nk, l = o / nk;
   cplx<T> acc = czero<T>();
@@ -87,19 +88,23 @@ __device__ void contract_k(cplx<T>* __restrict__ out, const cplx<T>* X, const cp
   }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(TB)
+// NT threads a node: 1024 for node tensors of at least 1024 elements, where
+// 256 leave a serial chain of ~10 elements a thread in every product and one
+// of R terms in the contraction (3136 elements: 55 us with 256, 31 with 1024).
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT)
     sandwich_kernel(const SwItem* __restrict__ items, const DNode* __restrict__ nodes, const cplx<T>* bra_base,
                     const cplx<T>* ket_base, cplx<T>* pool, int nmax) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* buf0 = reinterpret_cast<cplx<T>*>(smem_raw);
-  cplx<T>* buf1 = buf0 + nmax;  // nmax >= TB (scratch of contract_k)
+  cplx<T>* buf1 = buf0 + nmax;  // nmax >= NT (scratch of contract_k)
   cplx<T>* buf2 = buf1 + nmax;
-  const SwItem it = items[blockIdx.x];
-  const DNode nd = nodes[it.node];
+  // by reference: the entries indexed at run time stay out of scratch
+  const SwItem& it = items[blockIdx.x];
+  const DNode& nd = nodes[it.node];
   const int N = nd.N;
   // ket into buf0; the bra stays in global memory unless it is the ket
-  stage_to_lds<TB>(buf0, ket_base + it.ket, N);
+  stage_to_lds<NT>(buf0, ket_base + it.ket, N);
   const bool same = (bra_base == ket_base) && (it.bra == it.ket);
   __syncthreads();
   cplx<T>* cur = buf0;
@@ -107,7 +112,7 @@ __global__ void __launch_bounds__(TB)
   int nb = 0;
   for (int f = 0; f < it.nf; ++f) {
     cplx<T>* dst = bufs[nb];
-    mode_apply<T>(dst, cur, pool + it.fmat[f], nd, it.fmode[f]);
+    mode_apply<NT, T>(dst, cur, pool + it.fmat[f], nd, it.fmode[f]);
     __syncthreads();
     cur = dst;
     nb ^= 1;
@@ -120,11 +125,11 @@ __global__ void __launch_bounds__(TB)
     cplx<T>* b = (cur == buf0) ? buf1 : buf0;
     scratch = (cur == buf0) ? buf2 : ((cur == buf1) ? buf2 : buf1);
     __syncthreads();
-    stage_to_lds<TB>(b, bra_base + it.bra, N);
+    stage_to_lds<NT>(b, bra_base + it.bra, N);
     __syncthreads();
     bra = b;
   }
-  contract_k<T>(pool + it.out, bra, cur, nd, it.k, scratch, false);
+  contract_k<NT, T>(pool + it.out, bra, cur, nd, it.k, scratch, false);
 }
 
 // ---------------------------------------------------------------------- apply
@@ -153,7 +158,7 @@ __global__ void __launch_bounds__(TB)
     int nb = 0;
     cplx<T>* bufs[2] = {buf1, buf2};
     for (int f = 0; f + 1 < tm.nf; ++f) {
-      mode_apply<T>(bufs[nb], cur, pool + tm.fmat[f], nd, tm.fmode[f]);
+      mode_apply<TB, T>(bufs[nb], cur, pool + tm.fmat[f], nd, tm.fmode[f]);
       __syncthreads();
       cur = bufs[nb];
       nb ^= 1;
@@ -561,8 +566,12 @@ int launch_sandwich(const SwItem* items, int64_t count, const DNode* nodes, cons
                     void* pool, int nmax, hipStream_t s) {
   if (count == 0) return QTG_OK;
   const size_t lds = 3 * (size_t)nmax * sizeof(cplx<T>);
-  hipLaunchKernelGGL(sandwich_kernel<T>, dim3((unsigned)count), dim3(TB), lds, s, items, nodes,
-                     (const cplx<T>*)bra, (const cplx<T>*)ket, (cplx<T>*)pool, nmax);
+  if (nmax >= 1024)
+    hipLaunchKernelGGL((sandwich_kernel<T, 1024>), dim3((unsigned)count), dim3(1024), lds, s, items, nodes,
+                       (const cplx<T>*)bra, (const cplx<T>*)ket, (cplx<T>*)pool, nmax);
+  else
+    hipLaunchKernelGGL((sandwich_kernel<T, TB>), dim3((unsigned)count), dim3(TB), lds, s, items, nodes,
+                       (const cplx<T>*)bra, (const cplx<T>*)ket, (cplx<T>*)pool, nmax);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }
