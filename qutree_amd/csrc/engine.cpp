@@ -654,6 +654,8 @@ int Engine::plan() {
     if (reduced() && (rc = alloc((void**)&d_psiBuilt_, sizeof(double) * 2 * tree_.total))) return rc;
     if ((rc = up(&d_solve_, h_solve_))) return rc;
     device_buffers_.push_back(d_solve_);
+    if ((rc = up(&d_deriv_, h_deriv_))) return rc;
+    device_buffers_.push_back(d_deriv_);
     if ((rc = up(&d_combOut3_, h_comb3_))) return rc;
     device_buffers_.push_back(d_combOut3_);
     if ((rc = up(&d_combTerm3_, h_combt3_))) return rc;

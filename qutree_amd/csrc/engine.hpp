@@ -304,6 +304,7 @@ class Engine {
   int32_t* d_gmwg_ = nullptr;
   int32_t* d_gcwg_ = nullptr;
   std::vector<SolveItem> h_solve_;
+  std::vector<DerivChunk> h_deriv_;
   std::vector<GLaunch> gBuild_, gHole_, gApply_;
   std::vector<std::pair<int64_t, int>> idSlots_;  // identity matrices in the pool (offset, n)
   std::vector<CombOut> h_comb3_;
@@ -316,6 +317,7 @@ class Engine {
   GmDesc* d_gm_ = nullptr;
   GcDesc* d_gc_ = nullptr;
   SolveItem* d_solve_ = nullptr;
+  DerivChunk* d_deriv_ = nullptr;
   CombOut* d_combOut3_ = nullptr;
   CombTerm* d_combTerm3_ = nullptr;
   void* d_work_ = nullptr;

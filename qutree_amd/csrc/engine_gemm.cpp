@@ -77,6 +77,7 @@ int Engine::plan_gemm() {
   h_gmwg_.clear();
   h_gcwg_.clear();
   h_solve_.clear();
+  h_deriv_.clear();
   gBuild_.clear();
   gHole_.clear();
   gApply_.clear();
@@ -821,6 +822,22 @@ int Engine::plan_gemm() {
     g2.push_back(m2);
   }
   if (!gramInSolve_) push_gc(gApply_, fin, P64, B_PSI64, B_APPLY64, B_POOL64);
+  // D of nodes of more than 16 tiles (two a wavefront of the solve's
+  // workgroup) goes to a launch of its own, many workgroups a node, when the
+  // plan has a node that gains from it: 72 tiles (576 x 24) take 40 us in the
+  // solve, 13 tiles (196 x 16) 5 us, about what the launch costs.
+  if (fusedFinish) {
+    int64_t most = 0;
+    for (auto& si : h_solve_)
+      if (si.s >= 0) most = std::max(most, deriv_tiles(si));
+    if (most > 32)
+      for (size_t i = 0; i < h_solve_.size(); ++i) {
+        SolveItem& si = h_solve_[i];
+        if (si.s < 0 || deriv_tiles(si) <= 16) continue;
+        si.later = 1;
+        for (int t = 0; t < (si.rows + 15) / 16; t += kDerivTiles) h_deriv_.push_back({(int32_t)i, t});
+      }
+  }
   {
     GLaunch gl{};
     gl.kind = 2;
@@ -1288,6 +1305,13 @@ int Engine::run_launches(const std::vector<GLaunch>& L, size_t i0, size_t i1, vo
                              (const cplx<double>*)bases[B_PSI64], (const cplx<double>*)bases[B_APPLY64],
                              (cplx<double>*)bases[B_DPSI64], a, b, gramInSolve_)))
         return rc;
+      if (!h_deriv_.empty()) {
+        if ((rc = kernel_mark(8, &kt))) return rc;
+        if ((rc = launch_deriv(d_deriv_, (int64_t)h_deriv_.size(), d_solve_, (const cplx<double>*)bases[B_POOL64],
+                               nspf_, active, s, kt, (const cplx<double>*)bases[B_PSI64],
+                               (const cplx<double>*)bases[B_APPLY64], (cplx<double>*)bases[B_DPSI64], a, b)))
+          return rc;
+      }
       if (timing_) tfl_[8] += gl.flops;
     }
   }

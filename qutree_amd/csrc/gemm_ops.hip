@@ -1019,14 +1019,122 @@ __global__ void __launch_bounds__(256)
 // Systems with n <= 48: ping-pong Gauss-Jordan.  Each pair of column steps
 // reads the previous [S | X] buffer and writes the next one, so it costs one
 // barrier: every thread forms its elements of the scaled and eliminated
-// matrix directly from the old values (near-identity Gram matrices formed in
-// the launch take Newton-Schulz steps instead, see below).  S = A^H A is Hermitian positive definite
+// matrix directly from the old values (near-identity matrices take
+// Newton-Schulz steps instead, see below).  S = A^H A is Hermitian positive definite
 // (the node's columns are independent), so its diagonal pivots are positive
 // and elimination needs no row exchanges; for the near-orthonormal A of a
 // sweep or a CMF substep S is diagonally dominant, and the partial pivoting
 // of solve_kernel picks the same diagonal pivots, so the arithmetic per
 // element is solve_kernel's.
 constexpr int kSolveThreads = 512;  // 8 wavefronts: the derivative tiles of a node run side by side
+
+// One wavefront's 16 x 16 tiles (at most two: n <= 48 over 8 wavefronts) of
+// A B, or A B^T (kBt), for n x n matrices in LDS.
+typedef MF<double>::v4 dv4;
+template <bool kBt>
+__device__ __forceinline__ void lds_product(const cplx<double>* A, const cplx<double>* B, int n, dv4 (&re)[2],
+                                            dv4 (&im)[2]) {
+  const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4, CT = (n + 15) >> 4;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int t = wave_id() + u * (kSolveThreads / 64);
+    re[u] = im[u] = dv4{0, 0, 0, 0};
+    if (t >= CT * CT) continue;
+    const int r = (t % CT) * 16 + li, c = (t / CT) * 16 + li;
+    for (int k0 = 0; k0 < n; k0 += 16) {
+      cplx<double> a[4], b[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int k = k0 + 4 * v + kk;
+        const bool av = r < n && k < n, bv = c < n && k < n;
+        a[v] = A[av ? r + k * n : 0];
+        b[v] = B[bv ? (kBt ? c + k * n : k + c * n) : 0];
+        if (!av) a[v] = czero<double>();
+        if (!bv) b[v] = czero<double>();
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) cmma<double>(re[u], im[u], a[v], b[v]);
+    }
+  }
+}
+// f(offset in the n x n matrix, element) for this wavefront's tiles
+template <class F>
+__device__ __forceinline__ void lds_tiles(int n, const dv4 (&re)[2], const dv4 (&im)[2], const F& f) {
+  const int lane = threadIdx.x & 63, li = lane & 15, CT = (n + 15) >> 4;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int t = wave_id() + u * (kSolveThreads / 64);
+    if (t >= CT * CT) continue;
+    const int c = (t / CT) * 16 + li;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = (t % CT) * 16 + MF<double>::drow(lane, q);
+      if (r < n && c < n) f(r + c * n, mk<double>(re[u][q], im[u][q]));
+    }
+  }
+}
+
+// D = f (R x_last Y) - f (W x_last A) on row tiles rt0 .. rt1 - 1 of a node,
+// one wavefront per 16 x 16 tile: the two products of a tile load their Y and
+// A operands together, R and W come from LDS, and each product keeps the
+// accumulators and alpha scaling of the grouped mode product.
+__device__ __forceinline__ void deriv_rows(const SolveItem& it, int rt0, int rt1, const cplx<double>* Rm,
+                                           const cplx<double>* Wm, const cplx<double>* __restrict__ abase,
+                                           const cplx<double>* __restrict__ ybase, cplx<double>* obase, double fre,
+                                           double fim) {
+  typedef MF<double>::v4 v4;
+  const int n = it.n, lane = threadIdx.x & 63;
+  const int li = lane & 15, kk = lane >> 4;
+  const int rows = it.rows, CT = (n + 15) >> 4;
+  const cplx<double>* ya = ybase + it.y;
+  const cplx<double>* aa = abase + it.a;
+  for (int t = wave_id(); t < (rt1 - rt0) * CT; t += kSolveThreads / 64) {
+    const int rt = rt0 + t / CT, ct = t % CT;
+    const int r = rt * 16 + li, j = ct * 16 + li;
+    const bool rv = r < rows, cv = j < n;
+    v4 yr0 = {0, 0, 0, 0}, yi0 = yr0, yr1 = yr0, yi1 = yr0, ar0 = yr0, ai0 = yr0, ar1 = yr0, ai1 = yr0;
+    for (int k0 = 0; k0 < n; k0 += 16) {
+      cplx<double> ay[4], av[4], by[4], bw[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int kx = k0 + 4 * u + kk;
+        const bool kv = kx < n;
+        ay[u] = ldz(ya, r + (int64_t)kx * rows, rv && kv);
+        av[u] = ldz(aa, r + (int64_t)kx * rows, rv && kv);
+        const int mo = (cv && kv) ? j + kx * n : 0;
+        const cplx<double> rm = Rm[mo], wm = Wm[mo];
+        by[u] = (cv && kv) ? rm : czero<double>();
+        bw[u] = (cv && kv) ? wm : czero<double>();
+      }
+      cmma<double>(yr0, yi0, ay[0], by[0]);
+      cmma<double>(ar0, ai0, av[0], bw[0]);
+      if (k0 + 4 < n) {
+        cmma<double>(yr1, yi1, ay[1], by[1]);
+        cmma<double>(ar1, ai1, av[1], bw[1]);
+      }
+      if (k0 + 8 < n) {
+        cmma<double>(yr0, yi0, ay[2], by[2]);
+        cmma<double>(ar0, ai0, av[2], bw[2]);
+      }
+      if (k0 + 12 < n) {
+        cmma<double>(yr1, yi1, ay[3], by[3]);
+        cmma<double>(ar1, ai1, av[3], bw[3]);
+      }
+    }
+    if (!cv) continue;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int rr = rt * 16 + MF<double>::drow(lane, q);
+      if (rr >= rows) continue;
+      const double vr = yr0[q] + yr1[q], vi = yi0[q] + yi1[q];
+      const double wr = ar0[q] + ar1[q], wi = ai0[q] + ai1[q];
+      // f Y R^T and (-f) A W^T, each scaled as the mode product scales it
+      const cplx<double> py = mk<double>(fre * vr - fim * vi, fre * vi + fim * vr);
+      const cplx<double> pa = mk<double>(-fre * wr + fim * wi, -fre * wi - fim * wr);
+      obase[it.out + rr + (int64_t)j * rows] = cadd(py, pa);
+    }
+  }
+}
 
 __global__ void __launch_bounds__(kSolveThreads)
     solve_pp_kernel(const SolveItem* __restrict__ items, cplx<double>* pool, const uint8_t* __restrict__ active,
@@ -1078,29 +1186,47 @@ __global__ void __launch_bounds__(kSolveThreads)
   cplx<double> rpre = czero<double>();
   if (rpf && (int)threadIdx.x < nn) rpre = pool[it.r + threadIdx.x];
   if (gram) {
-    // S = A^H A (wavefronts 0-3) and X = A^H Y (4-7), each one 16 x 16 tile
-    // summed over four K chunks of the rows, partials added in chunk order
-    const int w = wave_id(), prod = w >> 2;
-    GcDesc gd{};
-    gd.x = it.a;
-    gd.y = prod ? it.y : it.a;
-    gd.bef = it.rows;
-    gd.aft = 1;
-    gd.nx = gd.ny = n;
-    gd.ksplit = 4;
-    const GcTile gt{0, 0, w & 3};
-    cplx<double> v[4];
-    gc_product<double, double>(gd, gt, abase, prod ? ybase : abase, v);
+    // S = A^H A and X = A^H Y, one 16 x 16 tile each, an eighth of the rows a
+    // wavefront: an element of A is both operands of S and one of X.  Partials
+    // are added in row order.
+    const int w = wave_id(), li = lane & 15, kk = lane >> 4, rows = it.rows;
+    const int span = ((rows + 31) / 32) * 4, r0 = w * span, r1 = min(rows, r0 + span);
+    const cplx<double>* ap = abase + it.a;
+    const cplx<double>* yp = ybase + it.y;
+    dv4 sre = {0, 0, 0, 0}, sim = sre, xre = sre, xim = sre;
+    for (int k0 = r0; k0 < r1; k0 += 16) {
+      cplx<double> av[4], yv[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) part[w * 256 + q * 64 + lane] = v[q];
+      for (int u = 0; u < 4; ++u) {
+        const int r = k0 + 4 * u + kk;
+        const int o = (li < n && r < r1) ? r + li * rows : 0;
+        av[u] = ap[o];
+        yv[u] = yp[o];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (k0 + 4 * u >= r1) break;  // uniform
+        const bool ok = li < n && k0 + 4 * u + kk < r1;
+        const cplx<double> a = ok ? av[u] : czero<double>(), y = ok ? yv[u] : czero<double>();
+        cmma<double>(sre, sim, cconj(a), a);
+        cmma<double>(xre, xim, cconj(a), y);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      part[w * 512 + q * 64 + lane] = mk<double>(sre[q], sim[q]);
+      part[w * 512 + 256 + q * 64 + lane] = mk<double>(xre[q], xim[q]);
+    }
     __syncthreads();
-    for (int o = threadIdx.x; o < 512; o += kSolveThreads) {
-      const int pr = o >> 8, idx = o & 255, q = idx >> 6, l = idx & 63;
+    {
+      const int o = threadIdx.x, idx = o & 255, q = idx >> 6, l = idx & 63;
       const int row = MF<double>::drow(l, q), col = l & 15;
+      static_assert(kSolveThreads == 512, "an element of [S | X] a thread");
       if (row < n && col < n) {
-        cplx<double> acc = part[(pr * 4) * 256 + idx];
-        for (int c = 1; c < 4; ++c) acc = cadd(acc, part[(pr * 4 + c) * 256 + idx]);
-        lds[pr * nn + row + col * n] = acc;
+        cplx<double> acc = part[o];
+#pragma unroll
+        for (int c = 1; c < 8; ++c) acc = cadd(acc, part[c * 512 + o]);
+        lds[(o >> 8) * nn + row + col * n] = acc;
       }
     }
   } else {
@@ -1115,19 +1241,19 @@ __global__ void __launch_bounds__(kSolveThreads)
   // rho = n max|E_ij| < 1/2 bounding the spectral radius of E, so the
   // Newton-Schulz iteration Z <- Z (2I - S Z) from Z = I converges to S^-1
   // quadratically (error rho^(2^k) after k steps); k is chosen for 1e-17 and
-  // X <- Z X.  Otherwise the elimination below runs.  (Gram mode, n <= 16.)
+  // X <- Z X, all products on the matrix cores.  Otherwise the elimination
+  // below runs (n = 48: 90 us, against 13 with one step).
   int nsk = -1;
-  if (gram) {
+  {
     double e = 0.0;
     for (int o = threadIdx.x; o < nn; o += kSolveThreads) {
       const int i = o % n, j = o / n;
       const cplx<double> v = lds[o];
       e = fmax(e, fabs((i == j ? 1.0 : 0.0) - v.re) + fabs(v.im));
     }
-    // the maximum over the wavefront, then over the 8 wavefronts (the
-    // partials are read before the barrier that precedes any write of part)
+    // the maximum over the wavefront, then over the 8 wavefronts
+    __shared__ double red[kSolveThreads / 64];
     for (int off = 32; off > 0; off >>= 1) e = fmax(e, __shfl_xor(e, off, 64));
-    double* red = reinterpret_cast<double*>(part);
     if (lane == 0) red[wave_id()] = e;
     __syncthreads();
     double em = red[0];
@@ -1140,42 +1266,34 @@ __global__ void __launch_bounds__(kSolveThreads)
       for (double r = rho; r > 1e-17 && nsk < 8; r *= r) ++nsk;
     }
   }
-  if (nsk >= 0) {
+  if (nsk > 0) {
     const cplx<double>* S = lds;
     const cplx<double>* X0 = lds + nn;
-    // Z alternates between the second [S | X] buffer and the partials; T = S Z
+    // Z and T = S Z are the second [S | X] buffer; the first step from the
+    // identity is 2I - S
     cplx<double>* Z = lds + 2 * nn;
     cplx<double>* T = lds + 3 * nn;
-    cplx<double>* Zn = part;
-    for (int o = threadIdx.x; o < nn; o += kSolveThreads) Z[o] = mk<double>(o % n == o / n ? 1.0 : 0.0, 0.0);
+    for (int o = threadIdx.x; o < nn; o += kSolveThreads) {
+      const cplx<double> v = S[o];
+      Z[o] = mk<double>((o % n == o / n ? 2.0 : 0.0) - v.re, -v.im);
+    }
     __syncthreads();
-    for (int k = 0; k < nsk; ++k) {
-      for (int o = threadIdx.x; o < nn; o += kSolveThreads) {
-        const int i = o % n, j = o / n;
-        cplx<double> acc = czero<double>();
-        for (int l = 0; l < n; ++l) cfma(acc, S[i + l * n], Z[l + j * n]);
-        T[o] = acc;
-      }
+    dv4 re[2], im[2];
+    for (int k = 1; k < nsk; ++k) {
+      lds_product<false>(S, Z, n, re, im);
+      lds_tiles(n, re, im, [&](int o, const cplx<double>& v) { T[o] = v; });
       __syncthreads();
-      for (int o = threadIdx.x; o < nn; o += kSolveThreads) {
-        const int i = o % n, j = o / n;
-        cplx<double> acc = czero<double>();
-        for (int l = 0; l < n; ++l) cfma(acc, Z[i + l * n], T[l + j * n]);
+      lds_product<false>(Z, T, n, re, im);
+      __syncthreads();
+      lds_tiles(n, re, im, [&](int o, const cplx<double>& v) {
         const cplx<double> z = Z[o];
-        Zn[o] = mk<double>(2.0 * z.re - acc.re, 2.0 * z.im - acc.im);
-      }
+        Z[o] = mk<double>(2.0 * z.re - v.re, 2.0 * z.im - v.im);
+      });
       __syncthreads();
-      cplx<double>* t = Z;
-      Z = Zn;
-      Zn = t;
     }
     // X <- Z X into the second buffer's X half
-    for (int o = threadIdx.x; o < nn; o += kSolveThreads) {
-      const int i = o % n, j = o / n;
-      cplx<double> acc = czero<double>();
-      for (int l = 0; l < n; ++l) cfma(acc, Z[i + l * n], X0[l + j * n]);
-      T[o] = acc;
-    }
+    lds_product<false>(Z, X0, n, re, im);
+    lds_tiles(n, re, im, [&](int o, const cplx<double>& v) { T[o] = v; });
     __syncthreads();
     cur = 1;
   }
@@ -1238,71 +1356,41 @@ __global__ void __launch_bounds__(kSolveThreads)
     for (int o = threadIdx.x; o < nn; o += kSolveThreads) Rm[o] = pool[it.r + o];
   }
   __syncthreads();
-  for (int o = threadIdx.x; o < nn; o += kSolveThreads) {
-    const int k = o % n, m = o / n;
-    cplx<double> acc = czero<double>();
-    for (int l = 0; l < n; ++l) cfma(acc, Rm[k + l * n], X[m + l * n]);
-    pool[it.w + o] = acc;
-    Wm[o] = acc;
+  {
+    dv4 re[2], im[2];
+    lds_product<true>(Rm, X, n, re, im);
+    lds_tiles(n, re, im, [&](int o, const cplx<double>& v) {
+      pool[it.w + o] = v;
+      Wm[o] = v;
+    });
   }
-  if (it.out < 0) return;
+  if (it.out < 0 || it.later) return;
   __syncthreads();
-  // D = f (R x_last Y) - f (W x_last A) on the node's (rows x n) tiles, one
-  // wavefront per 16 x 16 tile: the two products of a tile load their Y and A
-  // operands together, R and W come from LDS, and each product keeps the
-  // accumulators and alpha scaling of the grouped mode product.
-  typedef MF<double>::v4 v4;
-  const int li = lane & 15, kk = lane >> 4;
-  const int rows = it.rows, CT = (n + 15) >> 4;
-  const int64_t tiles = (int64_t)((rows + 15) >> 4) * CT;
-  const cplx<double>* ya = ybase + it.y;
-  const cplx<double>* aa = abase + it.a;
-  for (int64_t t = wave_id(); t < tiles; t += kSolveThreads / 64) {
-    const int rt = (int)(t / CT), ct = (int)(t - (int64_t)rt * CT);
-    const int r = rt * 16 + li, j = ct * 16 + li;
-    const bool rv = r < rows, cv = j < n;
-    v4 yr0 = {0, 0, 0, 0}, yi0 = yr0, yr1 = yr0, yi1 = yr0, ar0 = yr0, ai0 = yr0, ar1 = yr0, ai1 = yr0;
-    for (int k0 = 0; k0 < n; k0 += 16) {
-      cplx<double> ay[4], av[4], by[4], bw[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int kx = k0 + 4 * u + kk;
-        const bool kv = kx < n;
-        ay[u] = ldz(ya, r + (int64_t)kx * rows, rv && kv);
-        av[u] = ldz(aa, r + (int64_t)kx * rows, rv && kv);
-        const int mo = (cv && kv) ? j + kx * n : 0;
-        const cplx<double> rm = Rm[mo], wm = Wm[mo];
-        by[u] = (cv && kv) ? rm : czero<double>();
-        bw[u] = (cv && kv) ? wm : czero<double>();
-      }
-      cmma<double>(yr0, yi0, ay[0], by[0]);
-      cmma<double>(ar0, ai0, av[0], bw[0]);
-      if (k0 + 4 < n) {
-        cmma<double>(yr1, yi1, ay[1], by[1]);
-        cmma<double>(ar1, ai1, av[1], bw[1]);
-      }
-      if (k0 + 8 < n) {
-        cmma<double>(yr0, yi0, ay[2], by[2]);
-        cmma<double>(ar0, ai0, av[2], bw[2]);
-      }
-      if (k0 + 12 < n) {
-        cmma<double>(yr1, yi1, ay[3], by[3]);
-        cmma<double>(ar1, ai1, av[3], bw[3]);
-      }
-    }
-    if (!cv) continue;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int rr = rt * 16 + MF<double>::drow(lane, q);
-      if (rr >= rows) continue;
-      const double vr = yr0[q] + yr1[q], vi = yi0[q] + yi1[q];
-      const double wr = ar0[q] + ar1[q], wi = ai0[q] + ai1[q];
-      // f Y R^T and (-f) A W^T, each scaled as the mode product scales it
-      const cplx<double> py = mk<double>(fre * vr - fim * vi, fre * vi + fim * vr);
-      const cplx<double> pa = mk<double>(-fre * wr + fim * wi, -fre * wi - fim * wr);
-      obase[it.out + rr + (int64_t)j * rows] = cadd(py, pa);
-    }
+  deriv_rows(it, 0, (it.rows + 15) >> 4, Rm, Wm, abase, ybase, obase, fre, fim);
+}
+
+// D of the items with it.later, a chunk of kDerivTiles row tiles a workgroup:
+// one workgroup a node left most of the chip waiting for the largest nodes'
+// tiles (a plan whose largest is 1681 x 48: 300 us of the solve's 404, here 29;
+// 576 x 24: 40 of 59, here 12).
+__global__ void __launch_bounds__(kSolveThreads)
+    deriv_kernel(const DerivChunk* __restrict__ chunks, const SolveItem* __restrict__ items,
+                 const cplx<double>* __restrict__ pool, const uint8_t* __restrict__ active,
+                 const cplx<double>* __restrict__ abase, const cplx<double>* __restrict__ ybase,
+                 cplx<double>* obase, double fre, double fim) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const DerivChunk ch = chunks[blockIdx.x];
+  const SolveItem it = items[ch.item];
+  if (active && it.node >= 0 && !active[it.node]) return;
+  const int nn = it.n * it.n;
+  cplx<double>* Rm = reinterpret_cast<cplx<double>*>(smem_raw);
+  cplx<double>* Wm = Rm + nn;
+  for (int o = threadIdx.x; o < nn; o += kSolveThreads) {
+    Rm[o] = pool[it.r + o];
+    Wm[o] = pool[it.w + o];
   }
+  __syncthreads();
+  deriv_rows(it, ch.tile0, min(ch.tile0 + kDerivTiles, (it.rows + 15) >> 4), Rm, Wm, abase, ybase, obase, fre, fim);
 }
 
 }  // namespace
@@ -1393,10 +1481,10 @@ int launch_solve(const SolveItem* items, int64_t n, cplx<double>* pool, int nmax
     return QTG_EARG;
   }
   if (nmax <= 48) {
-    // two [S | X] buffers, then (gram) the 8 partial 16 x 16 tiles, which
-    // also hold the top node's 2 x kSolveThreads partial sums
-    static_assert(2 * kSolveThreads <= 8 * 256, "gram partials");
-    const size_t lds = sizeof(cplx<double>) * (4 * (size_t)nmax * nmax + (gram ? 8 * 256 : 0));
+    // two [S | X] buffers, then (gram) the 8 wavefronts' partial tiles of S
+    // and X, which also hold the top node's 2 x kSolveThreads partial sums
+    static_assert(2 * kSolveThreads <= 8 * 512, "gram partials");
+    const size_t lds = sizeof(cplx<double>) * (4 * (size_t)nmax * nmax + (gram ? 8 * 512 : 0));
     launch_timed(solve_pp_kernel, dim3((unsigned)n), dim3(kSolveThreads), (unsigned)lds, s, kt, items, pool, active,
                  abase, ybase, obase, fre, fim, nmax, gram ? 1 : 0);
     QTG_LAUNCH_CHECK();
@@ -1404,6 +1492,21 @@ int launch_solve(const SolveItem* items, int64_t n, cplx<double>* pool, int nmax
   }
   const size_t lds = 2 * sizeof(cplx<double>) * (size_t)nmax * nmax;
   launch_timed(solve_kernel, dim3((unsigned)n), dim3(256), (unsigned)lds, s, kt, items, pool, active);
+  QTG_LAUNCH_CHECK();
+  return QTG_OK;
+}
+
+int launch_deriv(const DerivChunk* chunks, int64_t nchunks, const SolveItem* items, const cplx<double>* pool,
+                 int nmax, const uint8_t* active, hipStream_t s, const KernelTiming* kt, const cplx<double>* abase,
+                 const cplx<double>* ybase, cplx<double>* obase, double fre, double fim) {
+  if (nchunks <= 0) return QTG_OK;
+  if (nmax > 48) {
+    set_error("solve: the derivative is formed for n <= 48");
+    return QTG_EARG;
+  }
+  launch_timed(deriv_kernel, dim3((unsigned)nchunks), dim3(kSolveThreads),
+               (unsigned)(2 * sizeof(cplx<double>) * (size_t)nmax * nmax), s, kt, chunks, items, pool, active, abase,
+               ybase, obase, fre, fim);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }

@@ -231,7 +231,7 @@ int launch_gm_real(const GmDesc& d, const double* x, const double* m, double* o,
 // Batched FP64 solve X <- S^-1 X for n x n column-major S and X at pool
 // offsets s, x; n <= nmax <= 64.  nmax > 48: Gauss-Jordan with partial
 // pivoting.  nmax <= 48: Gauss-Jordan on the diagonal pivots of the positive
-// definite S = A^H A, two columns per barrier, or (gram, near-identity S)
+// definite S = A^H A, two columns per barrier, or (near-identity S)
 // Newton-Schulz steps.  When r >= 0 it also forms W = R X^T at w
 // (R the n x n matrix at r).  When out >= 0 (nmax <= 48 only) it then writes
 // the projected derivative of the node, rows L = N / n, column-major:
@@ -244,11 +244,24 @@ int launch_gm_real(const GmDesc& d, const double* x, const double* m, double* o,
 struct SolveItem {
   int64_t s, x, r, w;
   int64_t a, y, out;
-  int32_t n, node, rows, pad;
+  int32_t n, node, rows, later;  // later: D by the second launch
 };
+// 16-row tiles tile0 .. tile0 + kDerivTiles - 1 of a solve item's D
+struct DerivChunk {
+  int32_t item, tile0;
+};
+constexpr int kDerivTiles = 8;
+// an item's 16 x 16 tiles of D
+inline int64_t deriv_tiles(const SolveItem& it) {
+  return (int64_t)((it.rows + 15) / 16) * ((it.n + 15) / 16);
+}
 int launch_solve(const SolveItem* items, int64_t n, cplx<double>* pool, int nmax, const uint8_t* active,
                  hipStream_t s, const KernelTiming* kt = nullptr, const cplx<double>* abase = nullptr,
                  const cplx<double>* ybase = nullptr, cplx<double>* obase = nullptr, double fre = 0.0,
                  double fim = 0.0, bool gram = false);
+// D of the items with later, whose W the solve has formed
+int launch_deriv(const DerivChunk* chunks, int64_t nchunks, const SolveItem* items, const cplx<double>* pool,
+                 int nmax, const uint8_t* active, hipStream_t s, const KernelTiming* kt, const cplx<double>* abase,
+                 const cplx<double>* ybase, cplx<double>* obase, double fre, double fim);
 
 }  // namespace qtg
