@@ -41,7 +41,10 @@ __device__ inline SmItem item_of(const SmItem* __restrict__ items, const SmItem&
   return it;
 }
 
-__device__ inline double wsum(double v) { return wave_total(v); }
+__device__ inline double wsum(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
 
 __global__ void __launch_bounds__(EW)
     heev_batch_kernel(const SmItem* __restrict__ items, SmItem u, SmItem st, const z* __restrict__ in, z* U,
@@ -343,7 +346,7 @@ __global__ void __launch_bounds__(64 * W)
 #pragma unroll
         for (int t = 0; t < RT; ++t)
           if (lane + 64 * t > j) s += a[c][t].re * a[c][t].re + a[c][t].im * a[c][t].im;
-        s = wsum(s);
+        s = wave_total(s);
         const z alpha = mk<double>(__shfl(a[c][0].re, j, 64), __shfl(a[c][0].im, j, 64));
         z t1 = czero<double>(), sc = mk<double>(1.0, 0.0);
         double beta = alpha.re;
@@ -383,8 +386,8 @@ __global__ void __launch_bounds__(64 * W)
         }
 #pragma unroll
         for (int d = c; d < CW; ++d) {
-          sr[d] = wsum(sr[d]);
-          si[d] = wsum(si[d]);
+          sr[d] = wave_total(sr[d]);
+          si[d] = wave_total(si[d]);
         }
 #pragma unroll
         for (int d = c; d < CW; ++d) {
@@ -440,8 +443,8 @@ __global__ void __launch_bounds__(64 * W)
       }
 #pragma unroll
       for (int d = c; d < CW; ++d) {
-        sr[d] = wsum(sr[d]);
-        si[d] = wsum(si[d]);
+        sr[d] = wave_total(sr[d]);
+        si[d] = wave_total(si[d]);
       }
 #pragma unroll
       for (int d = c; d < CW; ++d) {
@@ -506,6 +509,13 @@ int launch_inverse_batch(const SmItem* items, const SmItem& u, const SmItem& st,
   const size_t lds = 2 * (size_t)nmax * nmax * sizeof(z);
   hipLaunchKernelGGL(inverse_batch_kernel, dim3((unsigned)count), dim3(kInvThreads), lds, s, items, u, st,
                      (const z*)in, (z*)out);
+  QTG_LAUNCH_CHECK();
+  return QTG_OK;
+}
+
+int launch_qr_in_place(const SmItem& u, const void* in, void* out, hipStream_t s) {
+  hipLaunchKernelGGL(qr_batch_kernel, dim3(1), dim3(kQrThreads), 0, s, nullptr, u, SmItem{}, (const z*)in, (z*)out,
+                     (z*)nullptr);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }

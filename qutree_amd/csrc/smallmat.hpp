@@ -28,6 +28,10 @@ int launch_inverse_batch(const SmItem* items, const SmItem& u, const SmItem& st,
 // that qr_in_registers.
 int launch_qr_batch(const SmItem* items, const SmItem& u, const SmItem& st, int64_t count, int64_t mmax, int nmax,
                     const void* in, void* out, hipStream_t s, void* R = nullptr, bool positive = false);
+// thin Q of one matrix by the kernel of the larger matrices, whatever its
+// size: for matrices of nearly dependent columns whose Q, the rounding's own
+// choice in the directions they leave open, is to stay what it is
+int launch_qr_in_place(const SmItem& u, const void* in, void* out, hipStream_t s);
 inline bool qr_in_registers(int64_t m, int n) {
   return m <= 256 || (m <= 576 && n <= 24);
 }

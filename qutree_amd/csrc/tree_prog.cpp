@@ -463,8 +463,11 @@ int TreeProg::run_steps(const std::vector<Step>& P, hipStream_t s) {
         u.e = -1;
         u.m = st.bef;
         u.n = (int32_t)st.nn;
-        rc = launch_qr_batch(nullptr, u, zero, 1, u.m, u.n, st.abuf ? (void*)work_ : (void*)psi_,
-                             st.cbuf ? (void*)work_ : (void*)psi_, s);
+        // the SCF sweep's: Krylov vectors that leave nearly unoccupied
+        // directions to rounding, which the sweep amplifies up to 1e6 times
+        // (another order of the sums moved a state by 1.5e-10), and 2 % of
+        // its time
+        rc = launch_qr_in_place(u, st.abuf ? (void*)work_ : (void*)psi_, st.cbuf ? (void*)work_ : (void*)psi_, s);
         break;
       }
       case K_QRB:
