@@ -78,6 +78,30 @@ __device__ inline double wave_total(double v) {
                           __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
 
+// The same sum in the order of a butterfly over lane distances 32, 16, ... 1,
+// to the bit what v += __shfl_xor(v, 32), ... gives in every lane and
+// __shfl_down in lane 0, without the LDS: halves and rows exchanged by
+// permlane swaps, then rotations by 8 and by 4 within a row (whose values
+// repeat every 8 lanes by then, so lane i - 4 holds what lane i ^ 4 does) and
+// quad permutations.
+__device__ inline double swap_add32(double v) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ inline double swap_add16(double v) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ inline double wave_butterfly(double v) {
+  v = swap_add16(swap_add32(v));
+  v = dpp_add<0x128, 0xf>(v);   // row_ror:8
+  v = dpp_add<0x124, 0xf>(v);   // row_ror:4
+  v = dpp_add<0x4E, 0xf>(v);    // quad_perm [2,3,0,1]
+  return dpp_add<0xB1, 0xf>(v);  // quad_perm [1,0,3,2]
+}
+
 // per-thread last error of the C ABI
 void set_error(const std::string& msg);
 const char* get_error();

@@ -17,27 +17,21 @@ namespace {
 constexpr int kTB = 1024;
 using z = cplx<double>;
 
-// sum of v over the workgroup (every thread gets the result)
+// Sum of v over the workgroup (every thread gets the result): the wavefronts'
+// sums, then those of all in the same butterfly, which wavefronts that a
+// smaller workgroup lacks enter as zeros.  red is this call's own.
 __device__ double block_sum(double v, double* red) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  v = wave_butterfly(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
   if (lane == 0) red[wave] = v;
   __syncthreads();
-  double s = 0.0;
-  if (threadIdx.x < 64) {
-    s = threadIdx.x < (kTB / 64) ? red[threadIdx.x] : 0.0;
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-    if (threadIdx.x == 0) red[kTB / 64] = s;
-  }
-  __syncthreads();
-  return red[kTB / 64];
+  return wave_butterfly(lane < (int)(blockDim.x >> 6) ? red[lane] : 0.0);
 }
 
 // v0 = psi / |psi| into the Krylov slot 0 and the apply input slot
 __global__ void __launch_bounds__(kTB)
     lanczos_begin_kernel(const z* __restrict__ psi, int64_t N, z* __restrict__ kry0, z* __restrict__ in) {
-  __shared__ double red[kTB / 64 + 1];
+  __shared__ double red[kTB / 64];
   double s = 0.0;
   for (int64_t i = threadIdx.x; i < N; i += kTB) s += psi[i].re * psi[i].re + psi[i].im * psi[i].im;
   const double nrm = sqrt(block_sum(s, red));
@@ -48,6 +42,21 @@ __global__ void __launch_bounds__(kTB)
   }
 }
 
+// the last step: alpha_j and the k x k tridiagonal matrix
+__device__ void lanczos_tridiagonal(int j, int k, double alpha, double* scal, z* T) {
+  __syncthreads();
+  if (threadIdx.x == 0) scal[j] = alpha;
+  __syncthreads();
+  for (int e = threadIdx.x; e < k * k; e += blockDim.x) {
+    const int r = e % k, c = e / k;
+    double x = 0.0;
+    if (r == c) x = (r == j) ? alpha : scal[r];
+    else if (r == c + 1) x = scal[k + c];
+    else if (c == r + 1) x = scal[k + r];
+    T[e] = mk<double>(x, 0.0);
+  }
+}
+
 // Step j of the recurrence: alpha_j = Re <v_j|H v_j>, w = H v_j - alpha_j v_j
 // - beta_{j-1} v_{j-1}; below the last step beta_j = |w| and v_{j+1} = w /
 // beta_j, at the last step the k x k tridiagonal matrix is written to T.
@@ -55,7 +64,7 @@ __global__ void __launch_bounds__(kTB)
 __global__ void __launch_bounds__(kTB)
     lanczos_step_kernel(int j, int k, int64_t N, const z* __restrict__ ha, int parts, z* kry, z* __restrict__ in,
                         double* __restrict__ scal, z* __restrict__ T) {
-  __shared__ double red[kTB / 64 + 1];
+  __shared__ double red[2][kTB / 64];
   const z* v = kry + (int64_t)j * N;
   double s = 0.0;
   for (int64_t i = threadIdx.x; i < N; i += kTB) {
@@ -66,7 +75,7 @@ __global__ void __launch_bounds__(kTB)
     }
     s += v[i].re * hr + v[i].im * hi;
   }
-  const double alpha = block_sum(s, red);
+  const double alpha = block_sum(s, red[0]);
   const double bprev = j > 0 ? scal[k + j - 1] : 0.0;
   const z* vp = kry + (int64_t)(j > 0 ? j - 1 : 0) * N;
   z* w = kry + (int64_t)(j + 1 < k ? j + 1 : j) * N;  // the last step's w is not kept
@@ -88,7 +97,7 @@ __global__ void __launch_bounds__(kTB)
     }
   }
   if (j + 1 < k) {
-    const double beta = sqrt(block_sum(s2, red));
+    const double beta = sqrt(block_sum(s2, red[1]));
     for (int64_t i = threadIdx.x; i < N; i += kTB) {
       const z x = mk<double>(w[i].re / beta, w[i].im / beta);
       w[i] = x;
@@ -99,17 +108,80 @@ __global__ void __launch_bounds__(kTB)
       scal[k + j] = beta;
     }
   } else {
-    __syncthreads();
-    if (threadIdx.x == 0) scal[j] = alpha;
-    __syncthreads();
-    for (int e = threadIdx.x; e < k * k; e += kTB) {
-      const int r = e % k, c = e / k;
-      double x = 0.0;
-      if (r == c) x = (r == j) ? alpha : scal[r];
-      else if (r == c + 1) x = scal[k + c];
-      else if (c == r + 1) x = scal[k + r];
-      T[e] = mk<double>(x, 0.0);
+    lanczos_tridiagonal(j, k, alpha, scal, T);
+  }
+}
+
+// The same for N <= 1024 E with the elements in registers: every operand is
+// loaded before the first reduction and none twice.  A workgroup has as many
+// wavefronts as the tensor needs (E 1), so small nodes wait for fewer.  The
+// sums keep the order of the kernel above, so which of them runs changes no
+// bit.  The SCF of 16 modes (512 elements a node and fewer) is a chain of
+// launches of a few us: with these, the butterfly without LDS and the QR in
+// LDS 8615 -> 7880 us a sweep.
+template <int E>
+__global__ void __launch_bounds__(kTB)
+    lanczos_step_reg(int j, int k, int64_t N, const z* __restrict__ ha, int parts, z* __restrict__ kry,
+                     z* __restrict__ in, double* __restrict__ scal, z* __restrict__ T) {
+  __shared__ double red[2][kTB / 64];
+  const int n = (int)N;
+  const z* v = kry + (int64_t)j * N;
+  const z* vp = kry + (int64_t)(j > 0 ? j - 1 : 0) * N;
+  const double bprev = j > 0 ? scal[k + j - 1] : 0.0;
+  z vv[E], pv[E];
+  double hr[E], hi[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = min((int)threadIdx.x + e * kTB, n - 1);
+    vv[e] = v[i];
+    pv[e] = vp[i];
+    hr[e] = hi[e] = 0.0;
+  }
+#pragma unroll 4
+  for (int p = 0; p < parts; ++p)
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const z h = ha[min((int)threadIdx.x + e * kTB, n - 1) + p * N];
+      hr[e] += h.re;
+      hi[e] += h.im;
     }
+  double s = 0.0;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if ((int)threadIdx.x + e * kTB < n) s += vv[e].re * hr[e] + vv[e].im * hi[e];
+  const double alpha = block_sum(s, red[0]);
+  if (j + 1 < k) {
+    z* w = kry + (int64_t)(j + 1) * N;
+    double s2 = 0.0;
+    z wv[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if ((int)threadIdx.x + e * kTB < n) {
+        double wr = hr[e] - alpha * vv[e].re, wi = hi[e] - alpha * vv[e].im;
+        if (j > 0) {
+          wr -= bprev * pv[e].re;
+          wi -= bprev * pv[e].im;
+        }
+        wv[e] = mk<double>(wr, wi);
+        s2 += wr * wr + wi * wi;
+      }
+    }
+    const double beta = sqrt(block_sum(s2, red[1]));
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = (int)threadIdx.x + e * kTB;
+      if (i < n) {
+        const z x = mk<double>(wv[e].re / beta, wv[e].im / beta);
+        w[i] = x;
+        in[i] = x;
+      }
+    }
+    if (threadIdx.x == 0) {
+      scal[j] = alpha;
+      scal[k + j] = beta;
+    }
+  } else {
+    lanczos_tridiagonal(j, k, alpha, scal, T);
   }
 }
 
@@ -121,7 +193,7 @@ __global__ void __launch_bounds__(kTB)
     krylov_combine_kernel(int k, int64_t N, const z* __restrict__ U, const double* __restrict__ ev,
                           const z* __restrict__ kry, z* __restrict__ out, const ScfParams* __restrict__ par,
                           double* __restrict__ elog, int slot) {
-  __shared__ double red[kTB / 64 + 1];
+  __shared__ double red[kTB / 64];
   __shared__ z c[kMaxKrylov];
   const int itp = par->itp;
   if (threadIdx.x < k) {
@@ -177,7 +249,7 @@ __global__ void permute_kernel(const z* __restrict__ in, z* __restrict__ out, in
 // Tensor_Implementation.h:806-853)
 __global__ void __launch_bounds__(kTB)
     normalize_kernel(const z* __restrict__ in, z* __restrict__ out, int64_t N, double* __restrict__ nrm2) {
-  __shared__ double red[kTB / 64 + 1];
+  __shared__ double red[kTB / 64];
   double s = 0.0;
   for (int64_t i = threadIdx.x; i < N; i += kTB) s += in[i].re * in[i].re + in[i].im * in[i].im;
   const double t = block_sum(s, red);
@@ -206,8 +278,13 @@ int launch_lanczos_step(int j, int k, int64_t N, const void* ha, int parts, void
     set_error("lanczos: Krylov size outside 1..64");
     return QTG_EARG;
   }
-  hipLaunchKernelGGL(lanczos_step_kernel, dim3(1), dim3(kTB), 0, s, j, k, N, (const z*)ha, parts, (z*)kry, (z*)in,
-                     scal, (z*)T);
+#define QTG_STEP(K, THREADS)                                                                                       \
+  hipLaunchKernelGGL(K, dim3(1), dim3(THREADS), 0, s, j, k, N, (const z*)ha, parts, (z*)kry, (z*)in, scal, (z*)T)
+  if (N <= kTB) QTG_STEP(lanczos_step_reg<1>, (unsigned)((N + 63) / 64 * 64));
+  else if (N <= 2 * kTB) QTG_STEP(lanczos_step_reg<2>, kTB);
+  else if (N <= 4 * kTB) QTG_STEP(lanczos_step_reg<4>, kTB);
+  else QTG_STEP(lanczos_step_kernel, kTB);
+#undef QTG_STEP
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }

@@ -41,10 +41,7 @@ __device__ inline SmItem item_of(const SmItem* __restrict__ items, const SmItem&
   return it;
 }
 
-__device__ inline double wsum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+__device__ inline double wsum(double v) { return wave_butterfly(v); }
 
 __global__ void __launch_bounds__(EW)
     heev_batch_kernel(const SmItem* __restrict__ items, SmItem u, SmItem st, const z* __restrict__ in, z* U,
@@ -306,6 +303,20 @@ __global__ void __launch_bounds__(kQrThreads)
   qr_inplace(W, m, n, tau, (Rb && it.e >= 0) ? Rb + it.e : nullptr);
 }
 
+// One matrix, the same arithmetic on a copy in LDS (dynamic: m n elements):
+// every pass of a column reads what the one before wrote, an LDS round trip
+// instead of a global one.
+__global__ void __launch_bounds__(kQrThreads) qr_lds_kernel(SmItem it, const z* in, z* out) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ z tau[64];
+  z* W = reinterpret_cast<z*>(smem_raw);
+  const int N = (int)it.m * it.n;
+  for (int o = threadIdx.x; o < N; o += kQrThreads) W[o] = in[it.a + o];
+  __syncthreads();
+  qr_inplace(W, it.m, it.n, tau, nullptr);
+  for (int o = threadIdx.x; o < N; o += kQrThreads) out[it.q + o] = W[o];
+}
+
 // The same QR with the matrix in registers: wavefront w of W holds columns
 // w, w + W, ... (at most CW), a lane rows lane + 64 t (t < RT).  The
 // owner of column j forms the reflector and leaves v in LDS; after one
@@ -514,8 +525,12 @@ int launch_inverse_batch(const SmItem* items, const SmItem& u, const SmItem& st,
 }
 
 int launch_qr_in_place(const SmItem& u, const void* in, void* out, hipStream_t s) {
-  hipLaunchKernelGGL(qr_batch_kernel, dim3(1), dim3(kQrThreads), 0, s, nullptr, u, SmItem{}, (const z*)in, (z*)out,
-                     (z*)nullptr);
+  const int64_t N = u.m * u.n;
+  if (N <= 8192)  // 128 KB
+    hipLaunchKernelGGL(qr_lds_kernel, dim3(1), dim3(kQrThreads), N * sizeof(z), s, u, (const z*)in, (z*)out);
+  else
+    hipLaunchKernelGGL(qr_batch_kernel, dim3(1), dim3(kQrThreads), 0, s, nullptr, u, SmItem{}, (const z*)in, (z*)out,
+                       (z*)nullptr);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }
