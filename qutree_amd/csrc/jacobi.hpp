@@ -1,7 +1,7 @@
 // Wavefront Jacobi eigensolver for small Hermitian matrices (FP64, n <= 64)
 // held in LDS, column-major with leading dimension jacobi_ld(n) (even order,
 // see jacobi_dim).  All lanes of a
-// 64-lane workgroup call it.  Tournament (round-robin) ordering: each step
+// 64-lane workgroup, or threads 0..63 of a larger one, call it.  Tournament (round-robin) ordering: each step
 // rotates up to 32 disjoint (p,q) pairs whose parameters come from the same
 // matrix; one pass applies both sides at once, each lane owning 2 x 2 blocks
 // (rows of pair i, columns of pair j), and a wavefront vote skips steps in
