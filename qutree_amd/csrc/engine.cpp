@@ -66,6 +66,10 @@ void Engine::release() {
   for (void* p : device_buffers_)
     if (p) (void)hipFree(p);
   device_buffers_.clear();
+  // buffers that only some plans allocate
+  d_psiBuilt_ = nullptr;
+  d_part_ = nullptr;
+  d_work32_ = nullptr;
   d_grad64_ = nullptr;
   d_escal_ = nullptr;
   d_elog_ = nullptr;

@@ -133,3 +133,35 @@ def test_reduced_gradient_and_split_precision(name, every_size):
         assert abs(g.energy() - e_ref) < 1e-9 * abs(e_ref)
     print(f"  split derivative err, every matrix {errs[0]:.2e} reduced {errs[1]:.2e}", flush=True)
     assert errs[1] < max(4 * errs[0], 1e-7)
+
+
+@pytest.mark.parametrize("order", ["large_small", "small_large", "large_small_large"])
+def test_second_hamiltonian_on_the_other_side_of_the_line(order):
+    """One engine, Hamiltonians whose plans are reduced (large: 0.78 GFLOP of
+    single matrices) and are not (small: 0.18) one after the other: buffers
+    that only one of the plans has are not used by the other, and every matrix
+    is that of the plan at hand."""
+    print(f"case second hamiltonian {order}", flush=True)
+    text = W.balanced_tree_text(16, 6, [5, 14, 20, 20])
+    models = {"large": W.coupled_quartic(16, 5, c_sigma=0.01), "small": _one_mode(16)}
+    oracles = {k: O.OracleModel(text, H) for k, H in models.items()}
+    eng = Q.Engine(text)
+    for i, k in enumerate(order.split("_")):
+        om, H = oracles[k], models[k]
+        eng.set_hamiltonian(H)
+        for seed in (i, i + 10):
+            psi = om.fill_random(seed, delta_lowest=False)
+            ref = om.derivative(psi)
+            full = Q.Engine(text, H, compress=False)  # as in test_reduced_sweep_matches_oracle
+            full.set_psi(psi)
+            full.derivative()
+            lim = max(1e-12, 4 * _err(full.get(0), ref))
+            eng.set_psi(psi)
+            eng.derivative()
+            print(f"  {k} derivative rel err {_err(eng.get(0), ref):.2e} limit {lim:.2e}", flush=True)
+            assert _err(eng.get(0), ref) < lim
+            e = om.energy(psi)
+            assert abs(eng.energy() - e) < 1e-12 * abs(e)
+            a = om.sparse_tree(0)[0]
+            h = om.hmat(0, a)
+            assert np.max(np.abs(eng.matrix(2, 0, a) - h)) < 1e-11 * max(1, np.max(np.abs(h)))
