@@ -811,7 +811,16 @@ std::vector<Engine::Summand> Engine::aggregate(const std::vector<Summand>& tl, c
   return groups;
 }
 
+// The side stream of the last build still reads the state (its copy for
+// get_matrix): whoever writes d_psi64_ on stream s comes after it.
+int Engine::before_psi_write(hipStream_t s) {
+  if (heevPending_) QTG_HIP_TRY(hipStreamWaitEvent(s, evHeev_, 0));
+  return QTG_OK;
+}
+
 int Engine::set_psi(const double* host, hipStream_t s) {
+  const int rc = before_psi_write(s);
+  if (rc) return rc;
   QTG_HIP_TRY(hipMemcpyAsync(d_psi64_, host, sizeof(double) * 2 * tree_.total, hipMemcpyHostToDevice, s));
   QTG_HIP_TRY(hipStreamSynchronize(s));
   built_ = false;
@@ -819,6 +828,8 @@ int Engine::set_psi(const double* host, hipStream_t s) {
 }
 
 int Engine::set_psi_device(const double* dev, hipStream_t s) {
+  const int rc = before_psi_write(s);
+  if (rc) return rc;
   QTG_HIP_TRY(hipMemcpyAsync(d_psi64_, dev, sizeof(double) * 2 * tree_.total, hipMemcpyDeviceToDevice, s));
   built_ = false;
   return QTG_OK;

@@ -258,6 +258,7 @@ class Engine {
   double* d_psiBuilt_ = nullptr;
   int64_t builds_ = 0, fullBuild_ = -1;
   int full_engine(hipStream_t s);
+  int before_psi_write(hipStream_t s);
   std::vector<Summand> aggregate(const std::vector<Summand>& tl, const std::vector<int>& sdim, int64_t& off,
                                  double& combFlops);
   std::vector<CombOut> h_comb1_, h_comb2_;  // aggregated slots: partial sums, sums of partials

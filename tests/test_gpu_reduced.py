@@ -165,3 +165,34 @@ def test_second_hamiltonian_on_the_other_side_of_the_line(order):
             a = om.sparse_tree(0)[0]
             h = om.hmat(0, a)
             assert np.max(np.abs(eng.matrix(2, 0, a) - h)) < 1e-11 * max(1, np.max(np.abs(h)))
+
+
+def test_matrices_are_those_of_the_last_build_without_an_apply(every_size):
+    """build() alone, then another state: nothing but the setters themselves
+    orders the copy of the built state (side stream, behind the eigensolvers
+    of earlier builds) before the new one."""
+    text, H = _models()["wide8"]
+    print("case matrices after build, then set_psi", flush=True)
+    om = O.OracleModel(text, H)
+    eng = Q.Engine(text, H)
+    states = [om.fill_random(s, delta_lowest=False) for s in range(4)]
+    dev = [Q.DeviceBuffer.from_array(p) for p in states]
+    term, node = 0, om.sparse_tree(0)[0]
+
+    def check(i):
+        om.build(states[i])
+        for which, ref in ((2, om.hmat(term, node)), (3, om.hole(term, node))):
+            assert np.max(np.abs(eng.matrix(which, term, node) - ref)) < 1e-11 * max(1, np.max(np.abs(ref)))
+
+    for setter in (lambda i: eng.set_psi(states[i]),
+                   lambda i: Q.check(Q.lib().qtg_engine_set_psi_device(eng.ptr, dev[i].ptr, None))):
+        for rounds in (1, 3):
+            for r in range(rounds):  # eigensolvers of the earlier builds still queued
+                setter(r)
+                eng.build()
+            setter(3)
+            check(rounds - 1)
+    eng.set_psi(states[1])
+    eng.build()
+    Q.check(Q.lib().qtg_engine_canonicalize(eng.ptr, None, None))  # rewrites the state on the device
+    check(1)
