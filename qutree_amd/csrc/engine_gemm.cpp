@@ -204,6 +204,15 @@ int Engine::plan_gemm() {
   auto item_hi = [&](int64_t out) {
     return precision_ == 0 || (precision_ == 2 && highSlots_.count(out) > 0);
   };
+  // Summed contractions stand for many matrices, each of which the sweep
+  // that forms them all rounds on its own: in FP32 their coherent sums lose
+  // that averaging (Apply's error 3 % larger for 32 oscillators with pair
+  // couplings in the complex64 form).  They are formed in FP64 there, and in
+  // the split form while that costs nothing: the launches of both precisions
+  // in one win up to 35 GFLOP of single matrices (64 modes: 339 -> 323 us a
+  // sweep, 670 -> 651), from 75 on the FP64 products lose (1000 -> 1024, 128
+  // modes 2686 -> 3006).
+  const bool sums64 = precision_ == 1 || lflops_ < 5e10;
   int64_t wbase = 0, wbase32 = 0, wmax = 0, wmax32 = 0;
   // descriptors of one layer: first factors, second factors, contractions
   // ([0] FP32, [1] FP64)
@@ -235,8 +244,8 @@ int Engine::plan_gemm() {
       int64_t x, y;
       int sel;
     };
-    // (coef: a group's coefficient, carried by its first product, or by a
-    // copy of the ket where it has none)
+    // (coef: a group's coefficient on FP64 tensors, carried by its first
+    // product, or by a copy of the ket where it has none)
     auto operands = [&](Side& S, const HNode& p, int k, const std::vector<std::pair<int, int64_t>>& fac,
                         cd coef = cd(1.0, 0.0)) {
       const bool scaled = coef != cd(1.0, 0.0);
@@ -325,7 +334,7 @@ int Engine::plan_gemm() {
       S.con.push_back(g);
     }
     for (const Fused* f : fused) {
-      const int hp = item_hi(f->out) ? 1 : 0;
+      const int hp = sums64 || item_hi(f->out) ? 1 : 0;
       Side& S = sd[hp];
       const HNode& p = tree_.nodes[f->node];
       LayerLists::Sum sm{};
@@ -345,8 +354,10 @@ int Engine::plan_gemm() {
           const bool own = f->slots[q].kind == SlotRef::HOLE;
           fac.push_back({own ? p.order() - 1 : tree_.nodes[f->slots[q].node].childIdx, g.ids[q]});
         }
-        const XY o = operands(S, p, f->k, fac, g.coef);
-        sm.segs.push_back({o.x, o.y, o.sel, 0});
+        // FP32 kets stay unscaled: their coefficient is applied in FP64
+        const XY o = hp ? operands(S, p, f->k, fac, g.coef) : operands(S, p, f->k, fac);
+        const cd a = hp ? cd(1.0, 0.0) : g.coef;
+        sm.segs.push_back({o.x, o.y, o.sel, 0, a.real(), a.imag()});
       }
       out.sums[hp].push_back(sm);
     }

@@ -250,7 +250,9 @@ __global__ void __launch_bounds__(1024)
 // One workgroup per macro tile and share: its wavefronts split the
 // concatenated reduction of all segments evenly, so a sum over many small
 // contractions (the summed matrices of a sweep) is as wide as one long one
-// and needs neither a matrix per segment nor a pass to add them.
+// and needs neither a matrix per segment nor a pass to add them.  FP32
+// products keep what a matrix per segment gave: a segment's share is added,
+// with its coefficient, in FP64.
 template <typename T, int NT, int W>
 __global__ void __launch_bounds__(64 * W)
     gc_sum_kernel(const GcSum* __restrict__ tasks, const GcSeg* __restrict__ segs, const cplx<T>* __restrict__ X0,
@@ -277,6 +279,15 @@ __global__ void __launch_bounds__(64 * W)
   for (int i = 0; i < NT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) cr[i][j] = ci[i][j] = v4{0, 0, 0, 0};
+  constexpr bool kFlush = std::is_same<T, float>::value;
+  typedef MF<double>::v4 dv4;
+  dv4 dr[NT][NT], di[NT][NT];  // kFlush: the sum over segments
+  if constexpr (kFlush) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) dr[i][j] = di[i][j] = dv4{0, 0, 0, 0};
+  }
   int sg = kb < ke ? (int)(kb / K) : nseg;
   for (; sg < nseg && (int64_t)sg * K < ke; ++sg) {
     const int64_t s0 = (int64_t)sg * K;
@@ -294,6 +305,20 @@ __global__ void __launch_bounds__(64 * W)
       else if (ncb == 1) gc_block_product<T, NT, 2, 1, 2>(g, j0, l0, lo, hi, X, Y, cr, ci);
       else gc_block_product<T, NT, 2, 2, 2>(g, j0, l0, lo, hi, X, Y, cr, ci);
     }
+    if constexpr (kFlush) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const double vr = cr[i][j][q], vi = ci[i][j][q];
+            dr[i][j][q] += e.are * vr - e.aim * vi;
+            di[i][j][q] += e.are * vi + e.aim * vr;
+          }
+          cr[i][j] = ci[i][j] = v4{0, 0, 0, 0};
+        }
+    }
   }
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
@@ -303,7 +328,10 @@ __global__ void __launch_bounds__(64 * W)
       if (j >= ncb) break;
       cplx<double>* buf = red + (NB > 1 ? ((i * NT + j) & 1) * W * 256 : 0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) buf[wave * 256 + q * 64 + lane] = mk<double>((double)cr[i][j][q], (double)ci[i][j][q]);
+      for (int q = 0; q < 4; ++q) {
+        if constexpr (kFlush) buf[wave * 256 + q * 64 + lane] = mk<double>(dr[i][j][q], di[i][j][q]);
+        else buf[wave * 256 + q * 64 + lane] = mk<double>(cr[i][j][q], ci[i][j][q]);
+      }
       __syncthreads();
       if (threadIdx.x < 256) {
         const int e = threadIdx.x, el = e & 63;

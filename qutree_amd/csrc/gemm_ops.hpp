@@ -203,8 +203,9 @@ int launch_gc_one(const GcDesc& d, const GcOnePlan& p, const void* x, const void
                   hipStream_t s);
 
 // Summed hole contraction (gemm_block.hip): out(j, l) = add(j, l) + sum over
-// segments of sum_{b,a} conj(X(b,j,a)) Y(b,l,a), X and Y (bef, n, aft) at
-// the segment's offsets.  A GcSum is one macro tile of nt x nt 16 x 16 tiles
+// segments of alpha sum_{b,a} conj(X(b,j,a)) Y(b,l,a), X and Y (bef, n, aft) at
+// the segment's offsets.  Segments are added in FP64; FP32 products (T float)
+// are accumulated in FP32 within a segment only.  A GcSum is one macro tile of nt x nt 16 x 16 tiles
 // (of ceil(n / (16 nt))^2) and one of its S shares of the concatenated
 // reduction; with S > 1 the share leaves nt^2 256 elements at that many times
 // (part + share) and a second launch over one GcSum per macro tile adds them
@@ -213,6 +214,7 @@ int launch_gc_one(const GcDesc& d, const GcOnePlan& p, const void* x, const void
 struct GcSeg {
   int64_t x, y;
   int32_t sel, pad;  // as GcDesc::sel
+  double are, aim;   // coefficient of the segment (FP32 products only; FP64 kets carry it)
 };
 struct GcSum {
   int64_t out, add;  // add < 0: none

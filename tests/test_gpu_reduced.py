@@ -196,3 +196,54 @@ def test_matrices_are_those_of_the_last_build_without_an_apply(every_size):
     eng.build()
     Q.check(Q.lib().qtg_engine_canonicalize(eng.ptr, None, None))  # rewrites the state on the device
     check(1)
+
+
+def _coherent(f):
+    """Pair couplings of one sign: sums that many matrices enter alike."""
+    H = W.Hamiltonian()
+    for i in range(f):
+        H.add_term(1.0, [(i, W.FACTOR_KIN)])
+        H.add_term(0.5, [(i, W.FACTOR_X2)])
+    for i in range(f):
+        for j in range(i):
+            H.add_term(0.02, [(i, W.FACTOR_X2), (j, W.FACTOR_X2)])
+    return H
+
+
+def _apply_rms(text, H, precision, seeds):
+    """RMS over random states of the relative error of Apply at all nodes
+    against the complex128 engine."""
+    ref, eng = Q.Engine(text, H), Q.Engine(text, H, precision=precision)
+    err = []
+    for s in range(seeds):
+        psi = ref.fill_random(100 + s, delta_lowest=False)
+        for e in (ref, eng):
+            e.set_psi(psi)
+            e.derivative()
+        err.append(_err(eng.get(1), ref.get(1)))
+    return float(np.sqrt(np.mean(np.square(err))))
+
+
+# quartic64: more than 50 GFLOP, where the split form's sums are FP32 products
+PRECISION_MODELS = {
+    "coherent16": (1, 24, W.balanced_tree_text(16, 8, [4, 6, 6, 6]), _coherent(16)),
+    "coherent16_split": (2, 24, W.balanced_tree_text(16, 8, [4, 6, 6, 6]), _coherent(16)),
+    "ho16": (1, 24, W.balanced_tree_text(16, 8, [4, 6, 8, 8]), W.coupled_ho(16, 3, one_mode_matrix=True)),
+    "quartic64": (1, 4, W.balanced_tree_text(64, 8, [8, 14, 21, 27, 34, 41]), W.coupled_quartic(64, 64)),
+    "quartic64_split": (2, 4, W.balanced_tree_text(64, 8, [8, 14, 21, 27, 34, 41]), W.coupled_quartic(64, 64)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(PRECISION_MODELS))
+def test_reduced_precision_forms_lose_none_to_the_sums(name, monkeypatch):
+    """The FP32 products of a plan that forms every matrix are rounded matrix
+    by matrix and summed in FP64; sums formed as contractions must not be
+    further off.  0.5 %: the sampling of the RMS over the states."""
+    print(f"case reduced precision {name}", flush=True)
+    precision, seeds, text, H = PRECISION_MODELS[name]
+    err = {}
+    for form, line in (("every matrix", "1e30"), ("reduced", "0")):
+        monkeypatch.setenv("QTG_REDUCE_MIN_FLOPS", line)
+        err[form] = _apply_rms(text, H, precision, seeds)
+        print(f"  {form} {err[form]:.3e}", flush=True)
+    assert err["reduced"] < 1.005 * err["every matrix"]
