@@ -222,8 +222,12 @@ int qtg_engine_get_dpsi(qtg_engine engine, double* host, int which, qtg_stream s
 int qtg_engine_energy(qtg_engine engine, double* energy, qtg_stream stream);
 /* which: 0 rho[node], 1 rho^-1[node], 2 h-matrix[term][node], 3 hole[term][node]
  * of the last build (or derivative).  A compressed engine may form a term's
- * matrices only inside sums; the first call with which 2 or 3 after a build
- * then forms all of them at that build's state, in buffers of their own. */
+ * matrices only inside sums.  The first call with which 2 or 3 for such a
+ * matrix after a build forms all matrices of that term at the build's state, in
+ * buffers of their own (64 modes 0.15 ms, 128 modes 0.4); calls for other
+ * terms widen this to 64 terms, then to all (128 modes, 8256 terms: 12 ms a
+ * build and 3.5 GB), each time planning for them first (up to 0.4 s).  A group
+ * of terms that does not fit the memory is halved. */
 int qtg_engine_get_matrix(qtg_engine engine, int which, int64_t term, int64_t node, double* out,
                           qtg_stream stream);
 /* FLOPs of one H|Psi> sweep of the reference algorithm (8 per complex

@@ -5,6 +5,7 @@
 #include "engine.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -60,8 +61,8 @@ void Engine::invalidate_graph() {
 }
 
 void Engine::release() {
-  full_.reset();
-  fullBuild_ = -1;
+  terms_.reset();
+  termsCap_ = INT_MAX;
   builds_ = 0;
   for (void* p : device_buffers_)
     if (p) (void)hipFree(p);
@@ -79,6 +80,8 @@ void Engine::release() {
 
 int Engine::alloc(void** p, size_t bytes) {
   if (hipMalloc(p, std::max<size_t>(bytes, 16)) != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
     set_error("engine: device allocation failed");
     return QTG_ENOMEM;
   }
@@ -525,6 +528,7 @@ int Engine::plan() {
     fin.push_back(fn);
   }
   keep_.assign(items.size(), 1);
+  formed_.clear();
   // A plan whose single matrices cost less than kReduceFlops keeps them all:
   // there the launches decide, and the summed contractions add one (the sums
   // of h-matrices) and fuse no hole layer.  Sweeps measured on both sides:
@@ -574,6 +578,8 @@ int Engine::plan() {
       }
       keep_[i] = 0;
     }
+    for (size_t i = 0; i < items.size(); ++i)
+      if (keep_[i]) formed_.insert(items[i].out);
   }
   poolSize_ = off;
   nChunks_ = (int64_t)chunks.size();
@@ -1064,37 +1070,53 @@ int Engine::energy(hipStream_t s, double* out) {
   return QTG_OK;
 }
 
-// The engine that forms every matrix of every term, at the state of the last
-// build.
-int Engine::full_engine(hipStream_t s) {
+// An engine that forms every matrix of a group of terms with `term` among
+// them, at the state of the last build: the one term asked for, then 64 of
+// them, then all, as further terms are.  A program that watches one term pays
+// for one, one that reads all of them plans three times.  A group that does
+// not fit the memory is halved.
+int Engine::term_engine(int term, hipStream_t s) {
   if (builds_ == 0) {
     set_error("engine: build() first");
     return QTG_ESTATE;
   }
   int rc;
-  if (!full_) {
-    std::unique_ptr<Engine> e(new Engine());
-    if ((rc = e->create(treeText_, precision_))) return rc;
-    e->reduce_ = false;
-    e->graph_ = false;
-    e->tuning_ = false;
-    e->splitWaves_ = splitWaves_;
-    e->splitMinK_ = splitMinK_;
-    e->gmSplitK_ = gmSplitK_;
-    e->gcLongK_ = gcLongK_;
-    e->fuseHoles_ = fuseHoles_;
-    e->sop_ = sop_;
-    if ((rc = e->plan())) return rc;
-    full_ = std::move(e);
+  const int L = (int)sop_.terms.size();
+  if (!terms_ || term < terms0_ || term >= terms0_ + (int)terms_->sop_.terms.size()) {
+    int n = std::min(!terms_ ? 1 : termsN_ < 64 ? 64 : L, std::min(termsCap_, L));
+    for (;; n = termsCap_ = n / 2) {
+      terms_.reset();
+      terms0_ = term / n * n;
+      std::unique_ptr<Engine> e(new Engine());
+      if ((rc = e->create(treeText_, precision_))) return rc;
+      e->reduce_ = false;
+      e->matricesOnly_ = true;
+      e->graph_ = false;
+      e->tuning_ = false;
+      e->splitWaves_ = splitWaves_;
+      e->splitMinK_ = splitMinK_;
+      e->gmSplitK_ = gmSplitK_;
+      e->gcLongK_ = gcLongK_;
+      e->fuseHoles_ = fuseHoles_;
+      e->sop_ = sop_;
+      e->sop_.terms.assign(sop_.terms.begin() + terms0_, sop_.terms.begin() + std::min(L, terms0_ + n));
+      rc = e->plan();
+      if (rc == QTG_ENOMEM && n > 1) continue;
+      if (rc) return rc;
+      terms_ = std::move(e);
+      termsN_ = n;
+      termsBuild_ = -1;
+      break;
+    }
   }
-  if (fullBuild_ == builds_) return QTG_OK;
+  if (termsBuild_ == builds_) return QTG_OK;
   if (heevPending_) QTG_HIP_TRY(hipStreamWaitEvent(s, evHeev_, 0));  // the copy runs before it
   QTG_HIP_TRY(hipStreamSynchronize(s));
-  full_->eps_ = eps_;
-  if ((rc = full_->set_psi_device(d_psiBuilt_, full_->stream_))) return rc;
-  if ((rc = full_->build(full_->stream_))) return rc;
-  if ((rc = full_->synchronize())) return rc;
-  fullBuild_ = builds_;
+  terms_->eps_ = eps_;
+  if ((rc = terms_->set_psi_device(d_psiBuilt_, terms_->stream_))) return rc;
+  if ((rc = terms_->build(terms_->stream_))) return rc;
+  if ((rc = terms_->synchronize())) return rc;
+  termsBuild_ = builds_;
   return QTG_OK;
 }
 
@@ -1111,9 +1133,9 @@ int Engine::get_matrix(int which, int term, int node, double* out, hipStream_t s
     off = (which == 2) ? hslot_[term][node] : holeslot_[term][node];
   }
   if (off < 0) return QTG_EARG;
-  if (which >= 2 && reduced()) {
-    const int rc = full_engine(s);
-    return rc ? rc : full_->get_matrix(which, term, node, out, full_->stream_);
+  if (which >= 2 && reduced() && !formed_.count(off)) {
+    const int rc = term_engine(term, s);
+    return rc ? rc : terms_->get_matrix(which, term - terms0_, node, out, terms_->stream_);
   }
   if (heevPending_) QTG_HIP_TRY(hipStreamWaitEvent(s, evHeev_, 0));  // rho^-1 of the side stream
   if (from64 || !c64_ || path_ == 1) {

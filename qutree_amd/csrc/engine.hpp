@@ -251,13 +251,18 @@ class Engine {
   void want(const SlotRef& slot, int64_t id, bool early, bool hard);
   void reduce_plan(const std::vector<std::vector<std::pair<int64_t, int>>>& hent,
                    const std::vector<std::vector<std::pair<int64_t, int>>>& qent, int64_t& off);
-  // Matrices of single terms for get_matrix: an engine of the same tree and
-  // Hamiltonian that forms all of them, run on the state of the last build
-  // (d_psiBuilt_, copied beside the eigensolver) when one is asked for.
-  std::unique_ptr<Engine> full_;
+  // Matrices of single terms for get_matrix: those that the reduced sweep
+  // forms by themselves (formed_: pool offsets) are read from it; for the rest
+  // an engine of the same tree and a group of the terms forms all of theirs,
+  // run on the state of the last build (d_psiBuilt_, copied beside the
+  // eigensolver) when one is asked for.
+  std::set<int64_t> formed_;
+  std::unique_ptr<Engine> terms_;
+  bool matricesOnly_ = false;  // such an engine: build() ends with the holes
+  int terms0_ = 0, termsN_ = 0, termsCap_ = 0;  // its first term, group size, largest that fits
   double* d_psiBuilt_ = nullptr;
-  int64_t builds_ = 0, fullBuild_ = -1;
-  int full_engine(hipStream_t s);
+  int64_t builds_ = 0, termsBuild_ = -1;
+  int term_engine(int term, hipStream_t s);
   int before_psi_write(hipStream_t s);
   std::vector<Summand> aggregate(const std::vector<Summand>& tl, const std::vector<int>& sdim, int64_t& off,
                                  double& combFlops);

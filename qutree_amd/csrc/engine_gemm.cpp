@@ -1335,11 +1335,16 @@ int Engine::build_gemm(hipStream_t s) {
   void* bases[B_COUNT] = {d_psi32_, d_work32_, d_pool_, d_psi64_, d_apply64_, d_dpsi64_, d_pool64_, d_work_};
   // represent and the density tree, layer by layer in shared launches
   if ((rc = run_launches(gBuild_, bases, nullptr, 1.0, 0.0, s))) return rc;
-  // the state that get_matrix forms single terms' matrices from (full_engine)
+  // the state that get_matrix forms single terms' matrices from (term_engine)
   auto keep_state = [&](hipStream_t t) {
     return d_psiBuilt_ ? launch_copy_vec(d_psi64_, d_psiBuilt_, 2 * tree_.total, t) : (int)QTG_OK;
   };
   ++builds_;
+  if (matricesOnly_) {
+    if ((rc = run_launches(gHole_, bases, nullptr, 1.0, 0.0, s))) return rc;
+    built_ = true;
+    return QTG_OK;
+  }
   if (heevSide_) {
     // side stream: the eigensolver (it only feeds the solve of the finish,
     // which apply_gemm makes wait for it); engine stream: the holes, the

@@ -23,7 +23,7 @@
 // h-matrices (which no hole reads); the combinations of holes; Apply.
 //
 // Per-term matrices that no sum needs are not formed in a sweep;
-// qtg_engine_get_matrix forms them when it is asked for one (full_engine).
+// qtg_engine_get_matrix forms them when it is asked for one (term_engine).
 #include <algorithm>
 #include <map>
 

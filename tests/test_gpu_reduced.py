@@ -247,3 +247,29 @@ def test_reduced_precision_forms_lose_none_to_the_sums(name, monkeypatch):
         err[form] = _apply_rms(text, H, precision, seeds)
         print(f"  {form} {err[form]:.3e}", flush=True)
     assert err["reduced"] < 1.005 * err["every matrix"]
+
+
+@pytest.mark.parametrize("precision,tol", [(0, 1e-11), (1, 1e-4)])
+def test_matrices_of_all_terms_in_any_order(precision, tol, every_size):
+    """Every term's matrices from the growing groups of get_matrix, asked for
+    in random order and after several builds, against the engine that forms
+    all of them (complex64: 100 times the rounding of its sums, for the
+    amplification along the tree)."""
+    text, H = _models()["quartic16"]
+    print(f"case matrices of all terms precision={precision}", flush=True)
+    full = Q.Engine(text, H, compress=False)
+    eng = Q.Engine(text, H, precision=precision)
+    rng = np.random.default_rng(5)
+    om = O.OracleModel(text, H)
+    act = [(l, a) for l in range(H.nterms) for a in om.sparse_tree(l) if a != om.nnodes - 1]
+    for seed in (1, 2):
+        psi = full.fill_random(seed, delta_lowest=False)
+        full.set_psi(psi)
+        full.derivative()
+        eng.set_psi(psi)
+        eng.derivative()
+        for i in rng.permutation(len(act)):
+            l, a = act[i]
+            for which in (2, 3):
+                ref = full.matrix(which, l, a)
+                assert np.max(np.abs(eng.matrix(which, l, a) - ref)) < tol * max(1, np.max(np.abs(ref)))
