@@ -264,7 +264,9 @@ __device__ inline GmTile gm_tile_lean(const GmDesc& d, uint32_t t) {
 // one accumulator pair (the MFMAs of a k-step alternate between the real and
 // imaginary part, and consecutive MFMAs into the same accumulator chain
 // without a stall); ACC 2, a single product: every other k-step has a pair of
-// its own, as in gm_product, whose rounding it keeps.
+// its own, as in gm_product, whose rounding it keeps, as it keeps infinities:
+// the K tail is zeroed on both operands (zero times the clamped last k's
+// infinity is a NaN).
 template <typename T, typename TM, bool TR, bool CONJ, int ACC>
 __device__ inline void gm_lean_loop(const cplx<T>* __restrict__ xa, uint32_t xrow, uint32_t bef,
                                     const cplx<TM>* __restrict__ mb, uint32_t mrow, uint32_t mks, int kbeg, int kend,
@@ -280,6 +282,7 @@ __device__ inline void gm_lean_loop(const cplx<T>* __restrict__ xa, uint32_t xro
       const cplx<TM> m = ld32(mb, mrow + kc * mks);
       xv[u] = mk<T>(kv ? x.re : (T)0, kv ? x.im : (T)0);
       mv[u] = mk<T>((T)m.re, CONJ ? -(T)m.im : (T)m.im);
+      if (ACC == 2) mv[u] = mk<T>(kv ? mv[u].re : (T)0, kv ? mv[u].im : (T)0);
     }
     // every operand is taken here, so the compiler keeps the eight loads
     // together ahead of the MFMAs instead of sinking them into the k-step

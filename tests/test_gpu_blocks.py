@@ -152,3 +152,69 @@ def test_product_plan(c64):
         if d["add"][i]:
             ref = ref + C0[oT[i]:oT[i + 1]]
         close(got[oT[i]:oT[i + 1]], ref, n, c64)
+
+
+def _same_infinities(got, ref):
+    """Infinities of the same sign at the same places, no NaN, the rest finite
+    and equal to rounding."""
+    for g, r in ((got.real, ref.real), (got.imag, ref.imag)):
+        inf = np.isinf(r)
+        assert not np.isnan(g).any()
+        assert np.array_equal(np.isinf(g), inf)
+        assert np.array_equal(np.sign(g[inf]), np.sign(r[inf]))
+        assert np.allclose(g[~inf], r[~inf], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("c64", [False, True])
+@pytest.mark.parametrize("op", [0, 1, 2])
+@pytest.mark.parametrize("before", [1, 5])
+@pytest.mark.parametrize("nB", [3, 5, 6, 8, 17, 31])
+def test_single_product_infinity_in_the_last_column(nB, before, op, c64):
+    """An infinite entry of op(M) that meets the last k: reductions that end
+    within a k-step of four must not make a NaN of it."""
+    print(f"case product infinity {nB} {before} op={op} c64={c64}", flush=True)
+    rng = np.random.default_rng(nB)
+    nC, after = 7, 9
+    B, M = rand(rng, (after, nB, before), c64), rand(rng, (nC, nB), c64)  # M: op(M), row i, column l
+    M[3, nB - 1] = np.inf
+    stored = (M, M.T, M.conj().T)[op]
+    x, m = B.astype(np.complex128), M.astype(np.complex128)
+    re, im = (np.zeros((after, nC, before)) for _ in range(2))
+    for l in range(nB):
+        xr, xi, mr, mi = x[:, l, None, :].real, x[:, l, None, :].imag, m[None, :, l, None].real, m[None, :, l, None].imag
+        re += xr * mr - xi * mi
+        im += xr * mi + xi * mr
+    dB = Q.DeviceBuffer.from_array(B)
+    dM = Q.DeviceBuffer.from_array(np.asfortranarray(stored).T)  # column-major
+    dC = Q.DeviceBuffer(B.itemsize * after * nC * before)
+    fn = Q.lib().qtg_mode_product_c if c64 else Q.lib().qtg_mode_product_z
+    Q.check(fn(dC.ptr, dM.ptr, dB.ptr, before, nB, nC, after, op, 0, None))
+    got = dC.download(B.dtype).reshape(after, nC, before)
+    assert np.isinf(re).any() and np.isinf(im).any()
+    _same_infinities(got, _complex(re, im))
+
+
+def _complex(re, im):
+    z = np.empty(re.shape, np.complex128)
+    z.real, z.imag = re, im
+    return z
+
+
+@pytest.mark.parametrize("c64", [False, True])
+@pytest.mark.parametrize("before,after", [(1, 3), (5, 13), (3, 257), (7, 1001)])
+def test_single_hole_contraction_infinity_in_the_last_row(before, after, c64):
+    print(f"case hole infinity {before} {after} c64={c64}", flush=True)
+    rng = np.random.default_rng(before)
+    nA, nB = 6, 19
+    A, B = rand(rng, (after, nA, before), c64), rand(rng, (after, nB, before), c64)
+    A[-1, 2, -1] = np.inf
+    x, y = (v.astype(np.complex128).transpose(0, 2, 1).reshape(after * before, -1) for v in (A, B))
+    re, im = (np.zeros((nB, nA)) for _ in range(2))
+    for k in range(after * before):
+        a, b = x[k][None, :], y[k][:, None]
+        re += a.real * b.real + a.imag * b.imag
+        im += a.real * b.imag - a.imag * b.real
+    dA, dB, dS = Q.DeviceBuffer.from_array(A), Q.DeviceBuffer.from_array(B), Q.DeviceBuffer(A.itemsize * nA * nB)
+    fn = Q.lib().qtg_hole_contraction_c if c64 else Q.lib().qtg_hole_contraction_z
+    Q.check(fn(dS.ptr, dA.ptr, dB.ptr, before, nA, nB, after, 0, None))
+    _same_infinities(dS.download(A.dtype).reshape(nB, nA), _complex(re, im))
