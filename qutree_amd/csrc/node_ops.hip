@@ -361,37 +361,62 @@ int scratch_address(void** out) {
 // The slots of part_scratch, per device.  A call holds the lock while it
 // enqueues its two launches and records the slot's event behind them; the
 // next user of a slot, on whatever stream and thread, makes its stream wait
-// for that event unless it has passed.  Nothing is allocated but the events.
+// for that event.  A stream keeps to the slot it used last, another takes the
+// one used longest ago.  (Asking whether an event has passed would end a
+// capture that is open on any other stream of the thread.)  Nothing is
+// allocated but the events.
 struct PartPool {
   std::mutex mu;
   void* base[kMaxDevices] = {};
   hipEvent_t ev[kMaxDevices][kPartSlots] = {};
-  bool used[kMaxDevices][kPartSlots] = {};
-  unsigned next[kMaxDevices] = {};
+  hipStream_t last[kMaxDevices][kPartSlots] = {};
+  uint64_t use[kMaxDevices][kPartSlots] = {};  // 0: never
+  uint64_t uses = 0;
 };
 PartPool g_parts;
+
+// the array's address and the slots' events, which the first call makes (with
+// captures on other streams left alone by it)
+int part_slots(int dev, void** base) {
+  if (g_parts.base[dev] && g_parts.ev[dev][kPartSlots - 1]) {
+    *base = g_parts.base[dev];
+    return QTG_OK;
+  }
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  QTG_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  int rc = symbol_address(HIP_SYMBOL(part_scratch), dev, g_parts.base, "hole contraction", base);
+  for (int i = 0; i < kPartSlots && !rc; ++i)
+    if (!g_parts.ev[dev][i] &&
+        hipEventCreateWithFlags(&g_parts.ev[dev][i], hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      g_parts.ev[dev][i] = nullptr;
+      set_error("hole contraction: hipEventCreate failed");
+      rc = QTG_EDEVICE;
+    }
+  QTG_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  return rc;
+}
 
 template <typename R>
 int hole_split(const GcDesc& g, const GcOnePlan& p, const cplx<R>* A, const cplx<R>* B, cplx<R>* Sm, hipStream_t s) {
   int dev = 0;
   QTG_HIP_TRY(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDevices) {
+    set_error("hole contraction: device index out of range");
+    return QTG_EDEVICE;
+  }
   std::lock_guard<std::mutex> lock(g_parts.mu);
   void* base = nullptr;
-  int rc = symbol_address(HIP_SYMBOL(part_scratch), dev, g_parts.base, "hole contraction", &base);
+  int rc = part_slots(dev, &base);
   if (rc) return rc;
-  // a slot whose last use has ended, else the one used longest ago
-  int slot = -1;
-  for (int i = 0; i < kPartSlots && slot < 0; ++i)
-    if (!g_parts.used[dev][i] || hipEventQuery(g_parts.ev[dev][i]) == hipSuccess) slot = i;
-  (void)hipGetLastError();  // hipErrorNotReady of a query
-  if (slot < 0) {
-    slot = (int)(g_parts.next[dev] % kPartSlots);
-    QTG_HIP_TRY(hipStreamWaitEvent(s, g_parts.ev[dev][slot], 0));
-  }
-  g_parts.next[dev] = (unsigned)slot + 1;
-  if (!g_parts.ev[dev][slot])
-    QTG_HIP_TRY(hipEventCreateWithFlags(&g_parts.ev[dev][slot], hipEventDisableTiming));
-  g_parts.used[dev][slot] = true;
+  int slot = 0;
+  for (int i = 1; i < kPartSlots; ++i)
+    if (g_parts.use[dev][i] < g_parts.use[dev][slot]) slot = i;
+  for (int i = 0; i < kPartSlots; ++i)
+    if (g_parts.use[dev][i] && g_parts.last[dev][i] == s) slot = i;
+  if (g_parts.use[dev][slot]) QTG_HIP_TRY(hipStreamWaitEvent(s, g_parts.ev[dev][slot], 0));
+  g_parts.use[dev][slot] = ++g_parts.uses;
+  g_parts.last[dev][slot] = s;
   rc = launch_gc_one<R>(g, p, A, B, Sm, static_cast<unsigned char*>(base) + (size_t)slot * kPartBytes, s);
   // also after a failed launch: the first of the two may run
   const hipError_t e = hipEventRecord(g_parts.ev[dev][slot], s);
@@ -408,12 +433,16 @@ template <typename F>
 int with_all_parts(hipStream_t s, F&& launch) {
   int dev = 0;
   QTG_HIP_TRY(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDevices) {
+    set_error("hole contraction: device index out of range");
+    return QTG_EDEVICE;
+  }
   std::lock_guard<std::mutex> lock(g_parts.mu);
   void* base = nullptr;
-  int rc = symbol_address(HIP_SYMBOL(part_scratch), dev, g_parts.base, "hole contraction", &base);
+  int rc = part_slots(dev, &base);
   if (rc) return rc;
   for (int i = 0; i < kPartSlots; ++i)
-    if (g_parts.used[dev][i]) QTG_HIP_TRY(hipStreamWaitEvent(s, g_parts.ev[dev][i], 0));
+    if (g_parts.use[dev][i]) QTG_HIP_TRY(hipStreamWaitEvent(s, g_parts.ev[dev][i], 0));
   return launch(base);
 }
 

@@ -218,3 +218,149 @@ def test_single_hole_contraction_infinity_in_the_last_row(before, after, c64):
     fn = Q.lib().qtg_hole_contraction_c if c64 else Q.lib().qtg_hole_contraction_z
     Q.check(fn(dS.ptr, dA.ptr, dB.ptr, before, nA, nB, after, 0, None))
     _same_infinities(dS.download(A.dtype).reshape(nB, nA), _complex(re, im))
+
+
+class _Hip:
+    """The HIP runtime calls of a stream capture (the library the engine is
+    linked to)."""
+
+    def __init__(self):
+        import ctypes as C
+        self.C, self.L = C, C.CDLL("libamdhip64.so.7")
+        self.check(self.L.hipInit(0))
+
+    @staticmethod
+    def check(rc):
+        assert rc == 0, f"hip error {rc}"
+
+    def begin(self, stream, mode):
+        self.check(self.L.hipStreamBeginCapture(stream, mode))
+
+    def end(self, stream):
+        g, x = self.C.c_void_p(), self.C.c_void_p()
+        self.check(self.L.hipStreamEndCapture(stream, self.C.byref(g)))
+        self.check(self.L.hipGraphInstantiate(self.C.byref(x), g, None, None, self.C.c_size_t(0)))
+        self.check(self.L.hipGraphDestroy(g))
+        return x
+
+    def launch(self, graph, stream):
+        self.check(self.L.hipGraphLaunch(graph, stream))
+
+    def destroy(self, graph):
+        self.check(self.L.hipGraphExecDestroy(graph))
+
+
+def _streams(n):
+    import ctypes as C
+    out = []
+    for _ in range(n):
+        s = C.c_void_p()
+        Q.check(Q.lib().qtg_stream_create(C.byref(s)))
+        out.append(s)
+    return out
+
+
+def _hole_refs(shapes, oT, A, B):
+    refs = []
+    for i, (b, n, a) in enumerate(shapes):
+        x, y = (v[oT[i]:oT[i + 1]].reshape(a, n, b).astype(np.complex128) for v in (A, B))
+        refs.append(np.einsum("ajb,alb->lj", x.conj(), y, optimize=True).ravel())
+    return refs
+
+
+def _hole_plan(shapes, oT, oM, c64):
+    d = np.zeros(len(shapes), Q.HC_DESC)
+    d["offS"], d["offA"], d["offB"] = oM[:-1], oT[:-1], oT[:-1]
+    d["before"], d["after"] = [s[0] for s in shapes], [s[2] for s in shapes]
+    d["nA"] = d["nB"] = [s[1] for s in shapes]
+    return Q.Plan("hole_contraction", d, complex64=c64)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])  # global, thread-local, relaxed
+@pytest.mark.parametrize("c64", [False, True])
+@pytest.mark.parametrize("name", ["one_long", "mixed"])
+def test_captured_plan_and_long_contraction(name, c64, mode):
+    """Under capture a plan with shared reductions runs its unshared tables and
+    a long single contraction takes one workgroup a tile: a replay cannot be
+    ordered with other users of the partial tiles.  Replays with eager
+    executions of the same plan and of another long contraction on another
+    stream in between, and one such call while the capture is open."""
+    print(f"case captured plan {name} c64={c64} mode={mode}", flush=True)
+    hip, shapes = _Hip(), HOLE_PLANS[name]
+    rng = np.random.default_rng(len(shapes) + 7)
+    A, B, _, oT, oM, es = _plan_case(rng, shapes, c64)
+    plan = _hole_plan(shapes, oT, oM, c64)
+    b1, n1, a1 = 40, 33, 500  # the single contraction: 20000 long
+    X, Y = rand(rng, (a1, n1, b1), c64), rand(rng, (a1, n1, b1), c64)
+    fn = Q.lib().qtg_hole_contraction_c if c64 else Q.lib().qtg_hole_contraction_z
+    dA, dB, dX, dY = (Q.DeviceBuffer.from_array(x) for x in (A, B, X, Y))
+    item = np.dtype(es).itemsize
+    outs = [Q.DeviceBuffer(item * int(oM[-1])) for _ in range(2)]  # captured, eager
+    singles = [Q.DeviceBuffer(item * n1 * n1) for _ in range(2)]
+    s, other = _streams(2)
+
+    def plan_on(out, stream):
+        Q.check(Q.lib().qtg_plan_execute(plan.ptr, out.ptr, dA.ptr, dB.ptr, stream))
+
+    def single_on(out, stream):
+        Q.check(fn(out.ptr, dX.ptr, dY.ptr, b1, n1, n1, a1, 0, stream))
+
+    plan_on(outs[1], s)  # once outside
+    single_on(singles[1], other)
+    Q.synchronize()
+    hip.begin(s, mode)
+    plan_on(outs[0], s)
+    single_on(singles[0], s)
+    single_on(singles[1], other)  # not captured
+    graph = hip.end(s)
+    for r in range(4):
+        X, Y, A, B = (v * es(1 + r) for v in (X, Y, A, B))
+        for d, v in ((dA, A), (dB, B), (dX, X), (dY, Y)):
+            d.upload(v)
+        for d in outs + singles:
+            d.zero()
+        Q.synchronize()
+        hip.launch(graph, s)
+        plan_on(outs[1], other)
+        single_on(singles[1], other)
+        hip.launch(graph, s)
+        Q.synchronize()
+        ref = _hole_refs(shapes, oT, A, B)
+        one = np.einsum("ajb,alb->lj", X.conj().astype(np.complex128), Y.astype(np.complex128), optimize=True)
+        for d in outs:
+            got = d.download(es)
+            for i, (b, n, a) in enumerate(shapes):
+                close(got[oM[i]:oM[i + 1]], ref[i], b * a, c64)
+        for d in singles:
+            close(d.download(es).reshape(n1, n1), one, b1 * a1, c64)
+    hip.destroy(graph)
+    for st in (s, other):
+        Q.check(Q.lib().qtg_stream_destroy(st))
+
+
+@pytest.mark.parametrize("name", ["one_long", "mixed"])
+def test_one_plan_on_two_streams(name):
+    """Executions of one plan with shared reductions alternate over two
+    streams with operands and outputs of their own; they share the plan's
+    partial tiles."""
+    print(f"case one plan on two streams {name}", flush=True)
+    shapes = HOLE_PLANS[name]
+    rng = np.random.default_rng(3)
+    sets = []
+    for _ in range(4):
+        A, B, _, oT, oM, es = _plan_case(rng, shapes, False)
+        sets.append((A, B, Q.DeviceBuffer.from_array(A), Q.DeviceBuffer.from_array(B)))
+    plan = _hole_plan(shapes, oT, oM, False)
+    streams = _streams(2)
+    outs = [Q.DeviceBuffer(16 * int(oM[-1])) for _ in range(24)]
+    for i, o in enumerate(outs):
+        Q.check(Q.lib().qtg_plan_execute(plan.ptr, o.ptr, sets[i % 4][2].ptr, sets[i % 4][3].ptr,
+                                         streams[(i + i // 4) % 2]))
+    Q.synchronize()
+    refs = [_hole_refs(shapes, oT, A, B) for A, B, _, _ in sets]
+    for i, o in enumerate(outs):
+        got = o.download(np.complex128)
+        for k, (b, n, a) in enumerate(shapes):
+            close(got[oM[k]:oM[k + 1]], refs[i % 4][k], b * a, False)
+    for s in streams:
+        Q.check(Q.lib().qtg_stream_destroy(s))
