@@ -280,9 +280,17 @@ __device__ inline void gm_lean_loop(const cplx<T>* __restrict__ xa, uint32_t xro
       const uint32_t kc = (uint32_t)(kv ? kx : kend - 1);
       const cplx<T> x = ld32(xa, xrow + kc * bef);
       const cplx<TM> m = ld32(mb, mrow + kc * mks);
-      xv[u] = mk<T>(kv ? x.re : (T)0, kv ? x.im : (T)0);
+      const bool xk = ACC == 2 || kv;
+      xv[u] = mk<T>(xk ? x.re : (T)0, xk ? x.im : (T)0);
       mv[u] = mk<T>((T)m.re, CONJ ? -(T)m.im : (T)m.im);
-      if (ACC == 2) mv[u] = mk<T>(kv ? mv[u].re : (T)0, kv ? mv[u].im : (T)0);
+    }
+    if (ACC == 2 && k0 + 16 > kend) {  // the last k-steps (uniform)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool kv = k0 + 4 * u + kk < kend;
+        xv[u] = mk<T>(kv ? xv[u].re : (T)0, kv ? xv[u].im : (T)0);
+        mv[u] = mk<T>(kv ? mv[u].re : (T)0, kv ? mv[u].im : (T)0);
+      }
     }
     // every operand is taken here, so the compiler keeps the eight loads
     // together ahead of the MFMAs instead of sinking them into the k-step
