@@ -370,8 +370,9 @@ int Engine::plan_gemm() {
       app(out.con[hp], sd[hp].con);
     }
   };
-  // The summed contractions of a layer and precision, one launch for the
-  // matrices of up to 16 x 16 and one for the larger.  A reduction beyond
+  // The summed contractions of a layer and precision: one launch in 16 x 16
+  // tiles, and one in macro tiles for the matrices beyond 16 x 16 of a layer
+  // whose tiles and shares exceed 1024 workgroups.  A reduction beyond
   // `whole` elements is shared by workgroups of `share` each, whose partial
   // tiles a further launch adds: the top's children of the 64-mode tree
   // (K = 18 x 196) would hold one CU for 23 us.

@@ -160,9 +160,9 @@ void Engine::want(const SlotRef& slot, int64_t id, bool early, bool hard) {
 }
 
 // Chooses, for every node, the single matrices and the summed ones that the
-// wanted Apply and gradient summands need, and emits them: redItems_ (the
-// kept items of h_items_, by layer), fused_ (summed contractions) and the
-// combinations h_combA_ (sums of h-matrices) and h_comb1_ (sums of holes).
+// wanted Apply and gradient summands need: hWant_ and qWant_ (by which plan()
+// keeps items of h_items_), fused_ (summed contractions) and the combinations
+// h_combA_ (sums of h-matrices) and h_comb1_ (sums of holes).
 void Engine::reduce_plan(const std::vector<std::vector<std::pair<int64_t, int>>>& hent,
                          const std::vector<std::vector<std::pair<int64_t, int>>>& qent, int64_t& off) {
   const int NN = (int)tree_.nodes.size();

@@ -372,15 +372,15 @@ __global__ void __launch_bounds__(256)
 }
 
 // ------------------------------------------------------------- mode product
-// out(b,i,a) = alpha sum_l op(M)(i,l) X(b,l,a) (+ out) on RB x CB tiles of
+// out(b,i,a) = sum_l op(M)(i,l) X(b,l,a) (+ out) on RB x CB tiles of
 // 16 rows (flattened (b, a)) x 16 columns i, KS k-steps of four per stage,
 // staged as in gc_block_product.  TR (bef >= 4): accumulated transposed, so a
 // lane holds one row and the 16 lanes of a store write 16 consecutive
 // elements.  Rows and columns past the range are clamped into it (never
 // stored); the last, partial stage masks X past K.
-template <typename T, typename TM, typename TO, int RB, int CB, int KS, bool TR>
+template <typename T, int RB, int CB, int KS, bool TR>
 __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, const cplx<T>* __restrict__ X,
-                                      const cplx<TM>* __restrict__ M, cplx<TO>* O, double sre, double sim) {
+                                      const cplx<T>* __restrict__ M, cplx<T>* O) {
   typedef typename MF<T>::v4 v4;
   const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
   const uint32_t bef = (uint32_t)d.bef, R = bef * (uint32_t)d.aft;
@@ -400,13 +400,13 @@ __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, cons
     mrow[t] = d.op == GM_N ? (uint32_t)j : (uint32_t)j * (uint32_t)nin;
   }
   const cplx<T>* xp = X + d.x;
-  const cplx<TM>* mp = M + d.m;
+  const cplx<T>* mp = M + d.m;
   v4 cr[RB][CB], ci[RB][CB];
 #pragma unroll
   for (int i = 0; i < RB; ++i)
 #pragma unroll
     for (int j = 0; j < CB; ++j) cr[i][j] = ci[i][j] = v4{0, 0, 0, 0};
-  auto load = [&](int k, cplx<T>(&xv)[KS][RB], cplx<TM>(&mv)[KS][CB]) {
+  auto load = [&](int k, cplx<T>(&xv)[KS][RB], cplx<T>(&mv)[KS][CB]) {
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
       const uint32_t kc = (uint32_t)min(k + 4 * u + kk, nin - 1);
@@ -417,10 +417,10 @@ __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, cons
       for (int t = 0; t < CB; ++t) mv[u][t] = ld32(mp, mrow[t] + om);
     }
   };
-  auto kstep = [&](const cplx<T>(&xv)[RB], const cplx<TM>(&mv)[CB]) {
+  auto kstep = [&](const cplx<T>(&xv)[RB], const cplx<T>(&mv)[CB]) {
 #pragma unroll
     for (int j = 0; j < CB; ++j) {
-      const T mr = (T)mv[j].re, mi = msign * (T)mv[j].im;
+      const T mr = mv[j].re, mi = msign * mv[j].im;
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
         const T nxi = -xv[i].im;
@@ -438,7 +438,7 @@ __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, cons
       }
     }
   };
-  auto stage = [&](int k, cplx<T>(&xv)[KS][RB], const cplx<TM>(&mv)[KS][CB]) {
+  auto stage = [&](int k, cplx<T>(&xv)[KS][RB], const cplx<T>(&mv)[KS][CB]) {
     if (k + 4 * KS <= nin) {
 #pragma unroll
       for (int u = 0; u < KS; ++u) kstep(xv[u], mv[u]);
@@ -454,7 +454,7 @@ __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, cons
     }
   };
   cplx<T> xa[KS][RB], xb[KS][RB];
-  cplx<TM> ma[KS][CB], mb[KS][CB];
+  cplx<T> ma[KS][CB], mb[KS][CB];
   load(0, xa, ma);
   for (int k = 0; k < nin; k += 8 * KS) {
     load(k + 4 * KS, xb, mb);
@@ -462,10 +462,7 @@ __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, cons
     load(k + 8 * KS, xa, ma);
     if (k + 4 * KS < nin) stage(k + 4 * KS, xb, mb);
   }
-  const double fre = d.are * sre - d.aim * sim, fim = d.are * sim + d.aim * sre;
-  const bool one = fre == 1.0 && fim == 0.0;
-  const T are = (T)fre, aim = (T)fim;
-  cplx<TO>* ob = O + d.out;
+  cplx<T>* ob = O + d.out;
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
 #pragma unroll
@@ -476,9 +473,8 @@ __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, cons
         const int col = c0 + j * 16 + (TR ? MF<T>::drow(lane, q) : li);
         if (r < R && col < nout) {
           const uint32_t a = r / bef;
-          cplx<TO>* o = at32(ob, (r - a * bef) + (uint32_t)col * bef + a * bef * (uint32_t)nout);
-          const T vr = cr[i][j][q], vi = ci[i][j][q];
-          cplx<TO> v = one ? mk<TO>((TO)vr, (TO)vi) : mk<TO>((TO)(are * vr - aim * vi), (TO)(are * vi + aim * vr));
+          cplx<T>* o = at32(ob, (r - a * bef) + (uint32_t)col * bef + a * bef * (uint32_t)nout);
+          cplx<T> v = mk<T>(cr[i][j][q], ci[i][j][q]);
           if (d.acc) v = cadd(v, *o);
           *o = v;
         }
@@ -487,30 +483,27 @@ __device__ inline void gm_block_tiles(const GmDesc& d, uint32_t r0, int c0, cons
   }
 }
 
-// Four tasks (wavefronts) per workgroup; wgdesc null: one descriptor per
-// task.  A task is 2 x 2 tiles; its last column block may hold one column.
-template <typename T, typename TM, typename TO>
+// Four tasks (wavefronts) per workgroup.  A task is 2 x 2 tiles; its last
+// column block may hold one column.
+template <typename T>
 __global__ void __launch_bounds__(256)
     gm_block(const GmDesc* __restrict__ descs, const int32_t* __restrict__ wgdesc, int64_t ntasks,
-             const cplx<T>* __restrict__ X0, const cplx<T>* __restrict__ X1, const cplx<TM>* __restrict__ M,
-             cplx<TO>* O, const uint8_t* __restrict__ active, double sre, double sim) {
+             const cplx<T>* __restrict__ X, const cplx<T>* __restrict__ M, cplx<T>* O) {
   const int64_t task = (int64_t)blockIdx.x * 4 + wave_id();
   if (task >= ntasks) return;
-  const GmDesc d = descs[wgdesc ? (int64_t)wgdesc[task] : task];
-  if (active && d.node >= 0 && !active[d.node]) return;
+  const GmDesc d = descs[wgdesc[task]];
   const uint32_t t = (uint32_t)(task - d.tile0);
   const uint32_t CT = (uint32_t)(d.nout + 31) / 32u;
   const uint32_t rt = CT == 1 ? t : t / CT;
   const int c0 = (int)(t - rt * CT) * 32;
   const uint32_t r0 = rt * 32u;
   const bool two = d.nout - c0 > 16;
-  const cplx<T>* X = d.xsel ? X1 : X0;
   if (d.bef >= 4) {
-    if (two) gm_block_tiles<T, TM, TO, 2, 2, 1, true>(d, r0, c0, X, M, O, sre, sim);
-    else gm_block_tiles<T, TM, TO, 2, 1, 1, true>(d, r0, c0, X, M, O, sre, sim);
+    if (two) gm_block_tiles<T, 2, 2, 1, true>(d, r0, c0, X, M, O);
+    else gm_block_tiles<T, 2, 1, 1, true>(d, r0, c0, X, M, O);
   } else {
-    if (two) gm_block_tiles<T, TM, TO, 2, 2, 1, false>(d, r0, c0, X, M, O, sre, sim);
-    else gm_block_tiles<T, TM, TO, 2, 1, 1, false>(d, r0, c0, X, M, O, sre, sim);
+    if (two) gm_block_tiles<T, 2, 2, 1, false>(d, r0, c0, X, M, O);
+    else gm_block_tiles<T, 2, 1, 1, false>(d, r0, c0, X, M, O);
   }
 }
 
@@ -540,23 +533,19 @@ template int launch_gc_sum<double>(int, const GcSum*, int64_t, const GcSum*, int
 template int launch_gc_sum<float>(int, const GcSum*, int64_t, const GcSum*, int64_t, const GcSeg*, const void*,
                                   const void*, void*, void*, hipStream_t, const KernelTiming*);
 
-template <typename T, typename TM, typename TO>
-int launch_gm_block(const GmDesc* descs, const int32_t* wgdesc, int64_t ntasks, const void* x0, const void* x1,
-                    const void* mbase, void* obase, const uint8_t* active, double sre, double sim, hipStream_t s,
-                    const KernelTiming* kt) {
+template <typename T>
+int launch_gm_block(const GmDesc* descs, const int32_t* wgdesc, int64_t ntasks, const void* x, const void* m, void* o,
+                    hipStream_t s) {
   if (ntasks <= 0) return QTG_OK;
-  launch_timed(gm_block<T, TM, TO>, dim3((unsigned)((ntasks + 3) / 4)), dim3(256), 0, s, kt, descs, wgdesc, ntasks,
-               (const cplx<T>*)x0, (const cplx<T>*)x1, (const cplx<TM>*)mbase, (cplx<TO>*)obase, active, sre, sim);
+  hipLaunchKernelGGL(gm_block<T>, dim3((unsigned)((ntasks + 3) / 4)), dim3(256), 0, s, descs, wgdesc, ntasks,
+                     (const cplx<T>*)x, (const cplx<T>*)m, (cplx<T>*)o);
   QTG_LAUNCH_CHECK();
   return QTG_OK;
 }
-#define QTG_GM(T, TM, TO)                                                                                       \
-  template int launch_gm_block<T, TM, TO>(const GmDesc*, const int32_t*, int64_t, const void*, const void*,      \
-                                          const void*, void*, const uint8_t*, double, double, hipStream_t,       \
-                                          const KernelTiming*);
-QTG_GM(double, double, double)
-QTG_GM(float, float, float)
-#undef QTG_GM
+template int launch_gm_block<double>(const GmDesc*, const int32_t*, int64_t, const void*, const void*, void*,
+                                     hipStream_t);
+template int launch_gm_block<float>(const GmDesc*, const int32_t*, int64_t, const void*, const void*, void*,
+                                    hipStream_t);
 
 template <typename T>
 int launch_gc_block(const GcDesc* descs, const GcBlockWg* wgs, int64_t nwg, const GcBlockWg* sums, int64_t nsums,

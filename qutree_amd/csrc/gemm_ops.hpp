@@ -162,16 +162,15 @@ int launch_gc_single(const GcDesc& d, const void* x, const void* y, void* o, hip
 
 // Register-blocked forms (gemm_block.hip) for launches that fill the card;
 // every descriptor passes gm_lean_ok / gc_lean_ok and is no GM_COPY.
-// Mode product: 32 x 32 outputs a wavefront, no K split; tile0 and the table
-// count wavefront tasks.
+// Mode product: 32 x 32 outputs a wavefront, no K split, alpha 1, no active
+// mask; tile0 and the table count wavefront tasks.
 inline int64_t gm_block_tasks(const GmDesc& d) {
   const int64_t R = (int64_t)d.bef * d.aft;
   return ((R + 31) / 32) * ((d.nout + 31) / 32);
 }
-template <typename T, typename TM, typename TO>
-int launch_gm_block(const GmDesc* descs, const int32_t* wgdesc, int64_t ntasks, const void* x0, const void* x1,
-                    const void* mbase, void* obase, const uint8_t* active, double sre, double sim, hipStream_t s,
-                    const KernelTiming* kt = nullptr);
+template <typename T>
+int launch_gm_block(const GmDesc* descs, const int32_t* wgdesc, int64_t ntasks, const void* x, const void* m, void* o,
+                    hipStream_t s);
 // Hole contraction: a workgroup per 32 x 32 macro tile and share of the
 // reduction (ksplit shares, workgroups t = macro * ksplit + share of the
 // descriptor).  A workgroup with shares writes 1024 elements at 1024 * part;
@@ -188,14 +187,13 @@ int launch_gc_block(const GcDesc* descs, const GcBlockWg* wgs, int64_t nwg, cons
                     const void* x0, const void* x1, void* obase, void* part, hipStream_t s);
 
 // One hole contraction alone on the card (gemm_block.hip), for descriptors
-// with gc_lean_ok.  S 1: a workgroup of 16 wavefronts per 16 x 16 tile, each
-// on a sixteenth of K.  S > 1: S workgroups per 32 x 32 macro tile; their
-// partial tiles (part_elems() complex elements, caller's buffer) are then
-// summed by a second launch.
+// with gc_lean_ok.  S 1: a workgroup of 16 wavefronts (4 for K up to 128) per
+// 16 x 16 tile, each on its share of K.  S > 1: S workgroups per 32 x 32 macro
+// tile; their partial tiles (1024 macro S complex elements, caller's buffer)
+// are then summed by a second launch.
 struct GcOnePlan {
   int S;
   int64_t macro;  // workgroups per share
-  int64_t part_elems() const { return S > 1 ? macro * S * 1024 : 0; }
 };
 GcOnePlan plan_gc_one(const GcDesc& d, int64_t max_part_elems);
 template <typename T>
@@ -205,12 +203,13 @@ int launch_gc_one(const GcDesc& d, const GcOnePlan& p, const void* x, const void
 // Summed hole contraction (gemm_block.hip): out(j, l) = add(j, l) + sum over
 // segments of alpha sum_{b,a} conj(X(b,j,a)) Y(b,l,a), X and Y (bef, n, aft) at
 // the segment's offsets.  Segments are added in FP64; FP32 products (T float)
-// are accumulated in FP32 within a segment only.  A GcSum is one macro tile of nt x nt 16 x 16 tiles
-// (of ceil(n / (16 nt))^2) and one of its S shares of the concatenated
-// reduction; with S > 1 the share leaves nt^2 256 elements at that many times
-// (part + share) and a second launch over one GcSum per macro tile adds them
-// in order.  nt 1: 8 wavefronts a workgroup, for n <= 16; nt 2: 4 (twice as
-// many spill registers).
+// are accumulated in FP32 within a segment only.  A GcSum is one macro tile of
+// nt x nt 16 x 16 tiles (of ceil(n / (16 nt))^2) and one of its S shares of the
+// concatenated reduction; with S > 1 the share leaves nt^2 256 elements at that
+// many times (part + share) and a second launch over one GcSum per macro tile
+// adds them in order.  nt 1: 8 wavefronts a workgroup, for n <= 16 and for
+// launches of few tiles whatever their n (Engine::plan_gemm's push_sum); nt 2:
+// 4, whose accumulators and operands take 256 registers.
 struct GcSeg {
   int64_t x, y;
   int32_t sel, pad;  // as GcDesc::sel

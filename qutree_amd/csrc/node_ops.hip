@@ -1,11 +1,12 @@
 // Node-level contractions: mode-k products (matvec/tmatvec/ctmatvec semantics
 // of LA_lib.f, matrixTensorBLAS semantics of TensorBLAS.cpp) and hole
-// contractions (rhomat / contractionBLAS), single and grouped.  All of them
-// run on the MFMA tile kernels of gemm_ops.hip: a mode product is a GEMM over
-// the flattened (before, after) rows, a hole contraction a GEMM over the
-// flattened (before, after) reduction index.  Grouped hole contractions with
-// long reductions are split along K into 2 or 4 chunks that sum in LDS inside
-// their workgroup, in chunk order (deterministic).
+// contractions (rhomat / contractionBLAS), single and grouped, all on MFMA
+// tile kernels: a mode product is a GEMM over the flattened (before, after)
+// rows, a hole contraction a GEMM over the flattened (before, after) reduction
+// index.  Where 32-bit offsets reach, hole contractions and the products of
+// large plans take the register-blocked kernels of gemm_block.hip (long
+// reductions shared by workgroups, whose partial tiles are added in order),
+// the rest those of gemm_ops.hip.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -273,8 +274,7 @@ int run_plan(Plan& p, void* out, const void* first, const void* second, hipStrea
   if (p.kind == 0) {
     // first = M base, second = B base
     const GmDesc* g = (const GmDesc*)p.d_descs;
-    rc = launch_gm_block<T, T, T>(g, (const int32_t*)p.d_block, p.block_tasks, second, second, first, out, nullptr,
-                                  1.0, 0.0, s);
+    rc = launch_gm_block<T>(g, (const int32_t*)p.d_block, p.block_tasks, second, first, out, s);
     if (rc) return rc;
     return launch_gm<T, T, T>(g + p.nblock, (const int32_t*)p.d_wg, p.ngen, p.gen_tasks, second, second, first, out,
                               nullptr, 1.0, 0.0, s, nullptr, kGemmWaves, p.gen_lean);
