@@ -531,14 +531,14 @@ int Engine::plan() {
   formed_.clear();
   // A plan whose single matrices cost less than kReduceFlops keeps them all:
   // there the launches decide, and the summed contractions add one (the sums
-  // of h-matrices) and fuse no hole layer.  Sweeps measured on both sides:
-  // 0.03 and 0.2 GFLOP 0.99 and 0.97 times as fast reduced, 0.94 GFLOP 1.08,
-  // 3.3 GFLOP (the 64-mode tree) 1.15, 532 GFLOP (the 128-mode tree) 3.3.
-  // The reduced-precision forms mix sums in FP64 with single matrices in FP32,
-  // in more launches: complex64 / split 1.7 GFLOP (32 oscillators) 0.94 / 0.98,
-  // 3.3 GFLOP 1.09 / 1.09, 532 GFLOP 3.5 / 3.7.
+  // of h-matrices) and fuse no hole layer.  A sweep's time with every matrix
+  // over its time reduced, complex128 / complex64 / split: 0.02 GFLOP
+  // 0.95 / 1.00 / 1.02, 0.2 GFLOP 0.92 / 0.92 / 0.96, 0.8 GFLOP
+  // 0.96 / 0.93 / 0.96, 1.7 GFLOP (32 modes, SPF 16) 0.97 / 0.94 / 0.97,
+  // 3.3 GFLOP (the 64-mode tree) 1.16 / 1.08 / 1.08, 532 GFLOP (the 128-mode
+  // tree) 2.8 / 3.5 / 3.7.
   // (QTG_REDUCE_MIN_FLOPS moves the line, for tests.)
-  const double kReduceFlops = precision_ == 0 ? 5e8 : 2.5e9;
+  constexpr double kReduceFlops = 2.5e9;
   const char* rmin = std::getenv("QTG_REDUCE_MIN_FLOPS");
   if (reduced() && flops_ < (rmin ? std::atof(rmin) : kReduceFlops)) {
     planSmall_ = true;

@@ -136,11 +136,12 @@ def test_reduced_gradient_and_split_precision(name, every_size):
 
 
 @pytest.mark.parametrize("order", ["large_small", "small_large", "large_small_large"])
-def test_second_hamiltonian_on_the_other_side_of_the_line(order):
+def test_second_hamiltonian_on_the_other_side_of_the_line(order, monkeypatch):
     """One engine, Hamiltonians whose plans are reduced (large: 0.78 GFLOP of
     single matrices) and are not (small: 0.18) one after the other: buffers
     that only one of the plans has are not used by the other, and every matrix
     is that of the plan at hand."""
+    monkeypatch.setenv("QTG_REDUCE_MIN_FLOPS", "5e8")
     print(f"case second hamiltonian {order}", flush=True)
     text = W.balanced_tree_text(16, 6, [5, 14, 20, 20])
     models = {"large": W.coupled_quartic(16, 5, c_sigma=0.01), "small": _one_mode(16)}
