@@ -338,12 +338,13 @@ def test_captured_plan_and_long_contraction(name, c64, mode):
         Q.check(Q.lib().qtg_stream_destroy(st))
 
 
+@pytest.mark.parametrize("nstreams", [2, 6])  # fewer and more than sets of partial tiles
 @pytest.mark.parametrize("name", ["one_long", "mixed"])
-def test_one_plan_on_two_streams(name):
-    """Executions of one plan with shared reductions alternate over two
-    streams with operands and outputs of their own; they share the plan's
-    partial tiles."""
-    print(f"case one plan on two streams {name}", flush=True)
+def test_one_plan_on_several_streams(name, nstreams):
+    """Executions of one plan with shared reductions alternate over streams
+    with operands and outputs of their own; they share the plan's partial
+    tiles."""
+    print(f"case one plan on {nstreams} streams {name}", flush=True)
     shapes = HOLE_PLANS[name]
     rng = np.random.default_rng(3)
     sets = []
@@ -351,11 +352,11 @@ def test_one_plan_on_two_streams(name):
         A, B, _, oT, oM, es = _plan_case(rng, shapes, False)
         sets.append((A, B, Q.DeviceBuffer.from_array(A), Q.DeviceBuffer.from_array(B)))
     plan = _hole_plan(shapes, oT, oM, False)
-    streams = _streams(2)
-    outs = [Q.DeviceBuffer(16 * int(oM[-1])) for _ in range(24)]
+    streams = _streams(nstreams)
+    outs = [Q.DeviceBuffer(16 * int(oM[-1])) for _ in range(40)]
     for i, o in enumerate(outs):
         Q.check(Q.lib().qtg_plan_execute(plan.ptr, o.ptr, sets[i % 4][2].ptr, sets[i % 4][3].ptr,
-                                         streams[(i + i // 4) % 2]))
+                                         streams[(i + i // 4) % nstreams]))
     Q.synchronize()
     refs = [_hole_refs(shapes, oT, A, B) for A, B, _, _ in sets]
     for i, o in enumerate(outs):
