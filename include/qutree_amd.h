@@ -124,6 +124,10 @@ typedef struct {
   int64_t before, nA, nB, after;
   int32_t accumulate, pad;
 } qtg_hole_contraction_desc;
+/* A hole plan with long reductions holds partial tiles of them besides its
+ * tables (at most 32 MiB, until qtg_plan_destroy).  Executions of one plan may
+ * overlap on several streams; under stream capture it runs without the
+ * partial tiles. */
 typedef void* qtg_plan;
 int qtg_mode_product_plan_create(qtg_plan* plan, const qtg_mode_product_desc* descs, int64_t count,
                                  int complex64);
@@ -163,7 +167,7 @@ int qtg_qr_batch_z(const double* A, double* Q, int64_t m, int64_t n, int64_t cou
  * hole contractions as qtg_hole_contraction_plan_create + qtg_plan_execute
  * (complex128; X from A_base, Y from B_base, offsets in complex elements),
  * but the descriptor tables and partial tiles are staged in fixed device
- * arrays of the library (about 4.6 MB and 16 MB per GPU, held until the
+ * arrays of the library (about 4.6 MB and 32 MB per GPU, held until the
  * process ends) instead of a plan's allocation: at most 4096 descriptors and
  * 2^18 16 x 16 output tiles, a reduction beyond 1024 counting four-fold
  * (QTG_ESHAPE beyond).  Allocates no device memory; returns when the result

@@ -344,7 +344,7 @@ static_assert(kNoAllocTableOff % 256 == 0, "table alignment");
 static __device__ __align__(256) unsigned char scratch[qtg::kNoAllocBytes];
 // Partial tiles of single hole contractions split over workgroups, in slots
 // (see PartPool): 8 MiB hold the 128 shares of a 64 x 64 complex128 output.
-constexpr int kPartSlots = 2;
+constexpr int kPartSlots = 4;
 constexpr size_t kPartBytes = (size_t)8 << 20;
 static __device__ __align__(256) unsigned char part_scratch[kPartSlots * kPartBytes];
 

@@ -47,7 +47,7 @@ def test_single_hole_contraction(before, nA, nB, after, c64):
 
 
 def test_single_hole_contraction_streams():
-    """Long reductions back to back on several streams share two slots of
+    """Long reductions back to back on several streams share four slots of
     partial tiles: every result stays that of its own operands."""
     print("case single hole on streams", flush=True)
     import ctypes as C
@@ -55,7 +55,7 @@ def test_single_hole_contraction_streams():
     before, n, after = 40, 24, 400
     L = Q.lib()
     streams = []
-    for _ in range(3):
+    for _ in range(6):
         s = C.c_void_p()
         Q.check(L.qtg_stream_create(C.byref(s)))
         streams.append(s)
@@ -64,7 +64,7 @@ def test_single_hole_contraction_streams():
     out = [Q.DeviceBuffer(16 * n * n) for _ in range(36)]
     for i in range(36):
         Q.check(L.qtg_hole_contraction_z(out[i].ptr, d[i // 6].ptr, d[i % 6].ptr, before, n, n, after, 0,
-                                         streams[i % 3]))
+                                         streams[i % 6]))
     Q.synchronize()
     first = {}
     for i in range(36):
