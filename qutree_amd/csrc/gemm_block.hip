@@ -565,22 +565,23 @@ template int launch_gc_block<double>(const GcDesc*, const GcBlockWg*, int64_t, c
 template int launch_gc_block<float>(const GcDesc*, const GcBlockWg*, int64_t, const GcBlockWg*, int64_t, const void*,
                                     const void*, void*, void*, hipStream_t);
 
-// A reduction of up to kOneWgK elements stays in one workgroup per tile: its
-// 16 wavefronts take 14 us at K = 576 (24 x 24 output), where two launches
-// take at least 14; at K = 1024 (32 x 32) 18 against 17 us, at 2048 (64 x 64)
-// 32 against 18.  Beyond it, K is split over workgroups toward 512 of them
-// (two per CU), with shares of at least 32 elements per wavefront (K = 4096,
-// 64 x 64: 18 us; shares of 64: 27) and the partial tiles within
-// max_part_elems (0: no split over workgroups).  One wavefront per tile
-// (gc_single) took 4891 us at K = 65536, 64 x 64 complex128; this takes 80,
-// of which the operands' 134 MB at the card's copy rate are 28.
-GcOnePlan plan_gc_one(const GcDesc& d, int64_t max_part_elems) {
-  constexpr int64_t kOneWgK = 768;
+// A reduction of up to oneWgK elements stays in one workgroup per tile, 16
+// wavefronts: 14.4 us at K = 512 (24 x 24 complex128 output), where two launches
+// take at least 14; beyond, its wavefronts walk a third stage, 21 us at K = 576
+// and at 768 against 14.6 and 13.7.  complex64: 10.5 us at K = 720 against
+// 12.2, 19.0 at 768 against 11.8.  Beyond it, K is split over workgroups toward
+// 512 of them (two per CU), with shares of at least 32 elements per wavefront
+// (K = 4096, 64 x 64: 15 us) and the partial tiles within max_part_elems (0: no
+// split over workgroups).  One wavefront per tile (gc_single) took 4891 us at
+// K = 65536, 64 x 64 complex128; this takes 46, of which the operands' 134 MB
+// at the card's copy rate are 28.
+GcOnePlan plan_gc_one(const GcDesc& d, bool c64, int64_t max_part_elems) {
+  const int64_t oneWgK = c64 ? 720 : 512;
   const int64_t K = (int64_t)d.bef * d.aft;
   const int64_t m2 = gc_block_macros(d);
   GcOnePlan p{};
   p.S = 1;
-  if (K > kOneWgK) {
+  if (K > oneWgK) {
     int64_t S = std::min<int64_t>((512 + m2 - 1) / m2, K / 128);
     S = std::min<int64_t>(S, max_part_elems / (m2 * 1024));
     // workgroup macro * S + s: with 8 | S the macro tiles of a share, which
