@@ -363,8 +363,8 @@ int Cmf::copy(cplx<double>* dst, const cplx<double>* src) {
 }
 
 int Cmf::build(const cplx<double>* P) {
-  int rc = E.before_psi_write(s_);
-  if (rc || (rc = copy((cplx<double>*)E.d_psi64_, P))) return rc;
+  int rc = copy((cplx<double>*)E.d_psi64_, P);
+  if (rc) return rc;
   ++nbuild_;
   return E.build(s_);
 }
@@ -1145,7 +1145,7 @@ int Cmf::eigenstate(std::vector<double>& ev) {
   const HNode& top = E.tree_.nodes[NN_ - 1];
   const int n = top.n;
   int rc;
-  if ((rc = E.before_psi_write(s_)) || (rc = copy((cplx<double>*)E.d_psi64_, P_))) return rc;
+  if ((rc = copy((cplx<double>*)E.d_psi64_, P_))) return rc;
   if ((rc = E.build(s_))) return rc;
   // phase i: D = -i * i * H Psi = H Psi
   if ((rc = apply_top(P_, 0.0, 1.0, nullptr))) return rc;

@@ -48,7 +48,7 @@ Engine::~Engine() {
   for (auto e : evpool_) (void)hipEventDestroy(e);
   if (evFork_) (void)hipEventDestroy(evFork_);
   if (evHeev_) (void)hipEventDestroy(evHeev_);
-  if (evRho_) (void)hipEventDestroy(evRho_);
+  if (evCopy_) (void)hipEventDestroy(evCopy_);
   if (side_) (void)hipStreamDestroy(side_);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
@@ -124,7 +124,7 @@ int Engine::materialize() {
   if (!side_) QTG_HIP_TRY(hipStreamCreateWithFlags(&side_, hipStreamNonBlocking));
   if (!evFork_) QTG_HIP_TRY(hipEventCreateWithFlags(&evFork_, hipEventDisableTiming));
   if (!evHeev_) QTG_HIP_TRY(hipEventCreateWithFlags(&evHeev_, hipEventDisableTiming));
-  if (!evRho_) QTG_HIP_TRY(hipEventCreateWithFlags(&evRho_, hipEventDisableTiming));
+  if (!evCopy_) QTG_HIP_TRY(hipEventCreateWithFlags(&evCopy_, hipEventDisableTiming));
   std::vector<DNode> dn;
   for (auto& n : tree_.nodes) {
     DNode d{};
@@ -820,16 +820,7 @@ std::vector<Engine::Summand> Engine::aggregate(const std::vector<Summand>& tl, c
   return groups;
 }
 
-// The side stream of the last build still reads the state (its copy for
-// get_matrix): whoever writes d_psi64_ on stream s comes after it.
-int Engine::before_psi_write(hipStream_t s) {
-  if (heevPending_) QTG_HIP_TRY(hipStreamWaitEvent(s, evHeev_, 0));
-  return QTG_OK;
-}
-
 int Engine::set_psi(const double* host, hipStream_t s) {
-  const int rc = before_psi_write(s);
-  if (rc) return rc;
   QTG_HIP_TRY(hipMemcpyAsync(d_psi64_, host, sizeof(double) * 2 * tree_.total, hipMemcpyHostToDevice, s));
   QTG_HIP_TRY(hipStreamSynchronize(s));
   built_ = false;
@@ -837,8 +828,6 @@ int Engine::set_psi(const double* host, hipStream_t s) {
 }
 
 int Engine::set_psi_device(const double* dev, hipStream_t s) {
-  const int rc = before_psi_write(s);
-  if (rc) return rc;
   QTG_HIP_TRY(hipMemcpyAsync(d_psi64_, dev, sizeof(double) * 2 * tree_.total, hipMemcpyDeviceToDevice, s));
   built_ = false;
   return QTG_OK;

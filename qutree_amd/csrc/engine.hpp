@@ -263,7 +263,6 @@ class Engine {
   double* d_psiBuilt_ = nullptr;
   int64_t builds_ = 0, termsBuild_ = -1;
   int term_engine(int term, hipStream_t s);
-  int before_psi_write(hipStream_t s);
   std::vector<Summand> aggregate(const std::vector<Summand>& tl, const std::vector<int>& sdim, int64_t& off,
                                  double& combFlops);
   std::vector<CombOut> h_comb1_, h_comb2_;  // aggregated slots: partial sums, sums of partials
@@ -354,7 +353,7 @@ class Engine {
   std::vector<void*> device_buffers_;
   hipStream_t stream_ = nullptr;
   hipStream_t side_ = nullptr;  // density eigensolver, overlapping Apply
-  hipEvent_t evFork_ = nullptr, evHeev_ = nullptr, evRho_ = nullptr;
+  hipEvent_t evFork_ = nullptr, evHeev_ = nullptr, evCopy_ = nullptr;
   bool heevPending_ = false;
 
   hipGraph_t graph_h_ = nullptr;

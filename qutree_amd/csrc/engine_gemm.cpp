@@ -1352,7 +1352,10 @@ int Engine::build_gemm(hipStream_t s) {
     // combinations and Apply
     QTG_HIP_TRY(hipEventRecord(evFork_, s));
     QTG_HIP_TRY(hipStreamWaitEvent(side_, evFork_, 0));
-    if ((rc = keep_state(side_))) return rc;
+    if (d_psiBuilt_) {
+      if ((rc = keep_state(side_))) return rc;
+      QTG_HIP_TRY(hipEventRecord(evCopy_, side_));
+    }
     if ((rc = begin_mark(1, side_))) return rc;
     if ((rc = launch_heev<double>(d_eig_, nEig_, d_pool_, d_pool64_, eps_, nspf_, side_))) return rc;
     if ((rc = end_mark(side_))) return rc;
@@ -1378,6 +1381,9 @@ int Engine::build_gemm(hipStream_t s) {
   if ((rc = launch_combine<double>(d_combOut3_, nComb3_, d_combTerm3_, d_pool_, s))) return rc;
   if ((rc = end_mark(s))) return rc;
   if (timing_) tfl_[5] += phaseFlops_[5];
+  // the copy of the state has long passed: whatever writes the state after
+  // this build on its stream comes after it
+  if (heevSide_ && d_psiBuilt_) QTG_HIP_TRY(hipStreamWaitEvent(s, evCopy_, 0));
   built_ = true;
   return QTG_OK;
 }

@@ -92,8 +92,7 @@ int Engine::gradient(hipStream_t s, double* grad_host, double* energy) {
 
 int Engine::canonicalize(hipStream_t s) {
   void* bases[B_COUNT] = {d_psi32_, d_work32_, d_pool_, d_psi64_, d_apply64_, d_dpsi64_, d_pool64_, d_work_};
-  int rc = before_psi_write(s);
-  if (rc) return rc;
+  int rc;
   for (size_t d = 0; d < canonRange_.size(); ++d) {
     const auto& r = canonRange_[d];
     int64_t mmax = 0;

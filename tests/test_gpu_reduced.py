@@ -169,9 +169,10 @@ def test_second_hamiltonian_on_the_other_side_of_the_line(order, monkeypatch):
 
 
 def test_matrices_are_those_of_the_last_build_without_an_apply(every_size):
-    """build() alone, then another state: nothing but the setters themselves
-    orders the copy of the built state (side stream, behind the eigensolvers
-    of earlier builds) before the new one."""
+    """build() alone, then another state: no solve or tick waits for the side
+    stream, so the build itself has to order its copy of the state (behind
+    the eigensolvers of earlier builds there) before what its stream does
+    next."""
     text, H = _models()["wide8"]
     print("case matrices after build, then set_psi", flush=True)
     om = O.OracleModel(text, H)
