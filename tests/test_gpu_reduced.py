@@ -251,11 +251,11 @@ def test_reduced_precision_forms_lose_none_to_the_sums(name, monkeypatch):
     assert err["reduced"] < 1.005 * err["every matrix"]
 
 
-@pytest.mark.parametrize("precision,tol", [(0, 1e-11), (1, 1e-4)])
+@pytest.mark.parametrize("precision,tol", [(0, 1e-11), (1, 1e-4), (2, 1e-4)])
 def test_matrices_of_all_terms_in_any_order(precision, tol, every_size):
     """Every term's matrices from the growing groups of get_matrix, asked for
     in random order and after several builds, against the engine that forms
-    all of them (complex64: 100 times the rounding of its sums, for the
+    all of them (complex64 and split: 100 times the rounding of its sums, for the
     amplification along the tree)."""
     text, H = _models()["quartic16"]
     print(f"case matrices of all terms precision={precision}", flush=True)
