@@ -565,23 +565,25 @@ template int launch_gc_block<double>(const GcDesc*, const GcBlockWg*, int64_t, c
 template int launch_gc_block<float>(const GcDesc*, const GcBlockWg*, int64_t, const GcBlockWg*, int64_t, const void*,
                                     const void*, void*, void*, hipStream_t);
 
-// A reduction of up to oneWgK elements stays in one workgroup per tile, 16
-// wavefronts: 14.4 us at K = 512 (24 x 24 complex128 output), where two launches
-// take at least 14; beyond, its wavefronts walk a third stage, 21 us at K = 576
-// and at 768 against 14.6 and 13.7.  complex64: 10.5 us at K = 720 against
-// 12.2, 19.0 at 768 against 11.8.  Beyond it, K is split over workgroups toward
-// 512 of them (two per CU), with shares of at least 32 elements per wavefront
-// (K = 4096, 64 x 64: 15 us) and the partial tiles within max_part_elems (0: no
-// split over workgroups).  One wavefront per tile (gc_single) took 4891 us at
-// K = 65536, 64 x 64 complex128; this takes 46, of which the operands' 134 MB
-// at the card's copy rate are 28.
-GcOnePlan plan_gc_one(const GcDesc& d, bool c64, int64_t max_part_elems) {
-  const int64_t oneWgK = c64 ? 720 : 512;
+// A reduction of up to kOneWgK elements stays in one workgroup per tile, 16
+// wavefronts.  A split takes two launches and the slot's event besides, 4 us
+// more of the host: two products and a contraction of 552 elements (7 x 7
+// complex128 output) 17.7 against 21.4 us.  In a row of contractions alone the
+// split is level there (K = 520 to 750, 13-14 us either way for most shapes) and
+// ahead where `bef` is a multiple of eight (24 x 24, K = 576: 21 against 14.6);
+// at K = 1024 (32 x 32) it takes 14, at 2048 (64 x 64) 14.5.  Beyond the line, K
+// is split over workgroups toward 512 of them (two per CU), with shares of at
+// least 32 elements per wavefront (K = 4096, 64 x 64: 15 us) and the partial
+// tiles within max_part_elems (0: no split over workgroups).  One wavefront per
+// tile (gc_single) took 4891 us at K = 65536, 64 x 64 complex128; this takes 46,
+// of which the operands' 134 MB at the card's copy rate are 28.
+GcOnePlan plan_gc_one(const GcDesc& d, int64_t max_part_elems) {
+  constexpr int64_t kOneWgK = 768;
   const int64_t K = (int64_t)d.bef * d.aft;
   const int64_t m2 = gc_block_macros(d);
   GcOnePlan p{};
   p.S = 1;
-  if (K > oneWgK) {
+  if (K > kOneWgK) {
     int64_t S = std::min<int64_t>((512 + m2 - 1) / m2, K / 128);
     S = std::min<int64_t>(S, max_part_elems / (m2 * 1024));
     // workgroup macro * S + s: with 8 | S the macro tiles of a share, which

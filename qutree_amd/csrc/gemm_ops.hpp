@@ -195,7 +195,7 @@ struct GcOnePlan {
   int S;
   int64_t macro;  // workgroups per share
 };
-GcOnePlan plan_gc_one(const GcDesc& d, bool c64, int64_t max_part_elems);
+GcOnePlan plan_gc_one(const GcDesc& d, int64_t max_part_elems);
 template <typename T>
 int launch_gc_one(const GcDesc& d, const GcOnePlan& p, const void* x, const void* y, void* o, void* part,
                   hipStream_t s);

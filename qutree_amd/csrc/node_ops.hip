@@ -483,9 +483,8 @@ int hole_one(const qtg_hole_contraction_desc& d, cplx<R>* Sm, const cplx<R>* A, 
   int rc = to_gc(d, g);
   if (rc) return rc;
   if (!gc_lean_ok(g)) return launch_gc_single<R>(g, A, B, Sm, s);
-  constexpr bool c64 = sizeof(R) == sizeof(float);
-  GcOnePlan p = plan_gc_one(g, c64, (int64_t)(kPartBytes / sizeof(cplx<R>)));
-  if (p.S > 1 && capturing(s)) p = plan_gc_one(g, c64, 0);
+  GcOnePlan p = plan_gc_one(g, (int64_t)(kPartBytes / sizeof(cplx<R>)));
+  if (p.S > 1 && capturing(s)) p = plan_gc_one(g, 0);
   if (p.S > 1) return hole_split<R>(g, p, A, B, Sm, s);
   return launch_gc_one<R>(g, p, A, B, Sm, nullptr, s);
 }
