@@ -149,10 +149,12 @@ int Engine::materialize() {
 int Engine::set_hamiltonian(int64_t nterms, const double* coeff, const int64_t* term_off, const int64_t* fmode,
                             const int64_t* fkind, const int64_t* fpool, const double* pool) {
   std::string err;
-  if (build_sop(tree_, nterms, coeff, term_off, fmode, fkind, fpool, pool, sop_, err)) {
+  HSop sop;  // a refused one leaves the plan at hand and its terms as they are
+  if (build_sop(tree_, nterms, coeff, term_off, fmode, fkind, fpool, pool, sop, err)) {
     set_error("hamiltonian: " + err);
     return QTG_EARG;
   }
+  sop_ = std::move(sop);
   apply_tuning();
   planSmall_ = false;
   return plan();
@@ -190,6 +192,7 @@ std::vector<std::pair<int, int>> Engine::restrict_out(int l, int a) const {
 }
 
 int Engine::plan() {
+  planned_ = built_ = false;  // until the new plan stands
   active_sets();
   const int L = (int)sop_.terms.size();
   const int NN = (int)tree_.nodes.size();

@@ -275,3 +275,32 @@ def test_matrices_of_all_terms_in_any_order(precision, tol, every_size):
             for which in (2, 3):
                 ref = full.matrix(which, l, a)
                 assert np.max(np.abs(eng.matrix(which, l, a) - ref)) < tol * max(1, np.max(np.abs(ref)))
+
+
+def test_refused_hamiltonian_leaves_the_plan_at_hand(every_size):
+    """A Hamiltonian with a factor out of range, in its first or a later term,
+    is an error; the engine goes on with the one it has, matrices of single
+    terms included (formed from its terms on demand)."""
+    text, H = _models()["quartic16"]
+    print("case refused hamiltonian", flush=True)
+    om = O.OracleModel(text, H)
+    eng = Q.Engine(text, H)
+    psi = om.fill_random(1, delta_lowest=False)
+    om.build(psi)
+    ref = om.derivative(psi)
+    act = [(l, a) for l in range(H.nterms) for a in om.sparse_tree(l) if a != om.nnodes - 1]
+    for first in (True, False):
+        bad = W.Hamiltonian()
+        if not first:
+            bad.add_term(1.0, [(0, W.FACTOR_X2)])
+        bad.add_term(1.0, [(99, W.FACTOR_X)])
+        eng.set_psi(psi)
+        eng.derivative()
+        with pytest.raises(Q.QtgError, match="factor mode out of range"):
+            eng.set_hamiltonian(bad)
+        for l, a in act[::7]:
+            h, g = om.hmat(l, a), om.hole(l, a)
+            assert np.max(np.abs(eng.matrix(2, l, a) - h)) < 1e-11 * max(1, np.max(np.abs(h)))
+            assert np.max(np.abs(eng.matrix(3, l, a) - g)) < 1e-11 * max(1, np.max(np.abs(g)))
+        eng.derivative()
+        assert _err(eng.get(0), ref) < 1e-11
